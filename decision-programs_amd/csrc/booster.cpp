@@ -28,7 +28,6 @@
 
 namespace dp {
 
-void launch_any_nan(const float* values, int64_t n, int32_t* flag, hipStream_t s);
 void launch_check_labels(const float* label, int64_t n, int32_t objective, int32_t n_classes,
                          int32_t* bad, hipStream_t s);
 
@@ -129,16 +128,11 @@ std::string validate_hyperparameters(const std::string& text, uint32_t classes) 
 // ---------------------------------------------------------------------------
 // DMatrix quantisation
 // ---------------------------------------------------------------------------
-Quantized& DMatrix::quantize(int32_t max_bin, dp_workspace_s& ws, hipStream_t s) {
+Quantized& DMatrix::quantize(int32_t max_bin, hipStream_t s) {
   auto it = quantized.find(max_bin);
   if (it != quantized.end()) return *it->second;
   need(max_bin >= 2, "max_bin must be at least 2");
   auto q = std::make_unique<Quantized>();
-  DeviceBuffer<int32_t> flag(1);
-  launch_any_nan(values.p, n_rows * n_features, flag.p, s);
-  int32_t has_nan = 0;
-  DP_HIP(hipMemcpyAsync(&has_nan, flag.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  DP_HIP(hipStreamSynchronize(s));
   // Cuts for up to 256 bins, with or without missing values.  uint8 bins keep
   // byte 255 for missing values, so a matrix with NaN whose features use all
   // 256 bins keeps 16-bit columns instead (below).
@@ -147,9 +141,9 @@ Quantized& DMatrix::quantize(int32_t max_bin, dp_workspace_s& ws, hipStream_t s)
   q->cut_ptr.assign(size_t(n_features) + 1, 0);
   q->cut_values.assign(size_t(n_features) * eff, 0.0f);
   q->min_values.assign(size_t(n_features), 0.0f);
-  int32_t sketch_missing = 0;
-  sketch_cuts(ws, values.p, n_rows, n_features, eff, q->cut_ptr.data(), q->cut_values.data(),
-              q->min_values.data(), &sketch_missing, s);
+  int32_t has_nan = 0;
+  sketch_cuts(values.p, n_rows, n_features, eff, q->cut_ptr.data(), q->cut_values.data(),
+              q->min_values.data(), &has_nan, s);
   q->cut_values.resize(size_t(q->cut_ptr[size_t(n_features)]));
   std::vector<int32_t> nbins(static_cast<size_t>(n_features));
   int32_t widest = 1;
@@ -1116,12 +1110,7 @@ void Booster::run_round(DMatrix* d, bool with_gradients) {
   };
   words(inputs, &tp_, sizeof tp_);
   if (inputs != last_round_inputs_) flush();
-  Quantized* qp;
-  {
-    dp_workspace_s scratch;
-    qp = &d->quantize(tp_.max_bin, scratch, stream_);
-  }
-  Quantized& q = *qp;
+  Quantized& q = d->quantize(tp_.max_bin, stream_);
   effective_max_bin_ = q.max_bin;
   // Histogram layout: the present-value layout for mostly-missing matrices,
   // else the row-major copy of the tiles for gathered rows.

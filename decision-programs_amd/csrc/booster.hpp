@@ -67,7 +67,7 @@ struct DMatrix {
   DeviceBuffer<float> labels;
   bool has_labels = false;
   std::map<int32_t, std::unique_ptr<Quantized>> quantized;  // by requested max_bin
-  Quantized& quantize(int32_t max_bin, dp_workspace_s& ws, hipStream_t s);
+  Quantized& quantize(int32_t max_bin, hipStream_t s);
   // Boosters with a round in flight on this matrix.  Freeing the matrix
   // collects those rounds first (release_pending) and waits for the device.
   std::vector<const Booster*> pending;

@@ -588,7 +588,7 @@ int dp_sketch_cuts(dp_workspace ws, const float* values, int64_t n_rows, int32_t
                    int32_t* has_missing, void* stream) {
   return guarded([&] {
     dp::need(ws && values && cut_ptr && cut_values && min_values && has_missing, "null argument");
-    dp::sketch_cuts(*ws, values, n_rows, n_features, max_bin, cut_ptr, cut_values, min_values,
+    dp::sketch_cuts(values, n_rows, n_features, max_bin, cut_ptr, cut_values, min_values,
                     has_missing, as_stream(stream));
   });
 }

@@ -809,7 +809,7 @@ void launch_tiles_to_rows(const uint8_t* bins, const dp_bin_layout& layout, uint
 void launch_join_tiles(uint8_t* bins, const dp_bin_layout& layout, hipStream_t s);
 
 // Quantile cuts on the device; host outputs as in dp_sketch_cuts.
-void sketch_cuts(dp_workspace_s& ws, const float* values, int64_t n_rows, int32_t n_features,
+void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features,
                  int32_t max_bin, int32_t* cut_ptr, float* cut_values, float* min_values,
                  int32_t* has_missing, hipStream_t s);
 

@@ -1,0 +1,52 @@
+"""Quantile cuts against the oracle at the sizes and value patterns where the bucket
+passes change course: the row counts around the in-LDS sort and the sample, features
+whose distinct values are few, rare, repeated or adjacent, and missing values."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _columns(n, rng):
+    """Named value patterns, each float32 [n]."""
+    normal = rng.normal(size=n)
+    rare = rng.random(n) < 0.002
+    atom = np.where(rng.random(n) < 0.6, 1.5, normal)
+    missing = np.where(rng.random(n) < 0.999, np.nan, normal)
+    few = np.where(rng.random(n) < 0.97, np.nan, rng.integers(0, 9, n))
+    zero = np.where(rng.random(n) < 0.5, 0.0, -0.0)
+    edge = np.float32(1.0) + np.float32(2.0 ** -23) * rng.integers(0, 300, n).astype(np.float32)
+    wide = np.exp(30.0 * normal)
+    inf = np.where(rng.random(n) < 0.01, np.inf, np.where(rng.random(n) < 0.01, -np.inf, normal))
+    columns = {
+        "normal": normal, "constant": np.full(n, -3.25), "none": np.full(n, np.nan),
+        "int16": rng.integers(0, 16, n), "int256": rng.integers(0, 256, n),
+        "int257": rng.integers(0, 257, n),
+        # few common values and a few hundred rare ones: unseen or seen once in the sample
+        "rare200": np.where(rare, rng.integers(0, 200, n), 1000.0),
+        "rare400": np.where(rare, rng.integers(0, 400, n), rng.integers(1000, 1003, n)),
+        "atom": atom, "missing": missing, "few": few, "zero": zero, "adjacent": edge,
+        "wide": wide, "inf": inf, "denormal": normal * 1e-41, "sorted": np.arange(n) - n // 2,
+    }
+    return {k: np.asarray(v, dtype=np.float32) for k, v in columns.items()}
+
+
+@pytest.mark.parametrize("n,max_bin", [(1, 256), (2, 2), (257, 256), (8192, 255), (8193, 256),
+                                       (16384, 64), (16385, 256), (16385, 2), (60001, 255),
+                                       (300007, 256), (300007, 17)])
+def test_cuts_match_the_oracle(dp, oracle, ws, device, n, max_bin):
+    import torch
+    from dpgbdt import ops
+
+    columns = _columns(n, np.random.default_rng(n + max_bin))
+    x = np.ascontiguousarray(np.stack(list(columns.values()), axis=1))
+    for width in (x.shape[1], 1):  # 17 features: a ragged second tile; one feature alone
+        part = np.ascontiguousarray(x[:, :width])
+        ptr, cuts, mins, missing = ops.sketch_cuts(ws, torch.as_tensor(part, device=device),
+                                                   max_bin)
+        o_ptr, o_cuts, o_mins = oracle.compute_cuts(part, max_bin)
+        for f, name in enumerate(list(columns)[:width]):
+            got, want = cuts[ptr[f]:ptr[f + 1]], o_cuts[o_ptr[f]:o_ptr[f + 1]]
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=name)
+        np.testing.assert_array_equal(mins.view(np.uint32), o_mins.view(np.uint32))
+        assert missing == bool(np.isnan(part).any())
