@@ -176,10 +176,10 @@ Quantized& DMatrix::quantize(int32_t max_bin, hipStream_t s) {
     paired.paired_tiles = pair_tiles(nbins.data(), n_features, q->layout.n_tiles, has_nan);
     q->pairs = paired.paired_tiles;
     q->bins.resize(dp_layout_bytes(&paired));
-    launch_bin_values(values.p, q->layout, q->d_cut_ptr.p, q->d_cut_values.p, q->bins.p, s);
-    launch_join_tiles(q->bins.p, paired, s);
     q->cols.resize(size_t(n_rows) * size_t(n_features));
-    launch_tiles_to_columns(q->bins.p, q->layout, q->cols.p, s);
+    launch_bin_values(values.p, q->layout, q->d_cut_ptr.p, q->d_cut_values.p, q->bins.p,
+                      q->cols.p, s);
+    launch_join_tiles(q->bins.p, paired, s);
   }
   DP_HIP(hipStreamSynchronize(s));
   auto& ref = *q;

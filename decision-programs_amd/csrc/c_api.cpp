@@ -598,7 +598,8 @@ int dp_bin_values(const float* values, const dp_bin_layout* layout, const int32_
   return guarded([&] {
     dp::need(values && layout && cut_ptr && cut_values && bins, "null argument");
     require_paired_bins(bins, *layout);
-    dp::launch_bin_values(values, *layout, cut_ptr, cut_values, bins, as_stream(stream));
+    dp::launch_bin_values(values, *layout, cut_ptr, cut_values, bins, nullptr,
+                          as_stream(stream));
     dp::launch_join_tiles(bins, *layout, as_stream(stream));
   });
 }

@@ -528,7 +528,7 @@ struct LastLevel {
 
 // Partition: counts, then scatter (which writes the left totals of the
 // expanding nodes into node_left).  cols: column-major copy of the bins
-// (launch_tiles_to_columns) or null to read the tiles.  work_left: one word
+// (launch_bin_values) or null to read the tiles.  work_left: one word
 // per work item, the item's node in the upper 32 bits and its left rows in the
 // lower 32 (zero for a node that does not expand); masks: kPartMasks words per
 // work item (the count kernel's ballots, read back by the scatter).  node_left_zeroed: the caller has zeroed
@@ -708,9 +708,10 @@ void launch_quantise(const float* grad, const float* hess, int64_t n_rows, int32
 // *p = value (one thread), e.g. the round index the sampling kernels read.
 void launch_store_i32(int32_t* p, int32_t value, hipStream_t s);
 
+// bins: the tile-major bins (without joint tiles); cols: null, or their
+// column-major copy, cols[f * n_rows + r].
 void launch_bin_values(const float* values, const dp_bin_layout& layout, const int32_t* cut_ptr,
-                       const float* cut_values, uint8_t* bins, hipStream_t s);
-// cols[f * n_rows + r] = bin of (r, f), from the tile-major bins.
+                       const float* cut_values, uint8_t* bins, uint8_t* cols, hipStream_t s);
 // Present-value layout of a mostly-missing matrix.  Features are grouped in
 // tiles of tile_features (a multiple of 16, at most 256, sized so that one
 // tile's histogram fills kSparseLdsBytes of LDS).  For tile t and row r the
@@ -795,8 +796,6 @@ void launch_hist_reduce_flat(const int64_t* partial, const HistReduce* jobs, int
                              int32_t n_features, int32_t bin_stride, const int64_t* parent_base,
                              int64_t* hist, hipStream_t s);
 
-void launch_tiles_to_columns(const uint8_t* bins, const dp_bin_layout& layout, uint8_t* cols,
-                             hipStream_t s);
 // rows[r * n_tiles * 16 + t * 16 + j] = tile t's byte j of row r; for the
 // first tile t of each of the layout's pairs, the pair's joint tile instead
 // (from the tile-major bins, which hold it): the copy the gathered passes of

@@ -4,6 +4,7 @@
 // sketch.hip).  The reference bins inside XGDMatrixCreateFromCudaArrayInterface
 // and the first update (class_native_training.cuh:51).
 #include "dp_internal.hpp"
+#include "search.hpp"
 
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_reduce.hpp>
@@ -12,59 +13,114 @@
 namespace dp {
 namespace {
 
-// Bins for one tile of FT features; cuts of the tile staged in LDS.
-template <int FT>
-__global__ __launch_bounds__(256) void bin_kernel(const float* __restrict__ values,
-                                                  int64_t n_rows, int32_t n_features,
-                                                  const int32_t* __restrict__ cut_ptr,
-                                                  const float* __restrict__ cut_values,
-                                                  int32_t stride, int32_t missing_bin,
-                                                  uint8_t* __restrict__ bins) {
-  extern __shared__ float s_cuts[];  // [FT][stride]
-  __shared__ int s_count[FT];
-  const int tile = blockIdx.y;
-  const int f0 = tile * FT;
-  for (int e = threadIdx.x; e < FT; e += blockDim.x) {
-    const int f = f0 + e;
-    s_count[e] = f < n_features ? cut_ptr[f + 1] - cut_ptr[f] : 0;
-  }
+// Bins of one 16-feature tile: the tile-major uint8 bins and, when asked for,
+// their column-major copy; or (WIDE) 16-bit columns only (missing:
+// kWideMissing), for matrices whose missing values need a symbol beside 256
+// bins.
+//
+// A lane's feature is lane & 15: a load takes 4 rows' 64-byte runs.  Lane group
+// lane >> 4 owns kBinRows adjacent rows, whose searches run side by side; its
+// bytes are then adjacent in the column copy, and four lanes exchange theirs so
+// that each stores a 4-feature word of one row of the tile.  One workgroup takes
+// a chunk of rows; those of one XCD take adjacent tiles of the same rows, which
+// share 128-byte lines.
+//
+// Memory (4 B in, 1 or 2 B out per value) and the LDS reads of the search, 4 of
+// 16 bytes per value with 65-256 bins, bound it.  The row-per-thread kernel it
+// replaced (16 strided loads, 8 binary steps of one word each) took 0.70 ms for
+// 1M x 100 and 12.9 ms for 2M x 1,000 with 95 % missing, and the column copy a
+// pass of its own (0.71 ms at the latter); now 0.26 and 4.7 ms, copy included.
+constexpr int kBinRows = 8;
+constexpr int kBinThreads = 256;
+
+struct __attribute__((packed)) PackedWords {
+  uint32_t w[kBinRows / 4];
+};
+
+template <bool WIDE>
+__global__ __launch_bounds__(kBinThreads) void bin_kernel(
+    const float* __restrict__ values, int64_t n_rows, int32_t n_features,
+    const int32_t* __restrict__ cut_ptr, const float* __restrict__ cut_values,
+    int32_t missing_bin, int32_t tiles, int32_t chunks, int64_t chunk_rows,
+    uint8_t* __restrict__ bins, uint8_t* __restrict__ cols, uint16_t* __restrict__ cols16) {
+  __shared__ uint4 tree[search_nodes(4) * kTile];
+  const int32_t per = (tiles * chunks + 7) / 8;
+  const int32_t item = int32_t(blockIdx.x % 8) * per + int32_t(blockIdx.x / 8);
+  if (int32_t(blockIdx.x / 8) >= per || item >= tiles * chunks) return;
+  const int32_t chunk = item / tiles, f0 = item % tiles * kTile;
+  int widest = 1;
+  for (int k = 0; k < kTile && f0 + k < n_features; ++k)
+    widest = max(widest, cut_ptr[f0 + k + 1] - cut_ptr[f0 + k]);
+  const int levels = search_levels(min(widest, kMaxBins));
+  // bin(x) = cuts <= x, the last cut left out: the clamp to the last bin.
+  search_fill(tree, levels, [&](int j, int p) {
+    const int f = f0 + j;
+    if (f >= n_features || p >= cut_ptr[f + 1] - cut_ptr[f]) return kNanKey;
+    return order_key(cut_values[cut_ptr[f] + p - 1]);
+  });
   __syncthreads();
-  for (int e = threadIdx.x; e < FT * stride; e += blockDim.x) {
-    const int jf = e / stride, b = e % stride;
-    const int f = f0 + jf;
-    s_cuts[e] = (f < n_features && b < s_count[jf]) ? cut_values[cut_ptr[f] + b] : 0.0f;
-  }
-  __syncthreads();
-  constexpr int TPR = FT / 16;
-  const int sub = threadIdx.x % TPR;
-  const int64_t rows_per_block = blockDim.x / TPR;
-  uint8_t* tile_base = bins + int64_t(tile) * n_rows * FT;
-  for (int64_t r = int64_t(blockIdx.x) * rows_per_block + threadIdx.x / TPR; r < n_rows;
-       r += int64_t(gridDim.x) * rows_per_block) {
-    uint32_t word[4] = {0, 0, 0, 0};
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 15, f = f0 + j;
+  const bool live = f < n_features;
+  uint8_t* tile = WIDE ? nullptr : bins + int64_t(f0 / kTile) * n_rows * kTile;
+  const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
+  constexpr int kWaveRows = 4 * kBinRows;
+  for (int64_t w0 = chunk * chunk_rows + wave * kWaveRows; w0 < r1;
+       w0 += kBinThreads / 64 * kWaveRows) {
+    const int64_t r0 = w0 + (lane >> 4) * kBinRows;
+    // Loads without branches (rows and features past the end repeat the last),
+    // so that all are in flight before the first is waited for.
+    float x[kBinRows];
+    uint32_t key[kBinRows];
+    int bin[kBinRows];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int jf = sub * 16 + k;
-      const int f = f0 + jf;
-      uint32_t b = 0;
-      if (f < n_features) {
-        const float x = values[r * n_features + f];
-        if (x != x) {
-          b = uint32_t(missing_bin);
-        } else {
-          const float* c = s_cuts + jf * stride;
-          int lo = 0, hi = s_count[jf];
-          while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (c[mid] > x) hi = mid; else lo = mid + 1;
-          }
-          b = uint32_t(lo < s_count[jf] ? lo : s_count[jf] - 1);
-        }
-      }
-      word[k >> 2] |= (b & 0xffu) << ((k & 3) * 8);
+    for (int u = 0; u < kBinRows; ++u)
+      x[u] = values[min(r0 + u, r1 - 1) * n_features + min(f, n_features - 1)];
+#pragma unroll
+    for (int u = 0; u < kBinRows; ++u) key[u] = order_key(x[u]) & (live ? ~0u : 0u);
+    search<kBinRows>(tree, levels, j, key, bin);
+#pragma unroll
+    for (int u = 0; u < kBinRows; ++u)
+      if (live && x[u] != x[u]) bin[u] = WIDE ? kWideMissing : missing_bin & 0xff;
+    if constexpr (WIDE) {
+      if (!live) continue;
+      uint16_t* c = cols16 + int64_t(f) * n_rows + r0;
+#pragma unroll
+      for (int u = 0; u < kBinRows; ++u)
+        if (r0 + u < r1) c[u] = uint16_t(bin[u]);
+      continue;
     }
-    *reinterpret_cast<uint4*>(tile_base + r * FT + sub * 16) =
-        make_uint4(word[0], word[1], word[2], word[3]);
+    uint32_t word[kBinRows];  // the 4 bins of row r0 + u of this lane's group of 4 features
+#pragma unroll
+    for (int u = 0; u < kBinRows; ++u) {
+      const uint32_t b = uint32_t(bin[u]);
+      const uint32_t x = __builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+      const uint32_t h = lane & 1 ? x | b << 8 : b | x << 8;
+      const uint32_t y = __builtin_amdgcn_mov_dpp(h, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+      word[u] = lane & 2 ? y | h << 16 : h | y << 16;
+    }
+#pragma unroll
+    for (int u = 0; u < kBinRows; u += 4) {
+      const int k = lane & 3;
+      const uint32_t v = k < 2 ? (k == 0 ? word[u] : word[u + 1])
+                               : (k == 2 ? word[u + 2] : word[u + 3]);
+      const int64_t r = r0 + u + k;
+      if (r < r1) *reinterpret_cast<uint32_t*>(tile + r * kTile + (j & ~3)) = v;
+    }
+    if (!cols || !live) continue;
+    uint8_t* c = cols + int64_t(f) * n_rows + r0;
+    if (r0 + kBinRows <= r1) {
+      PackedWords w;
+#pragma unroll
+      for (int q = 0; q < kBinRows / 4; ++q)
+        w.w[q] = uint32_t(bin[4 * q]) | uint32_t(bin[4 * q + 1]) << 8 |
+                 uint32_t(bin[4 * q + 2]) << 16 | uint32_t(bin[4 * q + 3]) << 24;
+      *reinterpret_cast<PackedWords*>(c) = w;
+    } else {
+#pragma unroll
+      for (int u = 0; u < kBinRows; ++u)
+        if (r0 + u < r1) c[u] = uint8_t(bin[u]);
+    }
   }
 }
 
@@ -86,31 +142,6 @@ __global__ void copy_matrix_kernel(const float* __restrict__ src, int64_t row_st
     dst[i] = x;
   }
   if (__ballot(inf) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
-}
-
-// Column-major copy of tile-major bins: cols[f * n_rows + r].  A workgroup
-// stages 256 rows x 16 features in LDS and writes 16 runs of 256 bytes.
-__global__ __launch_bounds__(256) void tiles_to_columns_kernel(const uint8_t* __restrict__ bins,
-                                                               int64_t n_rows, int32_t n_features,
-                                                               uint8_t* __restrict__ cols) {
-  __shared__ uint8_t s[16][256 + 4];
-  const int tile = blockIdx.y;
-  const int f0 = tile * 16;
-  const uint8_t* tb = bins + int64_t(tile) * n_rows * 16;
-  for (int64_t r0 = int64_t(blockIdx.x) * 256; r0 < n_rows; r0 += int64_t(gridDim.x) * 256) {
-    const int64_t r = r0 + threadIdx.x;
-    if (r < n_rows) {
-      const uint4 v = *reinterpret_cast<const uint4*>(tb + r * 16);
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int k = 0; k < 16; ++k) s[k][threadIdx.x] = uint8_t(w[k >> 2] >> (8 * (k & 3)));
-    }
-    __syncthreads();
-    if (r < n_rows)
-      for (int k = 0; k < 16 && f0 + k < n_features; ++k)
-        cols[int64_t(f0 + k) * n_rows + r] = s[k][threadIdx.x];
-    __syncthreads();
-  }
 }
 
 // Joint tiles of the paired tiles (dp_bin_layout::paired_tiles): joint tile
@@ -221,48 +252,6 @@ __global__ void sparse_fill_kernel(const uint8_t* __restrict__ bins, int64_t n_r
   }
 }
 
-// 16-bit column copy of a matrix whose missing values need a symbol beside 256
-// bins: cols[f * n_rows + r] = the bin of (r, f), kWideMissing for NaN.  A
-// thread bins one row of one 16-feature tile (the tile's cuts staged in LDS)
-// and stores its 16 symbols, so that for each feature a wavefront stores 64
-// adjacent symbols.
-__global__ __launch_bounds__(256) void bin_columns16_kernel(const float* __restrict__ values,
-                                                            int64_t n_rows, int32_t n_features,
-                                                            const int32_t* __restrict__ cut_ptr,
-                                                            const float* __restrict__ cut_values,
-                                                            uint16_t* __restrict__ cols) {
-  __shared__ float s_cuts[16 * kMaxBins];
-  __shared__ int s_count[16];
-  const int f0 = blockIdx.y * 16;
-  if (threadIdx.x < 16) {
-    const int f = f0 + int(threadIdx.x);
-    s_count[threadIdx.x] = f < n_features ? cut_ptr[f + 1] - cut_ptr[f] : 0;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 16 * kMaxBins; e += blockDim.x) {
-    const int jf = e / kMaxBins, b = e % kMaxBins;
-    s_cuts[e] = b < s_count[jf] ? cut_values[cut_ptr[f0 + jf] + b] : 0.0f;
-  }
-  __syncthreads();
-  for (int64_t r = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; r < n_rows;
-       r += int64_t(gridDim.x) * blockDim.x) {
-    for (int k = 0; k < 16 && f0 + k < n_features; ++k) {
-      const float x = values[r * n_features + f0 + k];
-      uint32_t b = uint32_t(kWideMissing);
-      if (x == x) {
-        const float* c = s_cuts + k * kMaxBins;
-        int lo = 0, hi = s_count[k];
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (c[mid] > x) hi = mid; else lo = mid + 1;
-        }
-        b = uint32_t(lo < s_count[k] ? lo : s_count[k] - 1);
-      }
-      cols[int64_t(f0 + k) * n_rows + r] = uint16_t(b);
-    }
-  }
-}
-
 // The present-value layout from 16-bit columns (missing: kWideMissing); one
 // thread per (sparse tile, row) as sparse_count_kernel / sparse_fill_kernel,
 // reading the tile's features of its row from the columns (adjacent threads,
@@ -356,17 +345,6 @@ void launch_join_tiles(uint8_t* bins, const dp_bin_layout& layout, hipStream_t s
                      dim3(256), 0, s, bins, layout.n_rows, layout.n_tiles, layout.paired_tiles);
   DP_HIP(hipGetLastError());
 }
-
-void launch_tiles_to_columns(const uint8_t* bins, const dp_bin_layout& layout, uint8_t* cols,
-                             hipStream_t s) {
-  if (layout.n_rows <= 0) return;
-  need(layout.tile_width == 16, "column copy needs 16-feature tiles");
-  hipLaunchKernelGGL(tiles_to_columns_kernel, dim3(grid_for(layout.n_rows, 256, 4096),
-                     layout.n_tiles), dim3(256), 0, s, bins, layout.n_rows, layout.n_features,
-                     cols);
-  DP_HIP(hipGetLastError());
-}
-
 
 // Row-major present values: counts of (row r, tile t) at r * T + t, from the
 // tile-major offsets.
@@ -507,15 +485,6 @@ void build_sparse_bins_wide(const uint16_t* cols, int64_t n_rows, int32_t n_feat
            "missing values and 256 bins holds (use max_bin 255 or less)");
 }
 
-void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_features,
-                          const int32_t* cut_ptr, const float* cut_values, uint16_t* cols,
-                          hipStream_t s) {
-  if (n_rows <= 0 || n_features <= 0) return;
-  hipLaunchKernelGGL(bin_columns16_kernel, dim3(grid_for(n_rows, 256, 4096), (n_features + 15) / 16),
-                     dim3(256), 0, s, values, n_rows, n_features, cut_ptr, cut_values, cols);
-  DP_HIP(hipGetLastError());
-}
-
 void launch_copy_matrix(const float* src, int64_t row_stride, int64_t n_rows, int32_t n_features,
                         float missing, float* dst, int32_t* bad, hipStream_t s) {
   launch_fill_u8(reinterpret_cast<uint8_t*>(bad), 4, 0, s);
@@ -526,17 +495,35 @@ void launch_copy_matrix(const float* src, int64_t row_stride, int64_t n_rows, in
   DP_HIP(hipGetLastError());
 }
 
+// Row chunks of the binning grid: about eight workgroups per CU, of at least
+// 1,024 rows so that the tile's tables are worth their fill.
+static int32_t bin_chunks(int64_t n_rows, int32_t tiles) {
+  const int64_t chunks = std::min<int64_t>((n_rows + 1023) / 1024, (2048 + tiles - 1) / tiles);
+  return int32_t(std::max<int64_t>(chunks, 1));
+}
+
 void launch_bin_values(const float* values, const dp_bin_layout& layout, const int32_t* cut_ptr,
-                       const float* cut_values, uint8_t* bins, hipStream_t s) {
+                       const float* cut_values, uint8_t* bins, uint8_t* cols, hipStream_t s) {
   if (layout.n_rows <= 0) return;
-  const int stride = kMaxBins;
-  const int rows_per_block = 256 / (layout.tile_width / 16);
-  const int gx = grid_for(layout.n_rows, rows_per_block, 4096);
-  const size_t lds = size_t(layout.tile_width) * stride * sizeof(float);
-  need(layout.tile_width == 16, "binning needs 16-feature tiles");
-  hipLaunchKernelGGL(bin_kernel<16>, dim3(gx, layout.n_tiles), dim3(256), lds, s, values,
-                     layout.n_rows, layout.n_features, cut_ptr, cut_values, stride,
-                     layout.missing_bin, bins);
+  need(layout.tile_width == kTile, "binning needs 16-feature tiles");
+  const int32_t chunks = bin_chunks(layout.n_rows, layout.n_tiles);
+  hipLaunchKernelGGL(bin_kernel<false>, dim3(unsigned((layout.n_tiles * chunks + 7) / 8 * 8)),
+                     dim3(kBinThreads), 0, s, values, layout.n_rows, layout.n_features, cut_ptr,
+                     cut_values, layout.missing_bin, layout.n_tiles, chunks,
+                     (layout.n_rows + chunks - 1) / chunks, bins, cols,
+                     static_cast<uint16_t*>(nullptr));
+  DP_HIP(hipGetLastError());
+}
+
+void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_features,
+                          const int32_t* cut_ptr, const float* cut_values, uint16_t* cols,
+                          hipStream_t s) {
+  if (n_rows <= 0 || n_features <= 0) return;
+  const int32_t tiles = (n_features + kTile - 1) / kTile, chunks = bin_chunks(n_rows, tiles);
+  hipLaunchKernelGGL(bin_kernel<true>, dim3(unsigned((tiles * chunks + 7) / 8 * 8)),
+                     dim3(kBinThreads), 0, s, values, n_rows, n_features, cut_ptr, cut_values,
+                     kWideMissing, tiles, chunks, (n_rows + chunks - 1) / chunks,
+                     static_cast<uint8_t*>(nullptr), static_cast<uint8_t*>(nullptr), cols);
   DP_HIP(hipGetLastError());
 }
 

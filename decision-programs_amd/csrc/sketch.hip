@@ -32,9 +32,10 @@
 // Two reads of the matrix and its binary searches bound it.  Sorting every
 // feature (a radix sort each) moved 8 to 10 times the bytes in 4 to 21 launches
 // per feature.  Device time before and now: 1M x 100, 20 % missing, 255 bins
-// 19.0 -> 1.15 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 13 ms; 1M x 28 4.2
-// -> 0.38 ms; 10k x 8 0.22 -> 0.08 ms.
+// 19.0 -> 0.91 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 9.2 ms; 1M x 28 4.2
+// -> 0.3 ms; 10k x 8 0.22 -> 0.06 ms.
 #include "dp_internal.hpp"
+#include "search.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -42,28 +43,17 @@
 namespace dp {
 namespace {
 
-constexpr uint32_t kNanKey = 0xffffffffu;
-
-__device__ __forceinline__ uint32_t order_key(float x) {
-  if (x != x) return kNanKey;
-  if (x == 0.0f) return 0x80000000u;
-  const uint32_t b = __float_as_uint(x);
-  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-
-__device__ __forceinline__ float key_value(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
-
 __device__ __forceinline__ float end_cut(float v) { return v + (fabsf(v) + 1e-5f); }
 
 // Features are handled in tiles of 16: a row's 16 values are 64 adjacent bytes,
 // and a lane's feature is fixed (lane & 15), so tables interleaved [entry][16]
 // put the lanes of different features on different LDS banks.
-constexpr int kTile = 16;
-// 1,024 boundaries x 16 features of 4 bytes beside as many counters: 128 KiB of
-// a CU's 160 KiB of LDS.
-constexpr int kBuckets = 1024;
+// The buckets of 16 features that fit a CU's 160 KiB of LDS: 4-ary trees of five
+// levels (search.hpp) and as many counters.
+constexpr int kLevels = 5;
+constexpr int kBuckets = 1 << (2 * kLevels);
+constexpr size_t kBucketLds = sizeof(uint4) * search_nodes(kLevels) * kTile +
+                              sizeof(uint32_t) * kBuckets * kTile;
 constexpr int kSample = 8192;
 constexpr int kThreads = 1024;
 // Rows up to which a feature is sorted whole in LDS (68 KiB padded): one
@@ -86,28 +76,30 @@ struct SketchOut {
 __device__ __forceinline__ int sort_at(int i) { return i + (i >> 4); }
 constexpr int sort_words(int n) { return n + n / 16; }
 
-// G adjacent compare-exchange steps (strides lo << (G - 1) ... lo) of bitonic
-// stage k on the 2^G elements of unit u, in registers.
+// G adjacent compare-exchange steps (strides 2^(lg + G - 1) ... 2^lg) of bitonic
+// stage k on the 2^G elements of unit u, in registers.  Element i of the unit
+// lies sort_at(i << lg) words after its first (the unit's low bits carry into no
+// pad), a wave-uniform offset; descending units sort inverted keys.
 template <int G>
-__device__ __forceinline__ void bitonic_unit(uint32_t* s, int u, int lo, int k) {
-  const int base = (u / lo) * (lo << G) + (u % lo);
-  const bool up = (base & k) == 0;
+__device__ __forceinline__ void bitonic_unit(uint32_t* s, int u, int lg, int k) {
+  const int base = ((u >> lg) << (lg + G)) | (u & ((1 << lg) - 1));
+  const uint32_t flip = base & k ? ~0u : 0u;
+  uint32_t* const p = s + sort_at(base);
   uint32_t e[1 << G];
 #pragma unroll
-  for (int i = 0; i < (1 << G); ++i) e[i] = s[sort_at(base + i * lo)];
+  for (int i = 0; i < (1 << G); ++i) e[i] = p[sort_at(i << lg)] ^ flip;
 #pragma unroll
   for (int b = G - 1; b >= 0; --b) {
 #pragma unroll
     for (int i = 0; i < (1 << G); ++i) {
       if (i & (1 << b)) continue;
       const uint32_t x = e[i], y = e[i | (1 << b)];
-      const uint32_t mn = min(x, y), mx = max(x, y);
-      e[i] = up ? mn : mx;
-      e[i | (1 << b)] = up ? mx : mn;
+      e[i] = min(x, y);
+      e[i | (1 << b)] = max(x, y);
     }
   }
 #pragma unroll
-  for (int i = 0; i < (1 << G); ++i) s[sort_at(base + i * lo)] = e[i];
+  for (int i = 0; i < (1 << G); ++i) p[sort_at(i << lg)] = e[i] ^ flip;
 }
 
 // Ascending sort of N (a power of two, kThreads * 2^E) words; every thread of the
@@ -116,22 +108,20 @@ __device__ __forceinline__ void bitonic_unit(uint32_t* s, int u, int lo, int k) 
 template <int N, int E>
 __device__ void sort_lds(uint32_t* s) {
   static_assert(N == kThreads << E, "one unit of 2^E elements per thread");
-  for (int k = 2; k <= N; k <<= 1) {
-    int hi = k >> 1;
-    while (hi > 0) {
-      const int steps = 32 - __builtin_clz(unsigned(hi));  // strides hi .. 1
-      const int g = steps < E ? steps : E;
-      const int lo = hi >> (g - 1);
+  for (int stage = 1; (1 << stage) <= N; ++stage) {
+    for (int left = stage; left > 0;) {  // strides 2^(left - 1) .. 1 to go
+      const int g = left < E ? left : E;
+      const int lg = left - g;
       __syncthreads();
       for (int u = threadIdx.x; u < (N >> g); u += kThreads) {
         switch (g) {
-          case 1: bitonic_unit<1>(s, u, lo, k); break;
-          case 2: bitonic_unit<2>(s, u, lo, k); break;
-          case 3: bitonic_unit<3>(s, u, lo, k); break;
-          default: bitonic_unit<E>(s, u, lo, k); break;
+          case 1: bitonic_unit<1>(s, u, lg, 1 << stage); break;
+          case 2: bitonic_unit<2>(s, u, lg, 1 << stage); break;
+          case 3: bitonic_unit<3>(s, u, lg, 1 << stage); break;
+          default: bitonic_unit<E>(s, u, lg, 1 << stage); break;
         }
       }
-      hi = lo >> 1;
+      left = lg;
     }
   }
   __syncthreads();
@@ -320,13 +310,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 
 // The count and gather passes.  A workgroup takes rows [chunk * chunk_rows,
 // ...) of one tile; lane & 15 is the feature, so a wavefront reads 4 rows'
-// 64-byte runs per load, kRows loads in flight, and kRows independent binary
-// searches hide each other's LDS latency.
+// 64-byte runs per load, kRows loads in flight, and kRows independent searches
+// hide each other's LDS latency.
 //   count   slots[chunk][tile][bucket][16] = values per bucket
 //   gather  slots holds each (chunk, bucket)'s offset in its segment and
 //           seg[tile][bucket][16] the segment's in the feature (kNanKey: not
 //           wanted); the keys go to out[plan.base + segment + offset].
-// Tables and counters take 128 KiB of LDS: one workgroup per CU.
+// Trees (85 KiB) and counters (64 KiB) leave one workgroup per CU.
 constexpr int kRows = 8;
 template <bool GATHER>
 __global__ __launch_bounds__(kThreads) void bucket_kernel(
@@ -336,9 +326,8 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
     const int32_t* __restrict__ used, uint32_t* __restrict__ slots,
     const uint32_t* __restrict__ seg, const FeaturePlan* __restrict__ plans,
     uint32_t* __restrict__ out) {
-  extern __shared__ uint32_t lds[];
-  uint32_t* s_bound = lds;                     // [kBuckets][16]
-  uint32_t* s_count = lds + kBuckets * kTile;  // [kBuckets][16]
+  extern __shared__ uint4 tree[];  // [search_nodes(kLevels)][16]
+  uint32_t* s_count = reinterpret_cast<uint32_t*>(tree + search_nodes(kLevels) * kTile);
   // Workgroups of one XCD (blockIdx % 8) take adjacent tiles of the same rows,
   // which share 128-byte lines.
   const int32_t per = (tiles * chunks + 7) / 8;
@@ -352,7 +341,6 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
   uint32_t* slot = slots + (int64_t(chunk) * tiles + tile) * kBuckets * kTile;
   const uint32_t* ts = GATHER ? seg + int64_t(tile) * kBuckets * kTile : nullptr;
   for (int e = threadIdx.x; e < kBuckets * kTile; e += kThreads) {
-    s_bound[e] = f_begin + tile * kTile + (e & (kTile - 1)) < f_end ? tb[e] : kNanKey;
     if constexpr (GATHER) {
       const uint32_t o = f_begin + tile * kTile + (e & (kTile - 1)) < f_end ? ts[e] : kNanKey;
       s_count[e] = o == kNanKey ? kNanKey : o + slot[e];
@@ -363,26 +351,26 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
   int32_t widest = 1;
   for (int k = 0; k < kTile && f_begin + tile * kTile + k < f_end; ++k)
     widest = max(widest, used[tile * kTile + k]);
-  int top = 1;  // the first step of a search over `widest` entries
-  while (top * 2 < widest) top *= 2;
+  const int levels = search_levels(widest);
+  search_fill(tree, levels, [&](int k, int p) {
+    return f_begin + tile * kTile + k < f_end ? tb[p * kTile + k] : kNanKey;
+  });
   uint32_t* keys = nullptr;
   if constexpr (GATHER) keys = live ? out + plans[tile * kTile + j].base : nullptr;
   __syncthreads();
   const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
   for (int64_t r0 = chunk * chunk_rows + (threadIdx.x >> 4); r0 < r1; r0 += 64 * kRows) {
+    // Loads without branches, so that all are in flight before the first wait.
+    float x[kRows];
     uint32_t key[kRows];
     int pos[kRows];
 #pragma unroll
-    for (int u = 0; u < kRows; ++u) {
-      const int64_t r = r0 + u * 64;
-      key[u] = live && r < r1 ? order_key(values[r * n_features + f]) : kNanKey;
-      pos[u] = 0;
-    }
-    for (int step = top; step > 0; step >>= 1) {
+    for (int u = 0; u < kRows; ++u)
+      x[u] = values[min(r0 + u * 64, r1 - 1) * n_features + min(f, n_features - 1)];
 #pragma unroll
-      for (int u = 0; u < kRows; ++u)
-        if (s_bound[(pos[u] + step) * kTile + j] <= key[u]) pos[u] += step;
-    }
+    for (int u = 0; u < kRows; ++u)
+      key[u] = order_key(x[u]) | (live && r0 + u * 64 < r1 ? 0u : ~0u);
+    search<kRows>(tree, levels, j, key, pos);
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
       if (key[u] == kNanKey) continue;
@@ -426,6 +414,9 @@ __global__ __launch_bounds__(256) void offsets_kernel(uint32_t* __restrict__ slo
   totals[e] = run;
 }
 
+constexpr int kPlanStride = sort_words(kBuckets) + 1;
+constexpr size_t kPlanLds = sizeof(uint32_t) * 2 * kPlanStride * kTile;
+
 // One workgroup per tile, one wavefront per feature: prefix sums of the bucket
 // counts, the bucket of every wanted rank (rank 0, floor(i * n / max_bin), n -
 // 1), the wanted buckets' segments.  totals becomes the prefix sums.
@@ -435,15 +426,18 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
     int32_t max_bin, uint32_t* __restrict__ totals, uint32_t* __restrict__ seg,
     int32_t* __restrict__ rank_bucket, FeaturePlan* __restrict__ plans,
     unsigned long long* __restrict__ gathered) {
+  // Per feature a run of kBuckets words with a pad word per 16: a lane's 16
+  // buckets are then 17 words from the next lane's.
   extern __shared__ uint32_t lds[];
-  uint32_t* s_first = lds;                      // [kBuckets][16]: exclusive prefix sums
-  uint32_t* s_need = lds + kBuckets * kTile;    // [kBuckets][16]: bucket size, 0 = not wanted
+  uint32_t* s_first = lds;                        // exclusive prefix sums
+  uint32_t* s_need = lds + kPlanStride * kTile;   // wanted, then the segment's offset
+  auto at = [](int b, int k) { return k * kPlanStride + sort_at(b); };
   const int32_t tile = blockIdx.x;
   uint32_t* tt = totals + int64_t(tile) * kBuckets * kTile;
   const uint32_t* tb = bounds + int64_t(tile) * kBuckets * kTile;
   for (int e = threadIdx.x; e < kBuckets * kTile; e += kThreads) {
-    s_first[e] = tt[e];
-    s_need[e] = 0u;
+    s_first[at(e / kTile, e % kTile)] = tt[e];
+    s_need[at(e / kTile, e % kTile)] = 0u;
   }
   __syncthreads();
   const int j = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -453,7 +447,7 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
   uint32_t size[kPer], sum = 0, nonempty = 0;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    size[k] = f < f_count ? s_first[(lane * kPer + k) * kTile + j] : 0u;
+    size[k] = f < f_count ? s_first[at(lane * kPer + k, j)] : 0u;
     sum += size[k];
     nonempty += size[k] ? 1u : 0u;
   }
@@ -467,7 +461,7 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
   uint32_t run = x - sum;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    s_first[(lane * kPer + k) * kTile + j] = run;
+    s_first[at(lane * kPer + k, j)] = run;
     run += size[k];
   }
   __syncthreads();
@@ -483,19 +477,19 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
       const uint32_t r = i == max_bin ? n - 1u : uint32_t((uint64_t(i) * n) / uint32_t(max_bin));
       int b = 0;  // the last bucket whose prefix sum is <= r: the non-empty one that holds r
       for (int step = kBuckets / 2; step > 0; step >>= 1)
-        if (s_first[(b + step) * kTile + j] <= r) b += step;
+        if (s_first[at(b + step, j)] <= r) b += step;
       rank_bucket[int64_t(f) * (max_bin + 1) + i] = b;
-      if (!enumerate && wide(b)) s_need[b * kTile + j] = 1u;
+      if (!enumerate && wide(b)) s_need[at(b, j)] = 1u;
     }
     if (enumerate)
       for (int k = 0; k < kPer; ++k)
-        if (size[k] && wide(lane * kPer + k)) s_need[(lane * kPer + k) * kTile + j] = 1u;
+        if (size[k] && wide(lane * kPer + k)) s_need[at(lane * kPer + k, j)] = 1u;
   }
   __syncthreads();
   uint32_t take = 0;
 #pragma unroll
   for (int k = 0; k < kPer; ++k)
-    take += s_need[(lane * kPer + k) * kTile + j] ? size[k] : 0u;
+    take += s_need[at(lane * kPer + k, j)] ? size[k] : 0u;
   x = take;
   for (int d = 1; d < 64; d <<= 1) {
     const uint32_t y = __shfl_up(x, d, 64);
@@ -510,7 +504,7 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const int e = (lane * kPer + k) * kTile + j;
+    const int e = at(lane * kPer + k, j);
     const bool need = s_need[e] != 0u;
     s_need[e] = need ? run : kNanKey;
     run += need ? size[k] : 0u;
@@ -518,8 +512,8 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(
   __syncthreads();
   uint32_t* ts = seg + int64_t(tile) * kBuckets * kTile;
   for (int e = threadIdx.x; e < kBuckets * kTile; e += kThreads) {
-    tt[e] = s_first[e];
-    ts[e] = s_need[e];
+    tt[e] = s_first[at(e / kTile, e % kTile)];
+    ts[e] = s_need[at(e / kTile, e % kTile)];
   }
 }
 
@@ -771,11 +765,11 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
     int dev = 0, cus = 0;
     DP_HIP(hipGetDevice(&dev));
     DP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    constexpr size_t lds = size_t(2) * kBuckets * kTile * sizeof(uint32_t);
     for (const void* k : {reinterpret_cast<const void*>(&bucket_kernel<false>),
-                          reinterpret_cast<const void*>(bucket_kernel<true>),
-                          reinterpret_cast<const void*>(plan_kernel)})
-      DP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+                          reinterpret_cast<const void*>(&bucket_kernel<true>)})
+      DP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(kBucketLds)));
+    DP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(plan_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kPlanLds)));
     // Blocks of features bound the tables (about 12 KiB a feature and chunk).
     constexpr int32_t kBlock = 1 << 16;
     for (int32_t f0 = 0; f0 < n_features; f0 += kBlock) {
@@ -799,13 +793,13 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
                          n_rows, n_features, f0, fc, max_bin, bounds.p, used.p, many);
       DP_HIP(hipGetLastError());
       const dim3 grid(unsigned((tiles * chunks + 7) / 8 * 8));
-      hipLaunchKernelGGL(bucket_kernel<false>, grid, dim3(kThreads), lds, s, values, n_rows,
+      hipLaunchKernelGGL(bucket_kernel<false>, grid, dim3(kThreads), kBucketLds, s, values, n_rows,
                          n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, slots.p,
                          nullptr, nullptr, nullptr);
       DP_HIP(hipGetLastError());
       hipLaunchKernelGGL(offsets_kernel, dim3(unsigned((table + 255) / 256)), dim3(256), 0, s,
                          slots.p, int64_t(table), chunks, totals.p);
-      hipLaunchKernelGGL(plan_kernel, dim3(tiles), dim3(kThreads), lds, s, bounds.p, many, fc,
+      hipLaunchKernelGGL(plan_kernel, dim3(tiles), dim3(kThreads), kPlanLds, s, bounds.p, many, fc,
                          max_bin, totals.p, seg.p, rank_bucket.p, plans.p, gathered.p);
       DP_HIP(hipGetLastError());
       unsigned long long n_keys = 0;
@@ -817,7 +811,7 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
         size_t cap = 1 << 16;
         while (cap < n_keys) cap += std::max<size_t>(1 << 16, cap / 8);
         if (keys.n < cap) keys.resize(cap);
-        hipLaunchKernelGGL(bucket_kernel<true>, grid, dim3(kThreads), lds, s, values, n_rows,
+        hipLaunchKernelGGL(bucket_kernel<true>, grid, dim3(kThreads), kBucketLds, s, values, n_rows,
                            n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, slots.p,
                            seg.p, plans.p, keys.p);
         DP_HIP(hipGetLastError());

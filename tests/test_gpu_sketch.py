@@ -1,4 +1,4 @@
-"""Quantile cuts against the oracle at the sizes and value patterns where the bucket
+"""Quantile cuts and bins against the oracle at the sizes and value patterns where the bucket
 passes change course: the row counts around the in-LDS sort and the sample, features
 whose distinct values are few, rare, repeated or adjacent, and missing values."""
 import numpy as np
@@ -49,4 +49,9 @@ def test_cuts_match_the_oracle(dp, oracle, ws, device, n, max_bin):
             got, want = cuts[ptr[f]:ptr[f + 1]], o_cuts[o_ptr[f]:o_ptr[f + 1]]
             np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=name)
         np.testing.assert_array_equal(mins.view(np.uint32), o_mins.view(np.uint32))
+        if max_bin <= 255:  # byte 255 marks a missing value
+            lay = ops.layout(n, width, 0, 255)
+            bins = ops.bin_values(torch.as_tensor(part, device=device), lay, ptr, cuts)
+            np.testing.assert_array_equal(ops.from_tiles(bins.cpu().numpy(), lay),
+                                          oracle.bin_matrix(part, o_ptr, o_cuts, 255))
         assert missing == bool(np.isnan(part).any())
