@@ -23,7 +23,6 @@
 #include <limits>
 
 #include "json.hpp"
-#include "predict.hpp"
 #include "tune.hpp"
 
 namespace dp {
@@ -1550,43 +1549,24 @@ void Booster::upload_forest(int32_t tree_begin, int32_t tree_end) {
   flush();
   if (forest_begin_ == tree_begin && forest_end_ == tree_end && forest_trees_ == trees_.size())
     return;
-  std::vector<PredNode> nodes;
-  std::vector<int32_t> roots;
-  std::vector<std::vector<int32_t>> per_group(size_t(std::max(n_groups_, 1)));
+  std::vector<ForestTree> trees;
   for (int32_t t = tree_begin; t < tree_end; ++t) {
     const Tree& tr = trees_[size_t(t)];
-    const int32_t base = int32_t(nodes.size());
+    ForestTree f;
+    f.group = tree_info_[size_t(t)];
     for (int32_t i = 0; i < tr.size(); ++i) {
       const bool leaf = tr.left[size_t(i)] == -1;
-      nodes.push_back({leaf ? -1 : base + tr.left[size_t(i)], leaf ? 0 : tr.feature[size_t(i)],
-                       tr.cond[size_t(i)], leaf ? 0 : int32_t(tr.default_left[size_t(i)])});
+      f.nodes.push_back({leaf ? -1 : tr.left[size_t(i)], leaf ? 0 : tr.feature[size_t(i)],
+                         tr.cond[size_t(i)], leaf ? 0 : int32_t(tr.default_left[size_t(i)])});
     }
-    per_group[size_t(tree_info_[size_t(t)])].push_back(base);
-  }
-  std::vector<int32_t> group_ptr{0};
-  for (const auto& g : per_group) {
-    roots.insert(roots.end(), g.begin(), g.end());
-    group_ptr.push_back(int32_t(roots.size()));
+    trees.push_back(std::move(f));
   }
   std::vector<float> base(size_t(std::max(n_groups_, 1)));
   for (size_t k = 0; k < base.size(); ++k) {
     const float b = base_score_.empty() ? 0.0f : base_score_[k < base_score_.size() ? k : 0];
     base[k] = objective_id_ == DP_OBJ_LOGISTIC ? float(std::log(double(b) / (1.0 - double(b)))) : b;
   }
-  forest_nodes_.resize(std::max<size_t>(nodes.size(), 1) * sizeof(PredNode));
-  forest_roots_.resize(std::max<size_t>(roots.size(), 1));
-  forest_group_ptr_.resize(group_ptr.size());
-  forest_base_.resize(base.size());
-  if (!nodes.empty())
-    DP_HIP(hipMemcpy(forest_nodes_.p, nodes.data(), nodes.size() * sizeof(PredNode),
-                     hipMemcpyHostToDevice));
-  if (!roots.empty())
-    DP_HIP(hipMemcpy(forest_roots_.p, roots.data(), roots.size() * sizeof(int32_t),
-                     hipMemcpyHostToDevice));
-  DP_HIP(hipMemcpy(forest_group_ptr_.p, group_ptr.data(), group_ptr.size() * sizeof(int32_t),
-                   hipMemcpyHostToDevice));
-  DP_HIP(hipMemcpy(forest_base_.p, base.data(), base.size() * sizeof(float),
-                   hipMemcpyHostToDevice));
+  build_forest(trees, base, n_features_, forest_);
   forest_begin_ = tree_begin;
   forest_end_ = tree_end;
   forest_trees_ = trees_.size();
@@ -1613,9 +1593,8 @@ const float* Booster::predict(const PredictRequest& req, std::vector<uint64_t>& 
   upload_forest(iteration_indptr_[size_t(begin)], iteration_indptr_[size_t(end)]);
   pred_out_.reserve(size_t(std::max<int64_t>(req.rows, 1)) * size_t(n_groups_));
   hipStream_t s = stream_;
-  launch_predict(req.values, req.rows, req.features, req.row_stride, req.missing,
-                 reinterpret_cast<const PredNode*>(forest_nodes_.p), forest_roots_.p,
-                 forest_group_ptr_.p, n_groups_, forest_base_.p, transform, pred_out_.p, s);
+  launch_predict(req.values, req.rows, req.features, req.row_stride, req.missing, forest_,
+                 transform, pred_out_.p, s);
   DP_HIP(hipStreamSynchronize(s));
   shape.clear();
   shape.push_back(uint64_t(req.rows));

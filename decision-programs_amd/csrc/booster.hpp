@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "dp_internal.hpp"
+#include "predict.hpp"
 
 namespace dp {
 
@@ -330,9 +331,8 @@ class Booster {
   mutable int rounds_ = 0;
   bool model_only_ = false;  // loaded or sliced: predicts, cannot train
   // device forest for prediction
-  DeviceBuffer<uint8_t> forest_nodes_;
-  DeviceBuffer<int32_t> forest_roots_, forest_group_ptr_;
-  DeviceBuffer<float> forest_base_, pred_out_;
+  Forest forest_;
+  DeviceBuffer<float> pred_out_;
   int32_t forest_begin_ = -1, forest_end_ = -1;
   size_t forest_trees_ = 0;
 };

@@ -1,18 +1,14 @@
-// Flattened forest for device prediction.
+// Forest prediction on the device.
 #pragma once
 
 #include <cstdint>
+#include <vector>
 
 #include <hip/hip_runtime.h>
 
-namespace dp {
+#include "dp_internal.hpp"
 
-struct PredNode {
-  int32_t left;     // absolute index of the left child, -1 for a leaf
-  int32_t feature;  // split feature
-  float cond;       // threshold (x < cond goes left), or the leaf value
-  int32_t flags;    // bit 0: missing goes left
-};
+namespace dp {
 
 enum PredTransform : int32_t {
   kPredIdentity = 0,  // margins (type 1) or regression values
@@ -21,9 +17,49 @@ enum PredTransform : int32_t {
   kPredArgmax = 3,    // multi:softmax class ids
 };
 
+// One tree node of the general form.
+struct PredNode {
+  int32_t left;     // left child's index in its tree (right = left + 1), -1 for a leaf
+  int32_t feature;  // split feature
+  float cond;       // threshold (x < cond goes left), or the leaf value
+  int32_t flags;    // bit 0: missing goes left
+};
+
+// The same in 8 bytes, for trees of at most 65,536 nodes over at most 32,768
+// features: bits 0-15 of `word` the left child's index (0: a leaf), bit 16
+// missing goes left, bits 17-31 the feature.
+struct PackedNode {
+  float cond;
+  uint32_t word;
+};
+
+// A forest laid out for prediction: trees grouped by output, in boosting order
+// within each.
+struct Forest {
+  DeviceBuffer<uint8_t> nodes;       // PackedNode or PredNode
+  DeviceBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
+  DeviceBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
+  DeviceBuffer<int32_t> batch_ptr;   // [batches + 1] first tree of each batch of
+                                     // trees whose nodes fit kPredBatchNodes
+  DeviceBuffer<float> base;          // [groups] margin before the first tree
+  bool packed = false;
+  int32_t trees = 0, groups = 1;
+  int32_t batches = 0;  // 0: some tree alone exceeds kPredBatchNodes (or is not packed)
+};
+
+constexpr int32_t kPredBatchNodes = 4096;
+
+// Host-side description of one tree for build_forest.
+struct ForestTree {
+  int32_t group;
+  std::vector<PredNode> nodes;
+};
+// trees: in boosting order.
+void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>& base,
+                  int32_t n_features, Forest& out);
+
 void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int64_t row_stride,
-                    float missing, const PredNode* nodes, const int32_t* group_roots,
-                    const int32_t* group_ptr, int32_t n_groups, const float* base,
-                    int32_t transform, float* out, hipStream_t s);
+                    float missing, const Forest& forest, int32_t transform, float* out,
+                    hipStream_t s);
 
 }  // namespace dp
