@@ -1275,7 +1275,7 @@ void Booster::run_round(DMatrix* d, bool with_gradients) {
       launch_quantise(grad_.p, hess_.p, N, K, quant_scratch_.p, maxima, exps_.p, gpair_.p,
                       nullptr, stream_, rows);
     }
-    const int32_t blocks = quantise_blocks(N);
+    const int32_t blocks = quantise_blocks(N, K);
     const int64_t* slots = quantise_sum_slots(quant_scratch_.p, N, K);
     auto sample_columns = [&](Grower& g, int32_t k) {
       g.colsample = ColSample{};

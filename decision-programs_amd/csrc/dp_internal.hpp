@@ -680,8 +680,8 @@ constexpr int64_t kLeafChunk = 16384;  // margin-update items of the operator AP
 void launch_init_margin(float* margin, int64_t n_rows, int32_t n_outputs, const float* base,
                         hipStream_t s);
 
-// Objective gradients.  With quant_scratch (quantise_scratch_bytes) and one
-// output, the per-workgroup maxima the quantiser needs are written too and
+// Objective gradients.  With quant_scratch (quantise_scratch_bytes) and at most
+// 256 outputs, the per-workgroup maxima the quantiser needs are written too and
 // true is returned (pass maxima_ready to launch_quantise).
 // values (optional, planes [n_classes][n_rows]): leaf values added to the
 // margins first (margin[r * n_classes + k] += values[k * n_rows + r], stored),
@@ -695,9 +695,9 @@ bool launch_gradients(int32_t objective, float* margin, const float* label,
 // Most workgroups (and reduction slots) per class: eight 256-thread workgroups
 // per CU keep enough loads in flight for the streaming passes over 10M rows.
 constexpr int kQuantBlocks = 2048;
-int quantise_blocks(int64_t n_rows);
+int quantise_blocks(int64_t n_rows, int32_t n_classes);
 // The quantiser's int64 sum slots in its scratch: class k's quantise_blocks
-// (g, h) pairs start at pair k * quantise_blocks(n_rows).
+// (g, h) pairs start at pair k * quantise_blocks(n_rows, n_classes).
 const int64_t* quantise_sum_slots(const void* scratch, int64_t n_rows, int32_t n_classes);
 size_t quantise_scratch_bytes(int64_t n_rows, int32_t n_classes);
 // rows: row sampling of the round (inactive by default): a dropped row's

@@ -15,10 +15,11 @@
 // exact int64.  Maxima (integer max of the bit patterns of |x|) and sums are
 // reduced through per-workgroup slots, never by same-address atomics (512
 // workgroups on one word serialise): each quantiser workgroup reduces the
-// maxima slots itself, and a finishing kernel reduces the sum slots.  Single-
-// output objectives produce the maxima slots in the gradient kernel.
+// maxima slots itself, and a finishing kernel reduces the sum slots.  The
+// gradient kernels produce the maxima slots too (up to 256 outputs).
 #include "dp_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace dp {
@@ -250,6 +251,245 @@ __global__ __launch_bounds__(kQuantThreads) void finish_sums_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Several outputs (2 .. kQuantThreads): [n_rows][n_classes] arrays
+// ---------------------------------------------------------------------------
+// The arrays are walked flat, so that every access is coalesced: a workgroup's
+// first `lanes` threads (the largest multiple of the class count) take adjacent
+// elements, kQuantThreads / n_classes rows a sweep, and a thread's class never
+// changes, so its class's maxima and sums stay in registers.  Work along a row
+// (the softmax's maximum and its sum in class order) or along a class (the
+// pairs' planes) goes through LDS.  Memory bounds them.  A thread per row, and a
+// grid of workgroups per class, had every access `n_classes` elements from its
+// neighbour's: 166 us for the gradients, 108 for the maxima and 125 for the
+// pairs of 1M rows x 10; now 33, 16 and 48 us.
+constexpr int kSweeps = 8;  // sweeps whose loads are in flight together
+
+struct ClassLanes {
+  int k, row, rows;  // the thread's class, its first row of a sweep, rows a sweep
+  bool live;
+  __device__ __forceinline__ explicit ClassLanes(int n_classes) {
+    rows = kQuantThreads / n_classes;
+    live = int(threadIdx.x) < rows * n_classes;
+    row = int(threadIdx.x) / n_classes;
+    k = int(threadIdx.x) - row * n_classes;
+  }
+};
+
+// Largest (a, b) over the threads of each class; threads t < n_classes get class
+// t's.  s: kQuantThreads LDS pairs.
+__device__ __forceinline__ uint2 class_max(const ClassLanes& l, int n_classes, unsigned a,
+                                           unsigned b, uint2* s) {
+  __syncthreads();
+  s[threadIdx.x] = make_uint2(a, b);
+  __syncthreads();
+  uint2 m = make_uint2(0u, 0u);
+  if (int(threadIdx.x) < n_classes)
+    for (int i = 0; i < l.rows; ++i) {
+      const uint2 v = s[i * n_classes + int(threadIdx.x)];
+      m = make_uint2(max(m.x, v.x), max(m.y, v.y));
+    }
+  return m;
+}
+
+// Rows of a softmax tile in LDS: rows of n_classes | 1 words (an odd stride, so
+// that the threads of a row pass use different banks).
+constexpr int kSoftWords = 8192;
+__host__ __device__ __forceinline__ int soft_rows(int n_classes) {
+  const int r = kSoftWords / (n_classes | 1);
+  return r < kQuantThreads ? r : kQuantThreads;
+}
+
+template <bool MAXIMA>
+__global__ __launch_bounds__(kQuantThreads) void softprob_kernel(
+    float* __restrict__ margin, const float* __restrict__ label, int64_t n_rows, int n_classes,
+    float* __restrict__ grad, float* __restrict__ hess, uint2* __restrict__ max_slots,
+    const float* __restrict__ values) {
+  __shared__ __attribute__((aligned(16))) float s[kSoftWords];
+  __shared__ float s_max[kQuantThreads], s_sum[kQuantThreads];
+  __shared__ int s_label[kQuantThreads];
+  const ClassLanes l(n_classes);
+  const int stride = n_classes | 1, tile = soft_rows(n_classes);
+  unsigned mg = 0, mh = 0;
+  for (int64_t r0 = int64_t(blockIdx.x) * tile; r0 < n_rows; r0 += int64_t(gridDim.x) * tile) {
+    const int n = int(min(int64_t(tile), n_rows - r0));
+    const int end = l.live ? n : 0;
+    const int y = int(label[r0 + min(int(threadIdx.x), n - 1)]);
+    for (int rb = l.row; rb < end; rb += kSweeps * l.rows) {
+      float m[kSweeps], v[kSweeps];
+#pragma unroll
+      for (int u = 0; u < kSweeps; ++u) {
+        const int64_t r = r0 + min(rb + u * l.rows, n - 1);
+        m[u] = margin[r * n_classes + l.k];
+        v[u] = values ? values[int64_t(l.k) * n_rows + r] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < kSweeps; ++u) {
+        const int r = rb + u * l.rows;
+        if (r >= n) break;
+        if (values) {  // the previous round's leaf values first, as in gradients_kernel
+          m[u] = m[u] + v[u];
+          margin[(r0 + r) * n_classes + l.k] = m[u];
+        }
+        s[r * stride + l.k] = m[u];
+      }
+    }
+    __syncthreads();
+    if (int(threadIdx.x) < n) {
+      const float* row = s + int(threadIdx.x) * stride;
+      float mx = row[0];
+      for (int k = 1; k < n_classes; ++k) mx = fmaxf(mx, row[k]);
+      s_max[threadIdx.x] = mx;
+    }
+    __syncthreads();
+    for (int r = l.row; r < end; r += l.rows)
+      s[r * stride + l.k] = dp_expf(s[r * stride + l.k] - s_max[r]);
+    __syncthreads();
+    if (int(threadIdx.x) < n) {
+      const float* row = s + int(threadIdx.x) * stride;
+      float t = 0.0f;
+      for (int k = 0; k < n_classes; ++k) t += row[k];
+      s_sum[threadIdx.x] = t;
+      s_label[threadIdx.x] = y;
+    }
+    __syncthreads();
+    for (int r = l.row; r < end; r += l.rows) {
+      const float p = s[r * stride + l.k] / s_sum[r];
+      const float g = p - (l.k == s_label[r] ? 1.0f : 0.0f);
+      const float h = fmaxf(2.0f * p * (1.0f - p), 1e-16f);
+      const int64_t e = (r0 + r) * n_classes + l.k;
+      grad[e] = g;
+      hess[e] = h;
+      mg = max(mg, __float_as_uint(fabsf(g)));
+      mh = max(mh, __float_as_uint(fabsf(h)));
+    }
+    __syncthreads();
+  }
+  if constexpr (MAXIMA) {
+    const uint2 m = class_max(l, n_classes, mg, mh, reinterpret_cast<uint2*>(s));
+    if (int(threadIdx.x) < n_classes)
+      max_slots[int64_t(threadIdx.x) * gridDim.x + blockIdx.x] = m;
+  }
+}
+
+__global__ __launch_bounds__(kQuantThreads) void class_absmax_kernel(
+    const float* __restrict__ grad, const float* __restrict__ hess, int64_t n_rows,
+    int n_classes, uint2* __restrict__ max_slots, RowSample rs) {
+  __shared__ uint2 s[kQuantThreads];
+  const ClassLanes l(n_classes);
+  const uint64_t prefix = row_prefix(rs, l.k);
+  unsigned mg = 0, mh = 0;
+  const int64_t step = int64_t(gridDim.x) * l.rows;
+  for (int64_t rb = int64_t(blockIdx.x) * l.rows + l.row; l.live && rb < n_rows;
+       rb += kSweeps * step) {
+    float g[kSweeps], h[kSweeps];
+#pragma unroll
+    for (int u = 0; u < kSweeps; ++u) {
+      const int64_t r = min(rb + u * step, n_rows - 1);
+      g[u] = grad[r * n_classes + l.k];
+      h[u] = hess[r * n_classes + l.k];
+    }
+#pragma unroll
+    for (int u = 0; u < kSweeps; ++u) {
+      const int64_t r = rb + u * step;
+      if (r >= n_rows || !row_kept(rs, prefix, r)) continue;
+      mg = max(mg, __float_as_uint(fabsf(g[u])));
+      mh = max(mh, __float_as_uint(fabsf(h[u])));
+    }
+  }
+  const uint2 m = class_max(l, n_classes, mg, mh, s);
+  if (int(threadIdx.x) < n_classes) max_slots[int64_t(threadIdx.x) * gridDim.x + blockIdx.x] = m;
+}
+
+// Rows of a quantiser tile: planes of rows + 1 pairs per class in LDS.
+constexpr int kQuantPairs = 2048;
+__host__ __device__ __forceinline__ int quant_rows(int n_classes) {
+  const int r = kQuantPairs / n_classes - 1;
+  return r < kQuantThreads ? r : kQuantThreads;
+}
+
+__global__ __launch_bounds__(kQuantThreads) void class_quantise_kernel(
+    const float* __restrict__ grad, const float* __restrict__ hess, int64_t n_rows,
+    int n_classes, const uint2* __restrict__ max_slots, int32_t* __restrict__ exps,
+    int2* __restrict__ gpair, long long* __restrict__ sum_slots, RowSample rs) {
+  __shared__ __attribute__((aligned(16))) int2 s[kQuantPairs];
+  __shared__ int2 s_exp[kQuantThreads];
+  const ClassLanes l(n_classes);
+  const int lane = threadIdx.x & 63;
+  // Every workgroup reduces the classes' maxima slots, a wavefront per class.
+  for (int k = int(threadIdx.x) >> 6; k < n_classes; k += kQuantThreads / 64) {
+    const uint2* slots = max_slots + int64_t(k) * gridDim.x;
+    unsigned a = 0, b = 0;
+    for (int i = lane; i < int(gridDim.x); i += 64) {
+      const uint2 v = slots[i];
+      a = max(a, v.x);
+      b = max(b, v.y);
+    }
+    for (int d = 32; d >= 1; d >>= 1) {
+      a = max(a, __shfl_xor(a, d, 64));
+      b = max(b, __shfl_xor(b, d, 64));
+    }
+    if (lane == 0) {
+      const int2 e = make_int2(quant_exp(a), quant_exp(b));
+      s_exp[k] = e;
+      if (blockIdx.x == 0) {
+        exps[2 * k] = e.x;
+        exps[2 * k + 1] = e.y;
+      }
+    }
+  }
+  __syncthreads();
+  const int2 ex = s_exp[l.k];
+  const uint64_t prefix = row_prefix(rs, l.k);
+  const int tile = quant_rows(n_classes), plane = tile + 1;
+  long long sg = 0, sh = 0;
+  for (int64_t r0 = int64_t(blockIdx.x) * tile; r0 < n_rows; r0 += int64_t(gridDim.x) * tile) {
+    const int n = int(min(int64_t(tile), n_rows - r0));
+    for (int rb = l.row; l.live && rb < n; rb += kSweeps * l.rows) {
+      float g[kSweeps], h[kSweeps];
+#pragma unroll
+      for (int u = 0; u < kSweeps; ++u) {
+        const int64_t e = (r0 + min(rb + u * l.rows, n - 1)) * n_classes + l.k;
+        g[u] = grad[e];
+        h[u] = hess[e];
+      }
+#pragma unroll
+      for (int u = 0; u < kSweeps; ++u) {
+        const int r = rb + u * l.rows;
+        if (r >= n) break;
+        const bool kept = row_kept(rs, prefix, r0 + r);
+        const int qg = kept ? int(rintf(ldexpf(g[u], ex.x))) : 0;
+        const int qh = kept ? int(rintf(ldexpf(h[u], ex.y))) : 0;
+        s[l.k * plane + r] = make_int2(qg, qh);
+        sg += qg;
+        sh += qh;
+      }
+    }
+    __syncthreads();
+    // The classes' planes, a wavefront's 64 rows of one class at a time.
+    const int runs = (n + 63) / 64;
+    for (int i = int(threadIdx.x) >> 6; i < runs * n_classes; i += kQuantThreads / 64) {
+      const int k = i / runs, r = (i - k * runs) * 64 + lane;
+      if (r < n) gpair[int64_t(k) * n_rows + r0 + r] = s[k * plane + r];
+    }
+    __syncthreads();
+  }
+  // The classes' sums, in the LDS of the planes.
+  longlong2* part = reinterpret_cast<longlong2*>(s);
+  part[threadIdx.x] = make_longlong2(sg, sh);
+  __syncthreads();
+  if (int(threadIdx.x) < n_classes) {
+    long long tg = 0, th = 0;
+    for (int i = 0; i < l.rows; ++i) {
+      tg += part[i * n_classes + int(threadIdx.x)].x;
+      th += part[i * n_classes + int(threadIdx.x)].y;
+    }
+    long long* slot = sum_slots + (int64_t(threadIdx.x) * gridDim.x + blockIdx.x) * 2;
+    slot[0] = tg;
+    slot[1] = th;
+  }
+}
+
 // Label checks in the spirit of the reference's prepare_labels
 // (class_native_training.cuh:36-41): class ids must be exact integers in [0, K),
 // logistic labels in [0, 1], regression labels finite.
@@ -288,15 +528,24 @@ void launch_check_labels(const float* label, int64_t n, int32_t objective, int32
   DP_HIP(hipGetLastError());
 }
 
-// At least four rows per thread: every quantise workgroup re-reads all the
-// maxima slots, so a 1M-row pass keeps about 1,000 of them (four per CU; eight
-// rows per thread measured 0.8 % slower on C2's trees), a 10M-row one 2048.
-int quantise_blocks(int64_t n_rows) {
-  return grid_for(n_rows, kQuantThreads * 4, kQuantBlocks);
+// The classes that the flat kernels take (one output: the kernels above; more
+// than a workgroup has threads: one workgroup grid per class).
+static bool flat_classes(int32_t n_classes) {
+  return n_classes >= 2 && n_classes <= kQuantThreads;
+}
+
+// One output: at least four rows per thread, since every quantise workgroup
+// re-reads all the maxima slots: a 1M-row pass keeps about 1,000 of them (four per
+// CU; eight rows per thread measured 0.8 % slower on C2's trees), a 10M-row one
+// 2048.  Several: a tile of rows each, at most 1,024 workgroups and, again for
+// the slots every one of them reads, at most 16,384 slots.
+int quantise_blocks(int64_t n_rows, int32_t n_classes) {
+  if (!flat_classes(n_classes)) return grid_for(n_rows, kQuantThreads * 4, kQuantBlocks);
+  return grid_for(n_rows, quant_rows(n_classes), std::clamp(16384 / n_classes, 64, 1024));
 }
 
 size_t quantise_scratch_bytes(int64_t n_rows, int32_t n_classes) {
-  const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows));
+  const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows, n_classes));
   return slots * 2 * sizeof(uint32_t) + 256 + slots * 2 * sizeof(int64_t);
 }
 
@@ -315,8 +564,17 @@ bool launch_gradients(int32_t objective, float* margin, const float* label,
   need(objective == DP_OBJ_LOGISTIC || objective == DP_OBJ_SOFTPROB ||
            objective == DP_OBJ_SQUARED,
        "unknown objective id");
+  if (objective == DP_OBJ_SOFTPROB && flat_classes(n_classes)) {
+    const auto kernel = quant_scratch ? softprob_kernel<true> : softprob_kernel<false>;
+    const int blocks = quant_scratch ? quantise_blocks(n_rows, n_classes)
+                                     : grid_for(n_rows, soft_rows(n_classes), 4096);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kQuantThreads), 0, s, margin, label, n_rows,
+                       n_classes, grad, hess, static_cast<uint2*>(quant_scratch), values);
+    DP_HIP(hipGetLastError());
+    return quant_scratch != nullptr;
+  }
   if (quant_scratch && n_classes == 1) {
-    hipLaunchKernelGGL(gradients_kernel<true>, dim3(quantise_blocks(n_rows)), dim3(kQuantThreads),
+    hipLaunchKernelGGL(gradients_kernel<true>, dim3(quantise_blocks(n_rows, n_classes)), dim3(kQuantThreads),
                        0, s, objective, margin, label, n_rows, n_classes, grad, hess,
                        static_cast<unsigned*>(quant_scratch), values);
     DP_HIP(hipGetLastError());
@@ -343,17 +601,28 @@ void launch_quantise(const float* grad, const float* hess, int64_t n_rows, int32
   need(!(rows.active() && maxima_ready), "row sampling needs the sampled maxima");
   need(n_classes >= 1 && n_classes <= 65535, "class count out of range");
   need(n_rows >= 1, "quantiser needs at least one row");
-  const int blocks = quantise_blocks(n_rows);
+  const int blocks = quantise_blocks(n_rows, n_classes);
   const size_t slots = size_t(n_classes) * size_t(blocks);
   auto* max_slots = static_cast<unsigned*>(scratch);
   auto* sum_slots = reinterpret_cast<long long*>(static_cast<uint8_t*>(scratch) +
                                                  ((slots * 2 * sizeof(uint32_t) + 255) & ~size_t(255)));
+  const bool flat = flat_classes(n_classes);
+  auto* pair_slots = reinterpret_cast<uint2*>(max_slots);
   if (!maxima_ready) {
-    hipLaunchKernelGGL(absmax_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
-                       hess, n_rows, n_classes, max_slots, rows);
+    if (flat)
+      hipLaunchKernelGGL(class_absmax_kernel, dim3(blocks), dim3(kQuantThreads), 0, s, grad, hess,
+                         n_rows, n_classes, pair_slots, rows);
+    else
+      hipLaunchKernelGGL(absmax_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
+                         hess, n_rows, n_classes, max_slots, rows);
     DP_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(quantise_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
+  if (flat)
+    hipLaunchKernelGGL(class_quantise_kernel, dim3(blocks), dim3(kQuantThreads), 0, s, grad, hess,
+                       n_rows, n_classes, pair_slots, exps, reinterpret_cast<int2*>(gpair),
+                       sum_slots, rows);
+  else
+    hipLaunchKernelGGL(quantise_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
                      hess, n_rows, n_classes, max_slots, exps, reinterpret_cast<int2*>(gpair),
                      sum_slots, rows);
   DP_HIP(hipGetLastError());
@@ -364,7 +633,7 @@ void launch_quantise(const float* grad, const float* hess, int64_t n_rows, int32
 }
 
 const int64_t* quantise_sum_slots(const void* scratch, int64_t n_rows, int32_t n_classes) {
-  const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows));
+  const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows, n_classes));
   return reinterpret_cast<const int64_t*>(static_cast<const uint8_t*>(scratch) +
                                           ((slots * 2 * sizeof(uint32_t) + 255) & ~size_t(255)));
 }
