@@ -29,7 +29,8 @@ namespace {
 // 16 bytes per value with 65-256 bins, bound it.  The row-per-thread kernel it
 // replaced (16 strided loads, 8 binary steps of one word each) took 0.70 ms for
 // 1M x 100 and 12.9 ms for 2M x 1,000 with 95 % missing, and the column copy a
-// pass of its own (0.71 ms at the latter); now 0.26 and 4.7 ms, copy included.
+// pass of its own (0.71 ms at the latter); now 0.20 and 4.6 ms, copy included.
+constexpr int32_t kBinFeatures = 1 << 20;
 constexpr int kBinRows = 8;
 constexpr int kBinThreads = 256;
 
@@ -59,23 +60,33 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
     return order_key(cut_values[cut_ptr[f] + p - 1]);
   });
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int j = lane & 15, f = f0 + j;
   const bool live = f < n_features;
   uint8_t* tile = WIDE ? nullptr : bins + int64_t(f0 / kTile) * n_rows * kTile;
   const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
   constexpr int kWaveRows = 4 * kBinRows;
+  // Loads from wave-uniform bases and one 32-bit byte offset per lane (below 2^32
+  // for the 2^20 features a matrix may have): no branches and no address
+  // arithmetic, so all are in flight before the first wait.
+  const uint32_t offset = (uint32_t((lane >> 4) * kBinRows) * uint32_t(n_features) +
+                           uint32_t(min(f, n_features - 1))) * 4u;
   for (int64_t w0 = chunk * chunk_rows + wave * kWaveRows; w0 < r1;
        w0 += kBinThreads / 64 * kWaveRows) {
     const int64_t r0 = w0 + (lane >> 4) * kBinRows;
-    // Loads without branches (rows and features past the end repeat the last),
-    // so that all are in flight before the first is waited for.
+    const float* base = values + w0 * n_features;
     float x[kBinRows];
     uint32_t key[kBinRows];
     int bin[kBinRows];
+    if (w0 + kWaveRows <= r1) {
 #pragma unroll
-    for (int u = 0; u < kBinRows; ++u)
-      x[u] = values[min(r0 + u, r1 - 1) * n_features + min(f, n_features - 1)];
+      for (int u = 0; u < kBinRows; ++u) x[u] = load_at(base + int64_t(u) * n_features, offset);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kBinRows; ++u)
+        x[u] = r0 + u < r1 ? load_at(base + int64_t(u) * n_features, offset) : 0.0f;
+    }
 #pragma unroll
     for (int u = 0; u < kBinRows; ++u) key[u] = order_key(x[u]) & (live ? ~0u : 0u);
     search<kBinRows>(tree, levels, j, key, bin);
@@ -506,6 +517,7 @@ void launch_bin_values(const float* values, const dp_bin_layout& layout, const i
                        const float* cut_values, uint8_t* bins, uint8_t* cols, hipStream_t s) {
   if (layout.n_rows <= 0) return;
   need(layout.tile_width == kTile, "binning needs 16-feature tiles");
+  need(layout.n_features <= kBinFeatures, "too many features to bin");
   const int32_t chunks = bin_chunks(layout.n_rows, layout.n_tiles);
   hipLaunchKernelGGL(bin_kernel<false>, dim3(unsigned((layout.n_tiles * chunks + 7) / 8 * 8)),
                      dim3(kBinThreads), 0, s, values, layout.n_rows, layout.n_features, cut_ptr,
@@ -519,6 +531,7 @@ void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_feature
                           const int32_t* cut_ptr, const float* cut_values, uint16_t* cols,
                           hipStream_t s) {
   if (n_rows <= 0 || n_features <= 0) return;
+  need(n_features <= kBinFeatures, "too many features to bin");
   const int32_t tiles = (n_features + kTile - 1) / kTile, chunks = bin_chunks(n_rows, tiles);
   hipLaunchKernelGGL(bin_kernel<true>, dim3(unsigned((tiles * chunks + 7) / 8 * 8)),
                      dim3(kBinThreads), 0, s, values, n_rows, n_features, cut_ptr, cut_values,

@@ -29,6 +29,16 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
+// *(base + byte offset) with a wave-uniform base: one load with a scalar base and a
+// 32-bit vector offset (the empty asm keeps the compiler from folding the two into
+// 64-bit vector additions per load).
+__device__ __forceinline__ float load_at(const float* base, uint32_t offset) {
+  uint64_t b = reinterpret_cast<uint64_t>(base);
+  asm("" : "+s"(b));
+  const auto* p = reinterpret_cast<const __attribute__((address_space(1))) char*>(b) + offset;
+  return *reinterpret_cast<const __attribute__((address_space(1))) float*>(p);
+}
+
 constexpr int kTile = 16;  // features of a tile
 
 constexpr int search_nodes(int levels) { return ((1 << (2 * levels)) - 1) / 3; }

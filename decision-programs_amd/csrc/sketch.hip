@@ -32,7 +32,7 @@
 // Two reads of the matrix and its binary searches bound it.  Sorting every
 // feature (a radix sort each) moved 8 to 10 times the bytes in 4 to 21 launches
 // per feature.  Device time before and now: 1M x 100, 20 % missing, 255 bins
-// 19.0 -> 0.91 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 9.2 ms; 1M x 28 4.2
+// 19.0 -> 0.84 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 8.4 ms; 1M x 28 4.2
 // -> 0.3 ms; 10k x 8 0.22 -> 0.06 ms.
 #include "dp_internal.hpp"
 #include "search.hpp"
@@ -359,17 +359,29 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
   if constexpr (GATHER) keys = live ? out + plans[tile * kTile + j].base : nullptr;
   __syncthreads();
   const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
-  for (int64_t r0 = chunk * chunk_rows + (threadIdx.x >> 4); r0 < r1; r0 += 64 * kRows) {
-    // Loads without branches, so that all are in flight before the first wait.
+  // Loads from wave-uniform bases and one 32-bit byte offset per lane: no branches
+  // and no address arithmetic, so all are in flight before the first wait.
+  const int lane4 = int(threadIdx.x >> 4) & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const uint32_t offset =
+      (uint32_t(lane4) * uint32_t(n_features) + uint32_t(min(f, n_features - 1))) * 4u;
+  auto step = [&](const float* base, int64_t rows) {  // rows: of this step, 64 * kRows or fewer
     float x[kRows];
     uint32_t key[kRows];
     int pos[kRows];
+    if (rows >= 64 * kRows) {
 #pragma unroll
-    for (int u = 0; u < kRows; ++u)
-      x[u] = values[min(r0 + u * 64, r1 - 1) * n_features + min(f, n_features - 1)];
+      for (int u = 0; u < kRows; ++u)
+        x[u] = load_at(base + int64_t(wave * 4 + u * 64) * n_features, offset);
+    } else {
 #pragma unroll
-    for (int u = 0; u < kRows; ++u)
-      key[u] = order_key(x[u]) | (live && r0 + u * 64 < r1 ? 0u : ~0u);
+      for (int u = 0; u < kRows; ++u)
+        x[u] = wave * 4 + lane4 + u * 64 < rows
+                   ? load_at(base + int64_t(wave * 4 + u * 64) * n_features, offset)
+                   : __builtin_nanf("");
+    }
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) key[u] = order_key(x[u]) | (live ? 0u : ~0u);
     search<kRows>(tree, levels, j, key, pos);
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
@@ -381,7 +393,9 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
         atomicAdd(c, 1u);
       }
     }
-  }
+  };
+  for (int64_t r0 = chunk * chunk_rows; r0 < r1; r0 += 64 * kRows)
+    step(values + r0 * n_features, r1 - r0);
   if constexpr (!GATHER) {
     __syncthreads();
     for (int e = threadIdx.x; e < kBuckets * kTile; e += kThreads) slot[e] = s_count[e];
