@@ -19,7 +19,7 @@
 //
 // One thread per row over global memory, the form these replaced, took 7,140 us
 // for 1M x 28 rows through 100 trees of depth 8, 2,700 us for 60k x 784 through
-// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 620, 493 and 12 us.  The LDS reads
+// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 448, 410 and 12 us.  The LDS reads
 // (8 bytes of node from random banks, 4 of value, per visit) bound the first.
 #include "predict.hpp"
 
@@ -51,56 +51,54 @@ __device__ __forceinline__ float pred_expf(float x) {
 constexpr int kPredThreads = 1024;
 constexpr int kWalk = 4;  // trees a lane walks side by side
 
-__device__ __forceinline__ bool is_leaf(const PackedNode& n) { return (n.word & 0xffffu) == 0u; }
-__device__ __forceinline__ bool is_leaf(const PredNode& n) { return n.left < 0; }
-__device__ __forceinline__ int32_t feature_of(const PackedNode& n) { return int32_t(n.word >> 17); }
-__device__ __forceinline__ int32_t feature_of(const PredNode& n) { return n.feature; }
-__device__ __forceinline__ int32_t left_of(const PackedNode& n) { return int32_t(n.word & 0xffffu); }
-__device__ __forceinline__ int32_t left_of(const PredNode& n) { return n.left; }
-__device__ __forceinline__ bool missing_left(const PackedNode& n) { return n.word >> 16 & 1u; }
-__device__ __forceinline__ bool missing_left(const PredNode& n) { return n.flags & 1; }
-
-template <class Node>
-__device__ __forceinline__ Node leaf_node();
-template <>
-__device__ __forceinline__ PackedNode leaf_node<PackedNode>() { return {0.0f, 0u}; }
-template <>
-__device__ __forceinline__ PredNode leaf_node<PredNode>() { return {-1, 0, 0.0f, 0}; }
-
-// Leaf values of the first `n` (1 .. kWalk) trees at tree[], each walked from its
-// root; value(f): the row's value, NaN when missing.  A finished walk stays at
-// its leaf until the wavefront's last one ends.
-template <class Node, class Value>
-__device__ __forceinline__ void walk(const Node* const* tree, int n, Value value, float* leaf) {
-  Node node[kWalk];
+// Walks kWalk trees of packed nodes from the nodes at[w] (a leaf walks in place)
+// to their leaves, which at[w] then names.  nodes: what the indices count from,
+// per tree; value(f): the row's value.  NANS: missing values may occur.  Every
+// step is straight-line code; whether all lanes are at leaves is asked every
+// fourth.
+template <bool NANS, class Value>
+__device__ __forceinline__ void walk(const PackedNode* const* nodes, int32_t* at, int32_t depth,
+                                     Value value) {
+  PackedNode node[kWalk];
 #pragma unroll
-  for (int w = 0; w < kWalk; ++w) {
-    node[w] = leaf_node<Node>();
-    if (w < n) node[w] = tree[w][0];
-  }
-  for (;;) {
-    bool inner = false;
-#pragma unroll
-    for (int w = 0; w < kWalk; ++w) inner = inner || !is_leaf(node[w]);
-    if (!__any(inner)) break;
+  for (int w = 0; w < kWalk; ++w) node[w] = nodes[w][at[w]];
+  for (int32_t d = 1; d <= depth; ++d) {
     float x[kWalk];
 #pragma unroll
-    for (int w = 0; w < kWalk; ++w) x[w] = is_leaf(node[w]) ? 0.0f : value(feature_of(node[w]));
+    for (int w = 0; w < kWalk; ++w) x[w] = value(int32_t(node[w].word >> 17));
 #pragma unroll
     for (int w = 0; w < kWalk; ++w) {
-      if (is_leaf(node[w])) continue;
-      const bool left = x[w] != x[w] ? missing_left(node[w]) : x[w] < node[w].cond;
-      node[w] = tree[w][left_of(node[w]) + (left ? 0 : 1)];
+      uint32_t right = x[w] >= node[w].cond ? 1u : 0u;
+      if constexpr (NANS) right = x[w] != x[w] ? node[w].word >> 16 & 1u : right;
+      at[w] = int32_t((node[w].word & 0xffffu) + right);
+      node[w] = nodes[w][at[w]];
+    }
+    if ((d & 3) == 0) {
+      bool inner = false;
+#pragma unroll
+      for (int w = 0; w < kWalk; ++w) inner = inner || node[w].cond == node[w].cond;
+      if (!__any(inner)) break;
     }
   }
-#pragma unroll
-  for (int w = 0; w < kWalk; ++w) leaf[w] = node[w].cond;
+}
+
+// The same for one tree of general nodes; returns the leaf's value.
+template <class Value>
+__device__ __forceinline__ float walk(const PredNode* tree, Value value) {
+  PredNode node = tree[0];
+  while (node.left >= 0) {
+    const float x = value(node.feature);
+    const bool left = x != x ? node.flags & 1 : x < node.cond;
+    node = tree[node.left + (left ? 0 : 1)];
+  }
+  return node.cond;
 }
 
 // A row's output from its margins, which its thread hands over output by output.
 struct RowOutput {
   float* out;  // [groups] (argmax: [1]) of the row
   int32_t groups, transform;
+  bool store;  // false: a row past the last
   float best = -INFINITY, mx = -INFINITY;
   int32_t best_k = 0;
   __device__ __forceinline__ void margin(int32_t g, float m) {
@@ -109,14 +107,13 @@ struct RowOutput {
         best = m;
         best_k = g;
       }
-    } else if (transform == kPredSigmoid) {
-      out[g] = 1.0f / (1.0f + pred_expf(-m));
-    } else {
-      out[g] = m;
+    } else if (store) {
+      out[g] = transform == kPredSigmoid ? 1.0f / (1.0f + pred_expf(-m)) : m;
     }
     mx = fmaxf(mx, m);
   }
   __device__ __forceinline__ void finish() {
+    if (!store) return;
     if (transform == kPredArgmax) {
       out[0] = float(best_k);
     } else if (transform == kPredSoftmax) {
@@ -156,116 +153,158 @@ struct Margins {
   }
 };
 
-// Rows [r0, r0 + R) feature-major into LDS, x[f * R + row]; `missing` values as
-// NaN.  A thread copies pieces of one row: the lanes of a wavefront read
-// different rows' lines, which stay in L1 for the row's next pieces.
-__device__ __forceinline__ void stage_rows(float* x, const float* __restrict__ values, int64_t r0,
-                                           int R, int64_t n_rows, int32_t n_features,
-                                           int64_t row_stride, float missing) {
-  const int row = threadIdx.x & (R - 1);
-  const int64_t r = min(r0 + row, n_rows - 1);
-  const float* v = values + r * row_stride;
-  const int parts = blockDim.x / R;
-  for (int32_t f0 = int32_t(threadIdx.x) / R * 8; f0 < n_features; f0 += parts * 8) {
+// Whether `y` stands for a missing value; missing ones become NaN.
+__device__ __forceinline__ bool as_missing(float& y, float missing) {
+  if (y == missing) y = __builtin_nanf("");
+  return y != y;
+}
+
+// R = blockDim.x rows per workgroup, feature-major in LDS: x[f * R + row].
+template <int R>
+__global__ __launch_bounds__(R) void predict_rows_kernel(
+    const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
+    float missing, const PackedNode* __restrict__ nodes, const float* __restrict__ leaf_values,
+    const int32_t* __restrict__ tree_ptr, const int32_t* __restrict__ group_ptr, int32_t groups,
+    const int32_t* __restrict__ batch_ptr, int32_t batches, int32_t depth,
+    const float* __restrict__ base, int32_t transform, float* __restrict__ out) {
+  extern __shared__ PackedNode s_nodes[];  // [kPredBatchNodes], then the rows
+  float* x = reinterpret_cast<float*>(s_nodes + kPredBatchNodes);
+  const int64_t r = int64_t(blockIdx.x) * R + threadIdx.x;
+  const int64_t rc = min(r, n_rows - 1);  // rows past the last repeat it and store nothing
+  // A thread copies its own row: the wavefront's lines stay in L1 for the row's
+  // next values.
+  const float* v = values + rc * row_stride;
+  bool nan = false;
+  for (int32_t f0 = 0; f0 < n_features; f0 += 8) {
     float y[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) y[k] = v[min(f0 + k, n_features - 1)];
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (f0 + k < n_features) x[(f0 + k) * R + row] = y[k] == missing ? __builtin_nanf("") : y[k];
+    for (int k = 0; k < 8; ++k) {
+      nan = as_missing(y[k], missing) || nan;
+      if (f0 + k < n_features) x[(f0 + k) * R + int(threadIdx.x)] = y[k];
+    }
   }
-}
-
-// R = blockDim.x rows per workgroup.
-__global__ __launch_bounds__(kPredThreads) void predict_rows_kernel(
-    const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
-    float missing, const PackedNode* __restrict__ nodes, const int32_t* __restrict__ tree_ptr,
-    const int32_t* __restrict__ group_ptr, int32_t groups, const int32_t* __restrict__ batch_ptr,
-    int32_t batches, const float* __restrict__ base, int32_t transform, float* __restrict__ out) {
-  extern __shared__ PackedNode s_nodes[];  // [kPredBatchNodes], then the rows
-  float* x = reinterpret_cast<float*>(s_nodes + kPredBatchNodes);
-  const int R = blockDim.x;
-  const int64_t r0 = int64_t(blockIdx.x) * R, r = r0 + threadIdx.x;
-  stage_rows(x, values, r0, R, n_rows, n_features, row_stride, missing);
+  const bool nans = __syncthreads_or(nan);
   const int32_t outputs = transform == kPredArgmax ? 1 : groups;
-  // Rows past the last repeat it and store nothing.
-  Margins sum(group_ptr, base, {out + min(r, n_rows - 1) * outputs, groups, transform});
-  const bool live = r < n_rows;
+  Margins sum(group_ptr, base, {out + rc * outputs, groups, transform, r < n_rows});
+  auto value = [&](int32_t f) { return x[f * R + int(threadIdx.x)]; };
   for (int32_t b = 0; b < batches; ++b) {
     const int32_t t0 = batch_ptr[b], t1 = batch_ptr[b + 1];
     const int32_t n0 = tree_ptr[t0], n1 = tree_ptr[t1];
-    __syncthreads();  // the rows are staged, the last batch is walked
+    __syncthreads();  // the last batch is walked
     for (int32_t i = threadIdx.x; i < n1 - n0; i += R) s_nodes[i] = nodes[n0 + i];
     __syncthreads();
     for (int32_t t = t0; t < t1; t += kWalk) {
-      const int n = min(kWalk, t1 - t);
-      const PackedNode* tree[kWalk];
+      const PackedNode* from[kWalk];
+      int32_t at[kWalk];
       float leaf[kWalk];
 #pragma unroll
-      for (int w = 0; w < kWalk; ++w) tree[w] = s_nodes + (tree_ptr[min(t + w, t1 - 1)] - n0);
-      walk<PackedNode>(tree, n, [&](int32_t f) { return x[f * R + int(threadIdx.x)]; }, leaf);
-      if (live)
-        for (int w = 0; w < n; ++w) sum.add(leaf[w]);
+      for (int w = 0; w < kWalk; ++w) {
+        from[w] = s_nodes;
+        at[w] = tree_ptr[min(t + w, t1 - 1)] - n0;
+      }
+      if (nans) walk<true>(from, at, depth, value);
+      else walk<false>(from, at, depth, value);
+#pragma unroll
+      for (int w = 0; w < kWalk; ++w) leaf[w] = leaf_values[n0 + at[w]];
+#pragma unroll
+      for (int w = 0; w < kWalk; ++w)
+        if (t + w < t1) sum.add(leaf[w]);
     }
   }
-  if (live) sum.finish();
+  sum.finish();
 }
 
 // R rows (a power of two) x blockDim.x / R tree lanes per workgroup.  STAGE: the
-// rows in LDS.  leaves: LDS, two buffers of a round's leaf values.
+// rows in LDS, x[f * (R + 1) + row] (coalesced loads; the odd stride spreads
+// their stores over the banks).
 template <class Node, bool STAGE>
 __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
-    float missing, const Node* __restrict__ nodes, const int32_t* __restrict__ tree_ptr,
-    const int32_t* __restrict__ group_ptr, int32_t groups, int32_t trees,
+    float missing, const Node* __restrict__ nodes, const float* __restrict__ leaf_values,
+    const int32_t* __restrict__ tree_ptr, const int32_t* __restrict__ tree_base,
+    const int32_t* __restrict__ group_ptr, int32_t groups, int32_t trees, int32_t depth,
     const float* __restrict__ base, int32_t transform, int R, float* __restrict__ out) {
   extern __shared__ float s_leaf[];  // [2][kWalk * blockDim.x], then the rows
   float* x = s_leaf + 2 * kWalk * blockDim.x;
   const int row = threadIdx.x & (R - 1), lane = int(threadIdx.x) / R, lanes = blockDim.x / R;
   const int64_t r0 = int64_t(blockIdx.x) * R, r = r0 + row;
+  const int64_t rc = min(r, n_rows - 1);
   if constexpr (STAGE) {
-    stage_rows(x, values, r0, R, n_rows, n_features, row_stride, missing);
+    const int l64 = threadIdx.x & 63;
+    for (int q = int(threadIdx.x) >> 6; q < R; q += int(blockDim.x) >> 6) {
+      const float* v = values + min(r0 + q, n_rows - 1) * row_stride;
+      for (int32_t f0 = l64; f0 < n_features; f0 += 4 * 64) {
+        float y[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[k] = v[min(f0 + 64 * k, n_features - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          (void)as_missing(y[k], missing);
+          if (f0 + 64 * k < n_features) x[(f0 + 64 * k) * (R + 1) + q] = y[k];
+        }
+      }
+    }
     __syncthreads();
   }
   const int32_t outputs = transform == kPredArgmax ? 1 : groups;
-  const float* v = values + min(r, n_rows - 1) * row_stride;
+  const float* v = values + rc * row_stride;
   const bool adds = lane == 0 && r < n_rows;
-  Margins sum(group_ptr, base, {out + min(r, n_rows - 1) * outputs, groups, transform});
+  Margins sum(group_ptr, base, {out + rc * outputs, groups, transform, adds});
   auto value = [&](int32_t f) {
-    if constexpr (STAGE) return x[f * R + row];
-    const float y = v[f];
-    return y == missing ? __builtin_nanf("") : y;
+    if constexpr (STAGE) return x[f * (R + 1) + row];
+    float y = v[f];
+    (void)as_missing(y, missing);
+    return y;
   };
   const int32_t per_round = kWalk * lanes;
   int buffer = 0;
   for (int32_t t0 = 0; t0 < trees; t0 += per_round, buffer ^= 1) {
     float* leaves = s_leaf + buffer * kWalk * int(blockDim.x);
     // Tree t0 + w * lanes + lane: the lanes of one w walk adjacent trees.
-    const Node* tree[kWalk];
-    float leaf[kWalk];
-    int n = 0;
+    if constexpr (sizeof(Node) == sizeof(PackedNode)) {
+      const PackedNode* from[kWalk];
+      int32_t at[kWalk];
+      if (t0 + lane < trees) {
 #pragma unroll
-    for (int w = 0; w < kWalk; ++w) {
-      const int32_t t = t0 + w * lanes + lane;
-      if (t < trees) n = w + 1;
-      tree[w] = nodes + tree_ptr[min(t, trees - 1)];
+        for (int w = 0; w < kWalk; ++w) {
+          const int32_t t = min(t0 + w * lanes + lane, trees - 1);
+          from[w] = nodes + tree_base[t];
+          at[w] = tree_ptr[t] - tree_base[t];
+        }
+        walk<true>(from, at, depth, value);
+#pragma unroll
+        for (int w = 0; w < kWalk; ++w)
+          if (t0 + w * lanes + lane < trees)
+            leaves[(w * lanes + lane) * R + row] = leaf_values[(from[w] - nodes) + at[w]];
+      }
+    } else {
+      for (int w = 0; w < kWalk; ++w) {
+        const int32_t t = t0 + w * lanes + lane;
+        if (t < trees) leaves[(w * lanes + lane) * R + row] = walk(nodes + tree_ptr[t], value);
+      }
     }
-    if (n > 0) walk<Node>(tree, n, value, leaf);
-#pragma unroll
-    for (int w = 0; w < kWalk; ++w)
-      if (w < n) leaves[(w * lanes + lane) * R + row] = leaf[w];
     __syncthreads();  // the next round writes the other buffer
     if (adds) {
       const int32_t m = min(per_round, trees - t0);
-      for (int32_t i = 0; i < m; ++i) sum.add(leaves[i * R + row]);
+      for (int32_t i = 0; i < m; i += 8) {  // eight LDS reads in flight
+        float y[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) y[k] = leaves[min(i + k, m - 1) * R + row];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (i + k < m) sum.add(y[k]);
+      }
     }
   }
   if (adds) sum.finish();
 }
 
-// Raises a kernel's dynamic LDS limit to the CU's 160 KiB.
+// Dynamic LDS of a workgroup: the CU's 160 KiB less what the kernels declare.
+constexpr size_t kPredLds = (size_t(160) << 10) - 1024;
 void allow_lds(const void* kernel) {
-  DP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10));
+  DP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(kPredLds)));
 }
 
 }  // namespace
@@ -275,37 +314,52 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
   const int32_t groups = int32_t(base.size());
   std::vector<std::vector<const ForestTree*>> by_group(static_cast<size_t>(groups));
   size_t total = 0;
-  bool packed = n_features <= (1 << 15);
+  bool packed = n_features <= (1 << 15), batched = true;
+  out.depth = 0;
   for (const ForestTree& t : trees) {
     by_group[size_t(t.group)].push_back(&t);
     total += t.nodes.size();
     packed = packed && t.nodes.size() <= (size_t(1) << 16);
+    batched = batched && t.nodes.size() <= size_t(kPredBatchNodes);
+    std::vector<int32_t> level(t.nodes.size(), 0);  // children follow their parents
+    for (size_t i = 0; i < t.nodes.size(); ++i) {
+      const PredNode& n = t.nodes[i];
+      if (n.left < 0) continue;
+      packed = packed && !std::isnan(n.cond);
+      level[size_t(n.left)] = level[size_t(n.left) + 1] = level[i] + 1;
+      out.depth = std::max(out.depth, level[i] + 1);
+    }
   }
   need(total < size_t(INT32_MAX), "forest has too many nodes");
-  std::vector<int32_t> tree_ptr{0}, group_ptr{0}, batch_ptr{0};
-  std::vector<uint8_t> bytes(total * (packed ? sizeof(PackedNode) : sizeof(PredNode)));
-  bool batched = packed;
-  size_t n = 0;
+  std::vector<int32_t> tree_ptr{0}, tree_base, group_ptr{0}, batch_ptr{0};
+  std::vector<PackedNode> small;
+  std::vector<PredNode> general;
+  std::vector<float> leaves;
+  int32_t n = 0, batch = 0;  // nodes so far; the first node of the batch
   for (const auto& group : by_group) {
     for (const ForestTree* t : group) {
-      for (const PredNode& nd : t->nodes) {
-        if (packed) {
-          PackedNode p;
-          p.cond = nd.cond;
-          p.word = nd.left < 0 ? 0u
-                               : uint32_t(nd.left) | uint32_t(nd.flags & 1) << 16 |
-                                     uint32_t(nd.feature) << 17;
-          std::memcpy(bytes.data() + n * sizeof p, &p, sizeof p);
-        } else {
-          std::memcpy(bytes.data() + n * sizeof nd, &nd, sizeof nd);
-        }
-        ++n;
+      const int32_t size = int32_t(t->nodes.size());
+      // Packed indices count from the batch (a large tree: from itself).
+      if (n > batch && n + size - batch > kPredBatchNodes) {
+        batch = n;
+        batch_ptr.push_back(int32_t(tree_ptr.size()) - 1);
       }
-      // Does the tree start a new batch?
-      const int32_t first = tree_ptr[size_t(batch_ptr.back())];
-      if (int32_t(n) - first > kPredBatchNodes) batch_ptr.push_back(int32_t(tree_ptr.size()) - 1);
-      batched = batched && t->nodes.size() <= size_t(kPredBatchNodes);
-      tree_ptr.push_back(int32_t(n));
+      for (int32_t i = 0; i < size; ++i) {
+        const PredNode& nd = t->nodes[size_t(i)];
+        if (!packed) {
+          general.push_back(nd);
+          continue;
+        }
+        const uint32_t at = uint32_t(n - batch);
+        small.push_back(nd.left < 0 ? PackedNode{std::nanf(""), at + uint32_t(i)}
+                                    : PackedNode{nd.cond, (at + uint32_t(nd.left)) |
+                                                              uint32_t(nd.flags & 1 ? 0 : 1) << 16 |
+                                                              uint32_t(nd.feature) << 17});
+        leaves.push_back(nd.left < 0 ? nd.cond : 0.0f);
+      }
+      tree_base.push_back(batch);
+      n += size;
+      tree_ptr.push_back(n);
     }
     group_ptr.push_back(int32_t(tree_ptr.size()) - 1);
   }
@@ -313,14 +367,17 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
   out.groups = groups;
   out.packed = packed;
   if (batch_ptr.back() != out.trees) batch_ptr.push_back(out.trees);
-  out.batches = batched ? int32_t(batch_ptr.size()) - 1 : 0;
+  out.batches = packed && batched ? int32_t(batch_ptr.size()) - 1 : 0;
   auto put = [](auto& dst, const auto& src) {
-    dst.resize(std::max<size_t>(src.size(), 1));
-    if (!src.empty())
-      DP_HIP(hipMemcpy(dst.p, src.data(), src.size() * sizeof(src[0]), hipMemcpyHostToDevice));
+    const size_t bytes = src.size() * sizeof(src[0]);
+    dst.resize(std::max<size_t>(bytes, 16) / sizeof(*dst.p));
+    if (bytes) DP_HIP(hipMemcpy(dst.p, src.data(), bytes, hipMemcpyHostToDevice));
   };
-  put(out.nodes, bytes);
+  if (packed) put(out.nodes, small);
+  else put(out.nodes, general);
+  put(out.leaf_values, leaves);
   put(out.tree_ptr, tree_ptr);
+  put(out.tree_base, tree_base);
   put(out.group_ptr, group_ptr);
   put(out.batch_ptr, batch_ptr);
   put(out.base, base);
@@ -333,7 +390,6 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   int dev = 0, cus = 0;
   DP_HIP(hipGetDevice(&dev));
   DP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  constexpr size_t kLds = size_t(160) << 10;
   const auto* packed = reinterpret_cast<const PackedNode*>(forest.nodes.p);
   // A row per thread when the rows fill the chip with workgroups of at least 256
   // and their values fit LDS beside a batch of nodes.
@@ -341,13 +397,17 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   auto rows_lds = [&](int rows) {
     return sizeof(PackedNode) * kPredBatchNodes + sizeof(float) * size_t(rows) * n_features;
   };
-  while (R > 256 && (rows_lds(R) > kLds || n_rows < int64_t(R) * cus)) R /= 2;
-  if (forest.batches > 0 && n_rows >= int64_t(R) * cus && rows_lds(R) <= kLds) {
-    allow_lds(reinterpret_cast<const void*>(predict_rows_kernel));
-    hipLaunchKernelGGL(predict_rows_kernel, dim3(unsigned((n_rows + R - 1) / R)), dim3(R),
-                       rows_lds(R), s, values, n_rows, n_features, row_stride, missing, packed,
-                       forest.tree_ptr.p, forest.group_ptr.p, forest.groups, forest.batch_ptr.p,
-                       forest.batches, forest.base.p, transform, out);
+  while (R > 256 && (rows_lds(R) > kPredLds || n_rows < int64_t(R) * cus)) R /= 2;
+  if (forest.batches > 0 && n_rows >= int64_t(R) * cus && rows_lds(R) <= kPredLds) {
+    const auto kernel = R == 1024  ? predict_rows_kernel<1024>
+                        : R == 512 ? predict_rows_kernel<512>
+                                   : predict_rows_kernel<256>;
+    allow_lds(reinterpret_cast<const void*>(kernel));
+    hipLaunchKernelGGL(kernel, dim3(unsigned((n_rows + R - 1) / R)), dim3(R), rows_lds(R), s,
+                       values, n_rows, n_features, row_stride, missing, packed,
+                       forest.leaf_values.p, forest.tree_ptr.p, forest.group_ptr.p, forest.groups,
+                       forest.batch_ptr.p, forest.batches, forest.depth, forest.base.p, transform,
+                       out);
     DP_HIP(hipGetLastError());
     return;
   }
@@ -365,17 +425,18 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   // row holds.
   const size_t leaf_lds = sizeof(float) * 2 * kWalk * size_t(threads);
   bool stage = int64_t(forest.trees) * 128 >= n_features;
-  while (stage && leaf_lds + sizeof(float) * size_t(rows) * n_features > kLds) {
+  while (stage && leaf_lds + sizeof(float) * size_t(rows + 1) * n_features > kPredLds) {
     if (rows > 8) rows /= 2;
     else stage = false;
   }
-  const size_t lds = leaf_lds + (stage ? sizeof(float) * size_t(rows) * n_features : 0);
+  const size_t lds = leaf_lds + (stage ? sizeof(float) * size_t(rows + 1) * n_features : 0);
   const dim3 grid(unsigned((n_rows + rows - 1) / rows));
   auto run = [&](auto kernel, const auto* nodes) {
     allow_lds(reinterpret_cast<const void*>(kernel));
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, values, n_rows, n_features,
-                       row_stride, missing, nodes, forest.tree_ptr.p, forest.group_ptr.p,
-                       forest.groups, forest.trees, forest.base.p, transform, rows, out);
+                       row_stride, missing, nodes, forest.leaf_values.p, forest.tree_ptr.p,
+                       forest.tree_base.p, forest.group_ptr.p, forest.groups, forest.trees,
+                       forest.depth, forest.base.p, transform, rows, out);
     DP_HIP(hipGetLastError());
   };
   const auto* general = reinterpret_cast<const PredNode*>(forest.nodes.p);

@@ -25,9 +25,11 @@ struct PredNode {
   int32_t flags;    // bit 0: missing goes left
 };
 
-// The same in 8 bytes, for trees of at most 65,536 nodes over at most 32,768
-// features: bits 0-15 of `word` the left child's index (0: a leaf), bit 16
-// missing goes left, bits 17-31 the feature.
+// The same in 8 bytes: bits 0-15 of `word` the left child's index in the node's
+// batch of trees, bit 16 missing goes right, bits 17-31 the feature.  A row goes
+// right when x >= cond, so a leaf (cond NaN, its own index as left child) keeps
+// every row, missing or not, and its value is in Forest::leaf_values.  Forests of
+// at most 32,768 features, 65,536 nodes a tree and no NaN threshold take it.
 struct PackedNode {
   float cond;
   uint32_t word;
@@ -37,7 +39,9 @@ struct PackedNode {
 // within each.
 struct Forest {
   DeviceBuffer<uint8_t> nodes;       // PackedNode or PredNode
+  DeviceBuffer<float> leaf_values;   // packed: [nodes] a leaf's value
   DeviceBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
+  DeviceBuffer<int32_t> tree_base;   // [trees] the node that the tree's indices count from
   DeviceBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
   DeviceBuffer<int32_t> batch_ptr;   // [batches + 1] first tree of each batch of
                                      // trees whose nodes fit kPredBatchNodes
@@ -45,6 +49,7 @@ struct Forest {
   bool packed = false;
   int32_t trees = 0, groups = 1;
   int32_t batches = 0;  // 0: some tree alone exceeds kPredBatchNodes (or is not packed)
+  int32_t depth = 0;    // of the deepest tree
 };
 
 constexpr int32_t kPredBatchNodes = 4096;
