@@ -19,8 +19,11 @@
 //
 // One thread per row over global memory, the form these replaced, took 7,140 us
 // for 1M x 28 rows through 100 trees of depth 8, 2,700 us for 60k x 784 through
-// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 448, 410 and 12 us.  The LDS reads
-// (8 bytes of node from random banks, 4 of value, per visit) bound the first.
+// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 360, 410 and 12 us.
+// The first is bound by its vector instructions (11 per visit) and LDS reads (8
+// bytes of node from random banks, 4 of value), the second by the node loads of
+// its lanes, which rarely share a line.  Staging the second's nodes in LDS too
+// took 548 us: a batch has too few trees for a wide-row workgroup's lanes.
 #include "predict.hpp"
 
 #include <algorithm>
@@ -52,26 +55,23 @@ constexpr int kPredThreads = 1024;
 constexpr int kWalk = 4;  // trees a lane walks side by side
 
 // Walks kWalk trees of packed nodes from the nodes at[w] (a leaf walks in place)
-// to their leaves, which at[w] then names.  nodes: what the indices count from,
-// per tree; value(f): the row's value.  NANS: missing values may occur.  Every
-// step is straight-line code; whether all lanes are at leaves is asked every
-// fourth.
-template <bool NANS, class Value>
-__device__ __forceinline__ void walk(const PackedNode* const* nodes, int32_t* at, int32_t depth,
-                                     Value value) {
+// to their leaves, which at[w] then names.  fetch(w, i): node i of tree w;
+// value(word): the row's value of the feature in bits 17-30.  Every step is
+// straight-line code; whether all lanes are at leaves is asked every fourth.
+template <class Fetch, class Value>
+__device__ __forceinline__ void walk(uint32_t* at, int32_t depth, Fetch fetch, Value value) {
   PackedNode node[kWalk];
 #pragma unroll
-  for (int w = 0; w < kWalk; ++w) node[w] = nodes[w][at[w]];
+  for (int w = 0; w < kWalk; ++w) node[w] = fetch(w, at[w]);
   for (int32_t d = 1; d <= depth; ++d) {
     float x[kWalk];
 #pragma unroll
-    for (int w = 0; w < kWalk; ++w) x[w] = value(int32_t(node[w].word >> 17));
+    for (int w = 0; w < kWalk; ++w) x[w] = value(node[w].word);
 #pragma unroll
     for (int w = 0; w < kWalk; ++w) {
-      uint32_t right = x[w] >= node[w].cond ? 1u : 0u;
-      if constexpr (NANS) right = x[w] != x[w] ? node[w].word >> 16 & 1u : right;
-      at[w] = int32_t((node[w].word & 0xffffu) + right);
-      node[w] = nodes[w][at[w]];
+      const float y = __uint_as_float(__float_as_uint(x[w]) ^ (node[w].word & 0x80000000u));
+      at[w] = (node[w].word & 0xffffu) + (y >= node[w].cond ? 1u : 0u);
+      node[w] = fetch(w, at[w]);
     }
     if ((d & 3) == 0) {
       bool inner = false;
@@ -153,10 +153,9 @@ struct Margins {
   }
 };
 
-// Whether `y` stands for a missing value; missing ones become NaN.
-__device__ __forceinline__ bool as_missing(float& y, float missing) {
-  if (y == missing) y = __builtin_nanf("");
-  return y != y;
+// y, or NaN where y stands for a missing value.
+__device__ __forceinline__ float or_nan(float y, float missing) {
+  return y == missing ? __builtin_nanf("") : y;
 }
 
 // R = blockDim.x rows per workgroup, feature-major in LDS: x[f * R + row].
@@ -164,8 +163,9 @@ template <int R>
 __global__ __launch_bounds__(R) void predict_rows_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
     float missing, const PackedNode* __restrict__ nodes, const float* __restrict__ leaf_values,
-    const int32_t* __restrict__ tree_ptr, const int32_t* __restrict__ group_ptr, int32_t groups,
-    const int32_t* __restrict__ batch_ptr, int32_t batches, int32_t depth,
+    const int32_t* __restrict__ batch_node, const int32_t* __restrict__ batch_tree,
+    const int32_t* __restrict__ quad_ptr, const int4* __restrict__ quads, int32_t batches,
+    const int32_t* __restrict__ group_ptr, int32_t groups, int32_t depth,
     const float* __restrict__ base, int32_t transform, float* __restrict__ out) {
   extern __shared__ PackedNode s_nodes[];  // [kPredBatchNodes], then the rows
   float* x = reinterpret_cast<float*>(s_nodes + kPredBatchNodes);
@@ -174,51 +174,50 @@ __global__ __launch_bounds__(R) void predict_rows_kernel(
   // A thread copies its own row: the wavefront's lines stay in L1 for the row's
   // next values.
   const float* v = values + rc * row_stride;
-  bool nan = false;
   for (int32_t f0 = 0; f0 < n_features; f0 += 8) {
     float y[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) y[k] = v[min(f0 + k, n_features - 1)];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      nan = as_missing(y[k], missing) || nan;
-      if (f0 + k < n_features) x[(f0 + k) * R + int(threadIdx.x)] = y[k];
+      if (f0 + k < n_features) x[(f0 + k) * R + int(threadIdx.x)] = or_nan(y[k], missing);
     }
   }
-  const bool nans = __syncthreads_or(nan);
   const int32_t outputs = transform == kPredArgmax ? 1 : groups;
   Margins sum(group_ptr, base, {out + rc * outputs, groups, transform, r < n_rows});
-  auto value = [&](int32_t f) { return x[f * R + int(threadIdx.x)]; };
+  constexpr int kShift = 17 - __builtin_ctz(R * unsigned(sizeof(float)));
+  auto value = [&](uint32_t word) {  // x[feature * R + thread]
+    const uint32_t at = (word >> kShift & (0x3fffu << (17 - kShift))) | threadIdx.x * 4u;
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(x) + at);
+  };
+  auto fetch = [&](int, uint32_t i) { return s_nodes[i]; };
+  int4 quad = batches > 0 ? quads[0] : make_int4(0, 0, 0, 0);
   for (int32_t b = 0; b < batches; ++b) {
-    const int32_t t0 = batch_ptr[b], t1 = batch_ptr[b + 1];
-    const int32_t n0 = tree_ptr[t0], n1 = tree_ptr[t1];
+    const int32_t n0 = batch_node[b], n1 = batch_node[b + 1];
+    const int32_t q0 = quad_ptr[b], q1 = quad_ptr[b + 1];
+    int32_t trees = batch_tree[b + 1] - batch_tree[b];
     __syncthreads();  // the last batch is walked
     for (int32_t i = threadIdx.x; i < n1 - n0; i += R) s_nodes[i] = nodes[n0 + i];
     __syncthreads();
-    for (int32_t t = t0; t < t1; t += kWalk) {
-      const PackedNode* from[kWalk];
-      int32_t at[kWalk];
+    for (int32_t q = q0; q < q1; ++q, trees -= kWalk) {
+      uint32_t at[kWalk] = {uint32_t(quad.x), uint32_t(quad.y), uint32_t(quad.z),
+                            uint32_t(quad.w)};
+      quad = quads[q + 1];  // ahead of the walk (one entry of padding ends the list)
+      walk(at, depth, fetch, value);
       float leaf[kWalk];
 #pragma unroll
-      for (int w = 0; w < kWalk; ++w) {
-        from[w] = s_nodes;
-        at[w] = tree_ptr[min(t + w, t1 - 1)] - n0;
-      }
-      if (nans) walk<true>(from, at, depth, value);
-      else walk<false>(from, at, depth, value);
-#pragma unroll
-      for (int w = 0; w < kWalk; ++w) leaf[w] = leaf_values[n0 + at[w]];
+      for (int w = 0; w < kWalk; ++w) leaf[w] = leaf_values[n0 + int32_t(at[w])];
 #pragma unroll
       for (int w = 0; w < kWalk; ++w)
-        if (t + w < t1) sum.add(leaf[w]);
+        if (w < trees) sum.add(leaf[w]);
     }
   }
   sum.finish();
 }
 
 // R rows (a power of two) x blockDim.x / R tree lanes per workgroup.  STAGE: the
-// rows in LDS, x[f * (R + 1) + row] (coalesced loads; the odd stride spreads
-// their stores over the banks).
+// rows in LDS, x[row * (n_features | 1) + f] (coalesced loads; the odd stride
+// spreads the rows over the banks).
 template <class Node, bool STAGE>
 __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
@@ -231,19 +230,20 @@ __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
   const int row = threadIdx.x & (R - 1), lane = int(threadIdx.x) / R, lanes = blockDim.x / R;
   const int64_t r0 = int64_t(blockIdx.x) * R, r = r0 + row;
   const int64_t rc = min(r, n_rows - 1);
+  const int stride = n_features | 1;
   if constexpr (STAGE) {
+    // A wavefront per row, kPieces runs of 64 values in flight.
+    constexpr int kPieces = 8;
     const int l64 = threadIdx.x & 63;
     for (int q = int(threadIdx.x) >> 6; q < R; q += int(blockDim.x) >> 6) {
       const float* v = values + min(r0 + q, n_rows - 1) * row_stride;
-      for (int32_t f0 = l64; f0 < n_features; f0 += 4 * 64) {
-        float y[4];
+      for (int32_t f0 = l64; f0 < n_features; f0 += kPieces * 64) {
+        float y[kPieces];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) y[k] = v[min(f0 + 64 * k, n_features - 1)];
+        for (int k = 0; k < kPieces; ++k) y[k] = v[min(f0 + 64 * k, n_features - 1)];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          (void)as_missing(y[k], missing);
-          if (f0 + 64 * k < n_features) x[(f0 + 64 * k) * (R + 1) + q] = y[k];
-        }
+        for (int k = 0; k < kPieces; ++k)
+          if (f0 + 64 * k < n_features) x[q * stride + f0 + 64 * k] = or_nan(y[k], missing);
       }
     }
     __syncthreads();
@@ -252,32 +252,34 @@ __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
   const float* v = values + rc * row_stride;
   const bool adds = lane == 0 && r < n_rows;
   Margins sum(group_ptr, base, {out + rc * outputs, groups, transform, adds});
-  auto value = [&](int32_t f) {
-    if constexpr (STAGE) return x[f * (R + 1) + row];
-    float y = v[f];
-    (void)as_missing(y, missing);
-    return y;
-  };
+  const float* xr = x + row * stride;
+  auto value = [&](int32_t f) { return STAGE ? xr[f] : or_nan(v[f], missing); };
   const int32_t per_round = kWalk * lanes;
   int buffer = 0;
   for (int32_t t0 = 0; t0 < trees; t0 += per_round, buffer ^= 1) {
     float* leaves = s_leaf + buffer * kWalk * int(blockDim.x);
     // Tree t0 + w * lanes + lane: the lanes of one w walk adjacent trees.
     if constexpr (sizeof(Node) == sizeof(PackedNode)) {
-      const PackedNode* from[kWalk];
-      int32_t at[kWalk];
+      uint32_t origin[kWalk], at[kWalk];  // origin: the node a tree's indices count from
       if (t0 + lane < trees) {
 #pragma unroll
         for (int w = 0; w < kWalk; ++w) {
           const int32_t t = min(t0 + w * lanes + lane, trees - 1);
-          from[w] = nodes + tree_base[t];
-          at[w] = tree_ptr[t] - tree_base[t];
+          origin[w] = uint32_t(tree_base[t]);
+          at[w] = uint32_t(tree_ptr[t]) - origin[w];
         }
-        walk<true>(from, at, depth, value);
+        // 32-bit byte offsets from the uniform base (a packed forest is below 4 GiB)
+        walk(
+            at, depth,
+            [&](int w, uint32_t i) {
+              const char* p = reinterpret_cast<const char*>(nodes) + (i + origin[w]) * 8u;
+              return *reinterpret_cast<const PackedNode*>(p);
+            },
+            [&](uint32_t word) { return value(int32_t(word >> 17 & 0x3fffu)); });
 #pragma unroll
         for (int w = 0; w < kWalk; ++w)
           if (t0 + w * lanes + lane < trees)
-            leaves[(w * lanes + lane) * R + row] = leaf_values[(from[w] - nodes) + at[w]];
+            leaves[(w * lanes + lane) * R + row] = leaf_values[origin[w] + at[w]];
       }
     } else {
       for (int w = 0; w < kWalk; ++w) {
@@ -314,7 +316,7 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
   const int32_t groups = int32_t(base.size());
   std::vector<std::vector<const ForestTree*>> by_group(static_cast<size_t>(groups));
   size_t total = 0;
-  bool packed = n_features <= (1 << 15), batched = true;
+  bool packed = n_features <= (1 << 14), batched = true;
   out.depth = 0;
   for (const ForestTree& t : trees) {
     by_group[size_t(t.group)].push_back(&t);
@@ -325,13 +327,14 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
     for (size_t i = 0; i < t.nodes.size(); ++i) {
       const PredNode& n = t.nodes[i];
       if (n.left < 0) continue;
-      packed = packed && !std::isnan(n.cond);
+      packed = packed && !std::isnan(n.cond) && (n.flags & 1 || n.cond != -INFINITY);
       level[size_t(n.left)] = level[size_t(n.left) + 1] = level[i] + 1;
       out.depth = std::max(out.depth, level[i] + 1);
     }
   }
   need(total < size_t(INT32_MAX), "forest has too many nodes");
-  std::vector<int32_t> tree_ptr{0}, tree_base, group_ptr{0}, batch_ptr{0};
+  packed = packed && total < (size_t(1) << 29);
+  std::vector<int32_t> tree_ptr{0}, tree_base, group_ptr{0}, batch_tree{0};
   std::vector<PackedNode> small;
   std::vector<PredNode> general;
   std::vector<float> leaves;
@@ -342,20 +345,32 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
       // Packed indices count from the batch (a large tree: from itself).
       if (n > batch && n + size - batch > kPredBatchNodes) {
         batch = n;
-        batch_ptr.push_back(int32_t(tree_ptr.size()) - 1);
+        batch_tree.push_back(int32_t(tree_ptr.size()) - 1);
       }
-      for (int32_t i = 0; i < size; ++i) {
-        const PredNode& nd = t->nodes[size_t(i)];
-        if (!packed) {
-          general.push_back(nd);
-          continue;
+      if (!packed) general.insert(general.end(), t->nodes.begin(), t->nodes.end());
+      if (packed) {
+        // Node i's place: children that missing values enter on the right swap.
+        std::vector<int32_t> place(static_cast<size_t>(size), 0);
+        for (const PredNode& nd : t->nodes) {
+          if (nd.left < 0) continue;
+          const int32_t second = nd.flags & 1 ? 1 : 0;  // the right child's place in the pair
+          place[size_t(nd.left)] = nd.left + 1 - second;
+          place[size_t(nd.left) + 1] = nd.left + second;
         }
+        small.resize(size_t(n) + size_t(size));
+        leaves.resize(small.size());
         const uint32_t at = uint32_t(n - batch);
-        small.push_back(nd.left < 0 ? PackedNode{std::nanf(""), at + uint32_t(i)}
-                                    : PackedNode{nd.cond, (at + uint32_t(nd.left)) |
-                                                              uint32_t(nd.flags & 1 ? 0 : 1) << 16 |
-                                                              uint32_t(nd.feature) << 17});
-        leaves.push_back(nd.left < 0 ? nd.cond : 0.0f);
+        for (int32_t i = 0; i < size; ++i) {
+          const PredNode& nd = t->nodes[size_t(i)];
+          PackedNode& out_node = small[size_t(n + place[size_t(i)])];
+          leaves[size_t(n + place[size_t(i)])] = nd.left < 0 ? nd.cond : 0.0f;
+          if (nd.left < 0)
+            out_node = {std::nanf(""), at + uint32_t(place[size_t(i)])};
+          else
+            out_node = {nd.flags & 1 ? nd.cond : std::nextafterf(-nd.cond, INFINITY),
+                        (at + uint32_t(nd.left)) | uint32_t(nd.feature) << 17 |
+                            (nd.flags & 1 ? 0u : 0x80000000u)};
+        }
       }
       tree_base.push_back(batch);
       n += size;
@@ -366,8 +381,17 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
   out.trees = int32_t(tree_ptr.size()) - 1;
   out.groups = groups;
   out.packed = packed;
-  if (batch_ptr.back() != out.trees) batch_ptr.push_back(out.trees);
-  out.batches = packed && batched ? int32_t(batch_ptr.size()) - 1 : 0;
+  if (batch_tree.back() != out.trees) batch_tree.push_back(out.trees);
+  out.batches = packed && batched ? int32_t(batch_tree.size()) - 1 : 0;
+  std::vector<int32_t> batch_node{0}, quad_ptr{0}, quads;
+  for (int32_t b = 0; b < out.batches; ++b) {
+    const int32_t t0 = batch_tree[size_t(b)], t1 = batch_tree[size_t(b) + 1];
+    for (int32_t t = t0; t < t1 || (t - t0) % 4 != 0; ++t)
+      quads.push_back(tree_ptr[size_t(std::min(t, t1 - 1))] - tree_ptr[size_t(t0)]);
+    quad_ptr.push_back(int32_t(quads.size()) / 4);
+    batch_node.push_back(tree_ptr[size_t(t1)]);
+  }
+  quads.insert(quads.end(), 4, 0);
   auto put = [](auto& dst, const auto& src) {
     const size_t bytes = src.size() * sizeof(src[0]);
     dst.resize(std::max<size_t>(bytes, 16) / sizeof(*dst.p));
@@ -379,7 +403,10 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
   put(out.tree_ptr, tree_ptr);
   put(out.tree_base, tree_base);
   put(out.group_ptr, group_ptr);
-  put(out.batch_ptr, batch_ptr);
+  put(out.batch_node, batch_node);
+  put(out.batch_tree, batch_tree);
+  put(out.quad_ptr, quad_ptr);
+  put(out.quads, quads);
   put(out.base, base);
 }
 
@@ -405,31 +432,44 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
     allow_lds(reinterpret_cast<const void*>(kernel));
     hipLaunchKernelGGL(kernel, dim3(unsigned((n_rows + R - 1) / R)), dim3(R), rows_lds(R), s,
                        values, n_rows, n_features, row_stride, missing, packed,
-                       forest.leaf_values.p, forest.tree_ptr.p, forest.group_ptr.p, forest.groups,
-                       forest.batch_ptr.p, forest.batches, forest.depth, forest.base.p, transform,
-                       out);
+                       forest.leaf_values.p, forest.batch_node.p, forest.batch_tree.p,
+                       forest.quad_ptr.p, reinterpret_cast<const int4*>(forest.quads.p),
+                       forest.batches, forest.group_ptr.p, forest.groups, forest.depth,
+                       forest.base.p, transform, out);
     DP_HIP(hipGetLastError());
     return;
   }
-  // Rows per workgroup: a workgroup per CU first, then as many rows as leave a
-  // tree to each of the other threads.
+  // Rows per workgroup: a workgroup per CU first, then as many rows as leave
+  // kWalk trees to each of the other threads, then up to 32.
   int rows = 1;
   while (rows < 256 && n_rows > int64_t(rows) * cus * 2 &&
-         int64_t(forest.trees) * rows < int64_t(kPredThreads) * kWalk)
+         (rows < 32 || int64_t(forest.trees) * rows < int64_t(kPredThreads) * kWalk))
     rows *= 2;
-  while (rows < 32 && n_rows > int64_t(rows) * cus * 2) rows *= 2;
-  int threads = 64;
-  while (threads < kPredThreads && threads < int64_t(forest.trees) * rows) threads *= 2;
-  threads = std::max(threads, rows);
   // Values in LDS where they fit, unless the few trees read fewer of them than a
-  // row holds.
-  const size_t leaf_lds = sizeof(float) * 2 * kWalk * size_t(threads);
+  // row holds: half a CU's LDS and threads, so that one workgroup stages its rows
+  // while another walks; all of it for rows too wide for that.
   bool stage = int64_t(forest.trees) * 128 >= n_features;
-  while (stage && leaf_lds + sizeof(float) * size_t(rows + 1) * n_features > kPredLds) {
-    if (rows > 8) rows /= 2;
-    else stage = false;
+  auto lds_of = [&](int rows, int threads) {
+    return sizeof(float) * (2 * kWalk * size_t(threads) + size_t(rows) * size_t(n_features | 1));
+  };
+  int most = kPredThreads;
+  if (stage) {
+    int half = rows, full = rows;
+    while (half > 1 && lds_of(half, kPredThreads / 2) > kPredLds / 2) half /= 2;
+    while (full > 1 && lds_of(full, kPredThreads) > kPredLds) full /= 2;
+    stage = lds_of(full, kPredThreads) <= kPredLds;
+    if (half >= std::min(rows, 32) && lds_of(half, kPredThreads / 2) <= kPredLds / 2) {
+      rows = half;
+      most = kPredThreads / 2;
+    } else if (stage) {
+      rows = full;
+    }
   }
-  const size_t lds = leaf_lds + (stage ? sizeof(float) * size_t(rows + 1) * n_features : 0);
+  int threads = 64;
+  while (threads < most && threads < int64_t(forest.trees) * rows) threads *= 2;
+  threads = std::max(threads, rows);
+  const size_t leaf_lds = sizeof(float) * 2 * kWalk * size_t(threads);
+  const size_t lds = leaf_lds + (stage ? sizeof(float) * size_t(rows) * size_t(n_features | 1) : 0);
   const dim3 grid(unsigned((n_rows + rows - 1) / rows));
   auto run = [&](auto kernel, const auto* nodes) {
     allow_lds(reinterpret_cast<const void*>(kernel));

@@ -25,12 +25,18 @@ struct PredNode {
   int32_t flags;    // bit 0: missing goes left
 };
 
-// The same in 8 bytes: bits 0-15 of `word` the left child's index in the node's
-// batch of trees, bit 16 missing goes right, bits 17-31 the feature.  A row goes
-// right when x >= cond, so a leaf (cond NaN, its own index as left child) keeps
-// every row, missing or not, and its value is in Forest::leaf_values.  Forests of
-// at most 32,768 features, 65,536 nodes a tree and no NaN threshold take it.
-struct PackedNode {
+// The same in 8 bytes: bits 0-15 of `word` the first child's index in the node's
+// batch of trees, bits 17-30 the feature, bit 31 a sign.  A row goes to the second
+// child when (sign ? -x : x) >= cond, to the first otherwise, so also when x is
+// missing (NaN): the first child is the one missing values take.
+//   missing left    children (left, right), cond the threshold t: x >= t is right
+//   missing right   children (right, left), sign, cond the float above -t:
+//                   -x >= cond exactly when x < t
+//   leaf            its own index, cond NaN: every row stays; its value is in
+//                   Forest::leaf_values
+// Forests of at most 16,384 features, 65,536 nodes a tree and no threshold that
+// would make a NaN take it.
+struct alignas(8) PackedNode {
   float cond;
   uint32_t word;
 };
@@ -43,8 +49,13 @@ struct Forest {
   DeviceBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
   DeviceBuffer<int32_t> tree_base;   // [trees] the node that the tree's indices count from
   DeviceBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
-  DeviceBuffer<int32_t> batch_ptr;   // [batches + 1] first tree of each batch of
-                                     // trees whose nodes fit kPredBatchNodes
+  // Batches of trees whose nodes fit kPredBatchNodes: their first nodes, and per
+  // batch the trees' first nodes, counted from the batch, in groups of four (the
+  // last group repeats the last tree), quad_ptr[b] .. quad_ptr[b + 1] of them.
+  DeviceBuffer<int32_t> batch_node;  // [batches + 1]
+  DeviceBuffer<int32_t> quad_ptr;    // [batches + 1]
+  DeviceBuffer<int32_t> quads;       // [groups of four][4]
+  DeviceBuffer<int32_t> batch_tree;  // [batches + 1] first tree
   DeviceBuffer<float> base;          // [groups] margin before the first tree
   bool packed = false;
   int32_t trees = 0, groups = 1;

@@ -1,0 +1,99 @@
+"""Prediction of random forests against a plain numpy walk, bit for bit, where the kernels
+change course: a row per thread or a tree per thread, nodes and rows in LDS or not, packed
+or general nodes, large trees, several outputs, missing values, infinities, row strides."""
+import json
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _forest(rng, trees, depth, features, full):
+    """Node arrays (left, feature, cond, default) per tree; `full` of the inner nodes split."""
+    out = []
+    for _ in range(trees):
+        left, level, i = [-1], [0], 0
+        while i < len(left):
+            if level[i] < depth and rng.random() < full:
+                left[i] = len(left)
+                left += [-1, -1]
+                level += [level[i] + 1] * 2
+            i += 1
+        n = len(left)
+        leaf = np.array(left) < 0
+        cond = np.where(leaf, rng.normal(size=n) * 0.1, rng.normal(size=n)).astype(np.float32)
+        cond[~leaf & (rng.random(n) < 0.1)] = 0.0  # zeros and the smallest numbers meet below
+        out.append((np.array(left, dtype=np.int64), np.where(leaf, 0, rng.integers(0, features, n)),
+                    cond, np.where(leaf, 0, rng.integers(0, 2, n))))
+    return out
+
+
+def _model(forest, features, classes):
+    trees = [{"left_children": left.tolist(),
+              "right_children": np.where(left < 0, -1, left + 1).tolist(),
+              "split_indices": feature.tolist(),
+              "split_conditions": [float(c) for c in cond], "default_left": default.tolist()}
+             for left, feature, cond, default in forest]
+    objective = "reg:squarederror" if classes == 1 else "multi:softprob"
+    return json.dumps({"learner": {
+        "gradient_booster": {"model": {
+            "iteration_indptr": list(range(0, len(trees) + 1, classes)),
+            "tree_info": [t % classes for t in range(len(trees))], "trees": trees}},
+        "learner_model_param": {"base_score": json.dumps([0.25] * classes),
+                                "num_class": str(classes if classes > 1 else 0),
+                                "num_feature": str(features)},
+        "objective": {"name": objective}}})
+
+
+def _margins(forest, x, classes):
+    m = np.full((x.shape[0], classes), 0.25, dtype=np.float32)
+    rows = np.arange(x.shape[0])
+    for t, (left, feature, cond, default) in enumerate(forest):
+        node = np.zeros(x.shape[0], dtype=np.int64)
+        while (left[node] >= 0).any():
+            v = x[rows, feature[node]]
+            with np.errstate(invalid="ignore"):
+                goes_left = np.where(np.isnan(v), default[node] == 1, v < cond[node])
+            node = np.where(left[node] >= 0, left[node] + np.where(goes_left, 0, 1), node)
+        m[:, t % classes] = m[:, t % classes] + cond[node]
+    return m
+
+
+@pytest.mark.parametrize("rows,features,trees,depth,full,classes", [
+    (1, 1, 1, 0, 1.0, 1),            # one leaf
+    (64, 28, 100, 8, 0.9, 1),        # a tree per thread
+    (33, 5, 300, 3, 1.0, 3),         # many small trees, several outputs
+    (5000, 28, 40, 8, 1.0, 1),       # between the two
+    (70001, 30, 9, 6, 0.95, 1),      # a row per thread, 256 rows a workgroup
+    (140000, 60, 6, 5, 1.0, 2),      # 512 rows
+    (270001, 9, 37, 7, 0.97, 1),     # 1,024 rows, several batches
+    (70000, 20, 5, 13, 1.0, 1),      # trees beyond a batch (16,383 nodes)
+    (9000, 784, 120, 6, 1.0, 10),    # wide rows, nodes and rows in LDS
+    (2000, 5000, 12, 7, 1.0, 1),     # rows too wide for many in LDS
+    (40, 17000, 3, 4, 1.0, 1),       # features beyond the packed nodes
+    (300, 7, 2, 17, 0.995, 1),       # trees beyond the packed nodes
+    (50, 60000, 1, 2, 1.0, 1),       # rows not worth staging
+])
+def test_margins_match_a_numpy_walk(dp, device, rows, features, trees, depth, full, classes):
+    import torch
+
+    rng = np.random.default_rng(rows + features)
+    forest = _forest(rng, trees * classes, depth, features, full)
+    bst = dp.Booster.from_buffer(_model(forest, features, classes))
+    x = rng.normal(size=(rows, features)).astype(np.float32)
+    tiny = rng.random(x.shape) < 0.02
+    x[tiny] = rng.choice(np.float32([0.0, -0.0, 1e-45, -1e-45, 1e-39]), tiny.sum())
+    for missing in (False, True):
+        if missing:
+            x[rng.random(x.shape) < 0.1] = np.nan
+            x[rng.random(x.shape) < 0.01] = np.inf
+            x[rng.random(x.shape) < 0.01] = -np.inf
+        got = bst.predict(torch.as_tensor(x, device=device), margin=True).cpu().numpy()
+        np.testing.assert_array_equal(got.view(np.uint32),
+                                      _margins(forest, x, classes).view(np.uint32))
+    # a sentinel for missing values
+    y = np.where(np.isnan(x), np.float32(-999.0), x)
+    got = bst.predict(torch.as_tensor(y, device=device), margin=True, missing=-999.0)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32),
+                                  _margins(forest, x, classes).view(np.uint32))
