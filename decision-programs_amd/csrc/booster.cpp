@@ -132,6 +132,7 @@ Quantized& DMatrix::quantize(int32_t max_bin, hipStream_t s) {
   if (it != quantized.end()) return *it->second;
   need(max_bin >= 2, "max_bin must be at least 2");
   auto q = std::make_unique<Quantized>();
+  const DrainStream drain{s};
   // Cuts for up to 256 bins, with or without missing values.  uint8 bins keep
   // byte 255 for missing values, so a matrix with NaN whose features use all
   // 256 bins keeps 16-bit columns instead (below).
@@ -193,7 +194,8 @@ Quantized& DMatrix::quantize(int32_t max_bin, hipStream_t s) {
 void build_skip_bins(Quantized& q, hipStream_t s) {
   const int64_t N = q.layout.n_rows;
   const int32_t F = q.layout.n_features, T = q.layout.n_tiles;
-  DeviceBuffer<unsigned int> counts(size_t(F) * 256);
+  PooledBuffer<unsigned int> counts(size_t(F) * 256);
+  const DrainStream drain{s};
   launch_bin_counts(q.cols.p, N, F, counts.p, s);
   std::vector<unsigned int> host(counts.n);
   DP_HIP(hipMemcpyAsync(host.data(), counts.p, counts.bytes(), hipMemcpyDeviceToHost, s));
@@ -994,7 +996,8 @@ void Booster::configure(DMatrix* d) {
     init[size_t(k)] =
         objective_id_ == DP_OBJ_LOGISTIC ? float(std::log(double(b) / (1.0 - double(b)))) : b;
   }
-  DeviceBuffer<float> base(init.size());
+  PooledBuffer<float> base(init.size());
+  const DrainStream drain{stream_};
   DP_HIP(hipMemcpy(base.p, init.data(), base.bytes(), hipMemcpyHostToDevice));
   launch_init_margin(margin_.p, N, n_groups_, base.p, stream_);
   DP_HIP(hipStreamSynchronize(stream_));  // before `base` is freed
@@ -1008,7 +1011,8 @@ void Booster::update_one_iter(int iter, DMatrix* d) {
   configure(d);
   need(d->has_labels, "training DMatrix has no labels");
   if (!labels_checked_) {
-    DeviceBuffer<int32_t> bad(1);
+    PooledBuffer<int32_t> bad(1);
+    const DrainStream drain{stream_};
     launch_check_labels(d->labels.p, d->n_rows, objective_id_, n_groups_, bad.p, stream_);
     int32_t flag = 0;
     DP_HIP(hipMemcpyAsync(&flag, bad.p, sizeof flag, hipMemcpyDeviceToHost, stream_));
@@ -1172,7 +1176,7 @@ void Booster::run_round(DMatrix* d, bool with_gradients) {
   if (!sparse && !q.row_major(rows_pairs)) {
     dp_bin_layout rl = q.layout;
     rl.paired_tiles = rows_pairs;
-    auto& copy = q.rows.emplace(rows_pairs, DeviceBuffer<uint8_t>(dp_layout_bytes(&q.layout)))
+    auto& copy = q.rows.emplace(rows_pairs, PooledBuffer<uint8_t>(dp_layout_bytes(&q.layout)))
                      .first->second;
     launch_tiles_to_rows(q.bins.p, rl, copy.p, stream_);
   }

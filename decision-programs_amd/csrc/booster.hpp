@@ -19,19 +19,19 @@ struct Quantized {
   int32_t bin_stride = 0;  // largest per-feature bin count
   std::vector<int32_t> cut_ptr;
   std::vector<float> cut_values, min_values;
-  DeviceBuffer<int32_t> d_cut_ptr, d_nbins;
-  DeviceBuffer<float> d_cut_values;
-  DeviceBuffer<uint8_t> bins;
-  DeviceBuffer<uint8_t> cols;  // column-major copy: cols[f * n_rows + r]
+  PooledBuffer<int32_t> d_cut_ptr, d_nbins;
+  PooledBuffer<float> d_cut_values;
+  PooledBuffer<uint8_t> bins;
+  PooledBuffer<uint8_t> cols;  // column-major copy: cols[f * n_rows + r]
   // A matrix with missing values some of whose features use all 256 bins
   // (layout.missing_bin == kWideMissing): no uint8 bins; 16-bit columns
   // (missing: kWideMissing) for the partition, and every histogram from the
   // present-value layout built from them.
-  DeviceBuffer<uint16_t> cols16;
+  PooledBuffer<uint16_t> cols16;
   // Row-major copies, rows[(r * n_tiles + t) * 16 + j], by the pairs whose
   // joint tiles replace their first tiles (0: the plain copy); each made on
   // first use and kept, so boosters sharing the matrix never rewrite one.
-  std::map<uint64_t, DeviceBuffer<uint8_t>> rows;
+  std::map<uint64_t, PooledBuffer<uint8_t>> rows;
   const uint8_t* row_major(uint64_t pairs) const {
     const auto it = rows.find(pairs);
     return it == rows.end() ? nullptr : it->second.p;
@@ -41,7 +41,7 @@ struct Quantized {
   // frequent bin, per feature and per 16-feature tile, and the share of the
   // histogram's element atomics they remove: the rows in those bins plus the
   // last tile's padding features, over n_tiles * 16 (-1: not counted yet).
-  DeviceBuffer<uint8_t> skip_features, skip_tiles;
+  PooledBuffer<uint8_t> skip_features, skip_tiles;
   double skip_share = -1.0;
   double sparse_limit = -1.0;  // largest density limit the layout was tried with
   double density = -1.0;       // share of present values, once counted
@@ -64,8 +64,8 @@ class Booster;
 struct DMatrix {
   int64_t n_rows = 0;
   int32_t n_features = 0;
-  DeviceBuffer<float> values;  // row-major copy
-  DeviceBuffer<float> labels;
+  PooledBuffer<float> values;  // row-major copy
+  PooledBuffer<float> labels;
   bool has_labels = false;
   std::map<int32_t, std::unique_ptr<Quantized>> quantized;  // by requested max_bin
   Quantized& quantize(int32_t max_bin, hipStream_t s);

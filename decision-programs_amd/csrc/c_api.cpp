@@ -240,8 +240,9 @@ int XGDMatrixCreateFromCudaArrayInterface(const char* data, const char* config,
     obj->m.n_rows = n;
     obj->m.n_features = int32_t(f);
     obj->m.values.resize(size_t(n * f));
-    dp::DeviceBuffer<int32_t> bad(1);
+    dp::PooledBuffer<int32_t> bad(1);
     hipStream_t s = nullptr;
+    const dp::DrainStream drain{s};
     dp::launch_copy_matrix(reinterpret_cast<const float*>(a.data), row_stride, n, int32_t(f),
                            missing, obj->m.values.p, bad.p, s);
     int32_t flag = 0;
@@ -256,6 +257,7 @@ int XGDMatrixSetInfoFromInterface(DMatrixHandle handle, const char* field, const
     dp::DMatrix& m = dm(handle);
     dp::need(field && std::string(field) == "label", "only the label field is supported");
     ArrayInterface a = parse_array(data);
+    if (m.labels.p) DP_HIP(hipDeviceSynchronize());  // rounds in flight may read the old labels
     m.labels.resize(size_t(m.n_rows));
     copy_float_array(a, m.n_rows, 1, m.labels.p);
     m.has_labels = true;

@@ -27,13 +27,13 @@ inline void hip_check(hipError_t status, const char* what) {
 }
 #define DP_HIP(call) ::dp::hip_check((call), #call)
 
-// Cached allocations for the booster's training buffers (pool.cpp).  A block
-// handed back is kept, by device and exact size, for the next allocation of
-// that size (a new booster on the same configuration, a study's next trial)
-// instead of going through hipMalloc / hipHostMalloc again.  Only buffers
-// whose last use has completed may be handed back: their owners synchronise
-// their streams first.  A miss that the device cannot serve empties the cache
-// and retries.
+// Cached allocations for the matrices' and boosters' buffers (pool.cpp).  A block
+// handed back is kept, by device and rounded size, for the next allocation of
+// that size (a new booster on the same configuration, a study's next trial, the
+// next matrix) instead of going through hipMalloc / hipHostMalloc again.  Only
+// buffers whose last use has completed may be handed back: their owners
+// synchronise their streams (a matrix: the device) first.  A miss that the device
+// cannot serve empties the cache and retries.
 // device_pool_get reports the device the block belongs to (the current one);
 // device_pool_put files the block under that device, whichever is current.
 void* device_pool_get(size_t bytes, int* device);
@@ -88,6 +88,14 @@ struct DeviceBuffer {
 };
 template <class T>
 using PooledBuffer = DeviceBuffer<T, true>;
+
+// Waits for a stream on the way out of a scope, however it is left: declared after
+// the pooled buffers that the scope's launches use, so that none goes back to the
+// pool under a kernel.
+struct DrainStream {
+  hipStream_t s;
+  ~DrainStream() { (void)hipStreamSynchronize(s); }
+};
 
 // Pinned host allocation (hipHostMalloc; never hipHostRegister).
 template <bool POOLED = false>
@@ -724,13 +732,13 @@ struct SparseBins {
   int32_t tile_features = 0, n_tiles = 0;  // n_tiles 0: not built
   int32_t bin_stride = 0;                  // the stride the entries' indexes use
   int64_t nnz = 0;
-  DeviceBuffer<uint32_t> ptr;      // [n_tiles * n_rows + 1]: (tile t, row r) at t * n_rows + r
-  DeviceBuffer<uint16_t> entries;  // [nnz], tile-major (the root pass's contiguous runs)
+  PooledBuffer<uint32_t> ptr;      // [n_tiles * n_rows + 1]: (tile t, row r) at t * n_rows + r
+  PooledBuffer<uint16_t> entries;  // [nnz], tile-major (the root pass's contiguous runs)
   // The same entries row-major, for gathered rows: (row r, tile t) at
   // rptr[r * n_tiles + t], so the tile items of one row chunk, which run on one
   // XCD, read each row's offsets and entries from the same L2 lines.
-  DeviceBuffer<uint32_t> rptr;      // [n_rows * n_tiles + 1]
-  DeviceBuffer<uint16_t> rentries;  // [nnz]
+  PooledBuffer<uint32_t> rptr;      // [n_rows * n_tiles + 1]
+  PooledBuffer<uint16_t> rentries;  // [nnz]
 };
 constexpr int64_t kSparseLdsBytes = 64 * 1024;
 // LDS of one present-value tile in the histogram kernel: g and h in planes of

@@ -44,19 +44,19 @@ struct alignas(8) PackedNode {
 // A forest laid out for prediction: trees grouped by output, in boosting order
 // within each.
 struct Forest {
-  DeviceBuffer<uint8_t> nodes;       // PackedNode or PredNode
-  DeviceBuffer<float> leaf_values;   // packed: [nodes] a leaf's value
-  DeviceBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
-  DeviceBuffer<int32_t> tree_base;   // [trees] the node that the tree's indices count from
-  DeviceBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
+  PooledBuffer<uint8_t> nodes;       // PackedNode or PredNode
+  PooledBuffer<float> leaf_values;   // packed: [nodes] a leaf's value
+  PooledBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
+  PooledBuffer<int32_t> tree_base;   // [trees] the node that the tree's indices count from
+  PooledBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
   // Batches of trees whose nodes fit kPredBatchNodes: their first nodes, and per
   // batch the trees' first nodes, counted from the batch, in groups of four (the
   // last group repeats the last tree), quad_ptr[b] .. quad_ptr[b + 1] of them.
-  DeviceBuffer<int32_t> batch_node;  // [batches + 1]
-  DeviceBuffer<int32_t> quad_ptr;    // [batches + 1]
-  DeviceBuffer<int32_t> quads;       // [groups of four][4]
-  DeviceBuffer<int32_t> batch_tree;  // [batches + 1] first tree
-  DeviceBuffer<float> base;          // [groups] margin before the first tree
+  PooledBuffer<int32_t> batch_node;  // [batches + 1]
+  PooledBuffer<int32_t> quad_ptr;    // [batches + 1]
+  PooledBuffer<int32_t> quads;       // [groups of four][4]
+  PooledBuffer<int32_t> batch_tree;  // [batches + 1] first tree
+  PooledBuffer<float> base;          // [groups] margin before the first tree
   bool packed = false;
   int32_t trees = 0, groups = 1;
   int32_t batches = 0;  // 0: some tree alone exceeds kPredBatchNodes (or is not packed)

@@ -402,7 +402,13 @@ double build_sparse(int64_t N, int32_t n_features, int32_t bin_stride, double ma
   const int32_t tf = sparse_tile_features(bin_stride);
   const int32_t T = (n_features + tf - 1) / tf;
   const int64_t n = N * T;
-  DeviceBuffer<uint32_t> counts(size_t(n + 1)), ptr(size_t(n + 1));
+  // Declared before `drain`, which waits for the launches that use them.
+  PooledBuffer<uint8_t> temp, sum_temp;
+  PooledBuffer<uint16_t> entries, rentries;
+  PooledBuffer<uint32_t> rptr;
+  PooledBuffer<uint32_t> counts(size_t(n + 1)), ptr(size_t(n + 1));
+  PooledBuffer<unsigned long long> total(1);
+  const DrainStream drain{s};
   launch_fill_u8(reinterpret_cast<uint8_t*>(counts.p + n), sizeof(uint32_t), 0, s);
   count(counts.p, tf, n);
   DP_HIP(hipGetLastError());
@@ -411,15 +417,14 @@ double build_sparse(int64_t N, int32_t n_features, int32_t bin_stride, double ma
   size_t temp_bytes = 0;
   DP_HIP(rocprim::exclusive_scan(nullptr, temp_bytes, counts.p, ptr.p, 0u, size_t(n + 1),
                                  rocprim::plus<uint32_t>(), s));
-  DeviceBuffer<uint8_t> temp(temp_bytes ? temp_bytes : 1);
+  temp.resize(temp_bytes ? temp_bytes : 1);
   DP_HIP(rocprim::exclusive_scan(temp.p, temp_bytes, counts.p, ptr.p, 0u, size_t(n + 1),
                                  rocprim::plus<uint32_t>(), s));
-  DeviceBuffer<unsigned long long> total(1);
   launch_fill_u8(reinterpret_cast<uint8_t*>(total.p), sizeof(unsigned long long), 0, s);
   size_t sum_bytes = 0;
   DP_HIP(rocprim::reduce(nullptr, sum_bytes, counts.p, total.p, 0ull, size_t(n),
                          rocprim::plus<unsigned long long>(), s));
-  DeviceBuffer<uint8_t> sum_temp(sum_bytes ? sum_bytes : 1);
+  sum_temp.resize(sum_bytes ? sum_bytes : 1);
   DP_HIP(rocprim::reduce(sum_temp.p, sum_bytes, counts.p, total.p, 0ull, size_t(n),
                          rocprim::plus<unsigned long long>(), s));
   unsigned long long nnz = 0;
@@ -427,18 +432,18 @@ double build_sparse(int64_t N, int32_t n_features, int32_t bin_stride, double ma
   DP_HIP(hipStreamSynchronize(s));
   const double density = double(nnz) / (double(N) * double(n_features));
   if (density > max_density || nnz >= (1ull << 32)) return density;
-  DeviceBuffer<uint16_t> entries(size_t(nnz + kSparseEntryPad));
+  entries.resize(size_t(nnz + kSparseEntryPad));
   fill(ptr.p, entries.p, tf, n);
   DP_HIP(hipGetLastError());
   // The row-major copy: counts in (row, tile) order, their exclusive scan,
   // then each (row, tile)'s entries copied to its place.
-  DeviceBuffer<uint32_t> rptr(size_t(n + 1));
+  rptr.resize(size_t(n + 1));
   const dim3 grid(grid_for(n, 256, 16384));
   hipLaunchKernelGGL(sparse_row_counts_kernel, grid, dim3(256), 0, s, ptr.p, N, T, counts.p);
   DP_HIP(hipGetLastError());
   DP_HIP(rocprim::exclusive_scan(temp.p, temp_bytes, counts.p, rptr.p, 0u, size_t(n + 1),
                                  rocprim::plus<uint32_t>(), s));
-  DeviceBuffer<uint16_t> rentries(size_t(nnz + kSparseEntryPad));
+  rentries.resize(size_t(nnz + kSparseEntryPad));
   hipLaunchKernelGGL(sparse_row_fill_kernel, grid, dim3(256), 0, s, ptr.p, entries.p, N, T,
                      rptr.p, rentries.p);
   DP_HIP(hipGetLastError());

@@ -765,11 +765,7 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
   PooledBuffer<int32_t> used, rank_bucket;
   PooledBuffer<FeaturePlan> plans;
   PooledBuffer<unsigned long long> gathered;
-  // Whatever ends the call, no buffer goes back to the pool under a kernel.
-  struct Drain {
-    hipStream_t s;
-    ~Drain() { (void)hipStreamSynchronize(s); }
-  } drain{s};
+  const DrainStream drain{s};
   if (n_rows <= kSortRows) {
     const auto kernel = n_rows <= 8192 ? sort_cuts_kernel<8192, 3> : sort_cuts_kernel<16384, 4>;
     hipLaunchKernelGGL(kernel, dim3(n_features), dim3(kThreads), 0, s, values, int32_t(n_rows),
