@@ -453,13 +453,12 @@ void Grower::grow(const Quantized& q, const int32_t* gpair, const int32_t* exps,
                          colsample, d, fmask_.p, s);
         fmask = fmask_.p;
       }
-      // The present-value layout's partial slots hold node-histogram words: its
-      // levels reduce and evaluate in one launch (up to 64 bins).
-      const bool fused = sparse_ && B <= 64 && tf % 16 == 0 && exps;
-      // The last split level's histograms have no readers: a fused launch
-      // evaluates them without storing them.
+      // Every level reduces and evaluates in one launch; the present-value layout
+      // with at most 64 bins by its own kernel (four features per wavefront).
+      const bool fused = sparse_ && B <= 64 && tf % 16 == 0;
+      // The last split level's histograms have no readers: they are evaluated
+      // without being stored.
       const bool keep = d + 1 < D;
-      bool dense_fused = false;  // set below for dense passes with at least kDenseFuseFeatures features
       if (d == 0 && sparse_) {
         launch_hist_sparse(q.sparse, N, F, gpair, nullptr, root_work_.p, root_items_, nullptr, B,
                            h, partial_.p, s);
@@ -468,19 +467,17 @@ void Grower::grow(const Quantized& q, const int32_t* gpair, const int32_t* exps,
                                       q.d_nbins.p, sums_[cur].p, exps, dtp, fmask,
                                       skip_features_, eval_scratch_.p, keep, s);
         else
-          launch_hist_reduce_flat(partial_.p, root_job_.p, 1, nullptr, T, tf, F, B, nullptr, h, s);
+          launch_reduce_evaluate_dense(partial_.p, root_job_.p, 1, nullptr, T, tf, F, B, nullptr, h,
+                                       q.d_nbins.p, sums_[cur].p, exps, dtp, fmask,
+                                       skip_features_, eval_scratch_.p, keep, s);
       } else if (d == 0) {
         // The root, as the levels below it: feature-major partial slots, and
         // the reduce and the evaluation in one launch (one job, no sibling).
-        dense_fused = F >= kDenseFuseFeatures && B <= 256 && exps;
         launch_hist(q.bins.p, lay_, gpair, nullptr, root_work_.p, root_items_, nullptr, B, h,
-                    partial_.p, s, nullptr, root_cfg_, skip_tiles_, dense_fused);
-        if (dense_fused)
-          launch_reduce_evaluate_dense(partial_.p, root_job_.p, 1, nullptr, T, F, B, nullptr, h,
-                                       q.d_nbins.p, sums_[cur].p, exps, dtp, fmask,
-                                       skip_features_, eval_scratch_.p, keep, s);
-        else
-          launch_hist_reduce(partial_.p, root_job_.p, 1, nullptr, T, F, B, nullptr, h, false, s);
+                    partial_.p, s, nullptr, root_cfg_, skip_tiles_, true);
+        launch_reduce_evaluate_dense(partial_.p, root_job_.p, 1, nullptr, T, 16, F, B, nullptr,
+                                     h, q.d_nbins.p, sums_[cur].p, exps, dtp, fmask, skip_features_,
+                                     eval_scratch_.p, keep, s);
       } else if (sparse_) {
         // On the last split level of a fused tree, and on levels of at least
         // kInPassNodes nodes (mostly small ones), the nodes built in one chunk
@@ -510,37 +507,23 @@ void Grower::grow(const Quantized& q, const int32_t* gpair, const int32_t* exps,
                                       h, q.d_nbins.p, sums_[cur].p, exps, dtp, fmask,
                                       skip_features_, eval_scratch_.p, keep, s, in_pass);
         else
-          launch_hist_reduce_flat(partial_.p, reduce_jobs_[cur].p, int32_t(nb / 2 + 1),
-                                  field(c, &PlanCounts::n_reduce), T, tf, F, B, hist_[nxt].p, h,
-                                  s);
+          launch_reduce_evaluate_dense(partial_.p, reduce_jobs_[cur].p, int32_t(nb / 2 + 1),
+                                       field(c, &PlanCounts::n_reduce), T, tf, F, B,
+                                       hist_[nxt].p, h, q.d_nbins.p, sums_[cur].p, exps, dtp,
+                                       fmask, skip_features_, eval_scratch_.p, keep, s);
       } else {
         const int32_t G =
             hist_groups(T, level_cfg_.tiles, hist_pairs(lay_.paired_tiles, level_cfg_.tiles));
-        // Levels below the root with more features than one evaluation
-        // workgroup takes: feature-major partial slots, and the reduce and the
-        // evaluation in one launch (measured: C2 2,474 -> 2,560, C3 455 ->
-        // 463, C4 3,321 -> 3,886 trees/s).
-        dense_fused = F >= kDenseFuseFeatures && B <= 256 && exps;
         launch_hist(q.bins.p, lay_, gpair, ridx_[cur].p, hist_work_[cur].p,
                     int32_t(plan_hist_items(nb, N, G, level_cfg_.items)),
                     field(c, &PlanCounts::n_hist), B, h, partial_.p, s, rows_major_, level_cfg_,
-                    skip_tiles_, dense_fused);
-        if (dense_fused)
-          launch_reduce_evaluate_dense(partial_.p, reduce_jobs_[cur].p, int32_t(nb / 2 + 1),
-                                       field(c, &PlanCounts::n_reduce), T, F, B, hist_[nxt].p, h,
-                                       q.d_nbins.p, sums_[cur].p, exps, dtp, fmask,
-                                       skip_features_, eval_scratch_.p, keep, s);
-        else
-          launch_hist_reduce(partial_.p, reduce_jobs_[cur].p, int32_t(nb / 2 + 1),
-                             field(c, &PlanCounts::n_reduce), T, F, B, hist_[nxt].p, h, false, s);
+                    skip_tiles_, true);
+        launch_reduce_evaluate_dense(partial_.p, reduce_jobs_[cur].p, int32_t(nb / 2 + 1),
+                                     field(c, &PlanCounts::n_reduce), T, 16, F, B, hist_[nxt].p,
+                                     h, q.d_nbins.p, sums_[cur].p, exps, dtp, fmask, skip_features_,
+                                     eval_scratch_.p, keep, s);
       }
-      // Without records from the evaluation, the count launch selects them.
-      const bool records =
-          fused || dense_fused
-              ? false
-              : launch_evaluate(h, int32_t(nb), field(c, &PlanCounts::n_level), F, B,
-                                q.d_nbins.p, sums_[cur].p, exps, 0, 0, dtp, eval_scratch_.p,
-                                splits_.p, s, false, fmask, skip_features_);
+      // The count launch selects each node's split from the candidates.
       SplitSelect sel;
       sel.cand = reinterpret_cast<const FeatCand*>(eval_scratch_.p);
       sel.n_features = F;
@@ -578,7 +561,7 @@ void Grower::grow(const Quantized& q, const int32_t* gpair, const int32_t* exps,
                        seg_begin_[cur].p, splits_.p, part_first_[cur].p, int32_t(nb),
                        field(c, &PlanCounts::n_level), work_left_.p, part_masks_.p,
                        node_left_[cur].p, true, s, d > 0 ? &prev : nullptr,
-                       records ? nullptr : &sel, merged && !fuse_last ? &scatter : nullptr,
+                       &sel, merged && !fuse_last ? &scatter : nullptr,
                        fuse_last ? &ll : nullptr);
     }
     PlanArgs a{};

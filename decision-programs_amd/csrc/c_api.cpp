@@ -683,8 +683,8 @@ void hist_call(dp_workspace ws, const uint8_t* bins, const dp_bin_layout* layout
   int64_t* partial = partial_words ? ws->take<int64_t>(partial_words) : nullptr;
   dp::launch_hist(bins, *layout, gpair, ridx, d_work, int32_t(work.size()), nullptr, bin_stride,
                   hist, partial, s, nullptr, cfg);
-  dp::launch_hist_reduce(partial, d_jobs, n_nodes, nullptr, layout->n_tiles, layout->n_features,
-                         bin_stride, nullptr, hist, accumulate, s);
+  dp::launch_hist_reduce(partial, d_jobs, n_nodes, layout->n_tiles, layout->n_features,
+                         bin_stride, hist, accumulate, s);
 }
 }  // namespace
 
@@ -738,8 +738,8 @@ int dp_evaluate_splits(dp_workspace ws, const int64_t* hist, int32_t n_nodes,
     ws->begin(0);
     ws->reserve_scratch(bytes + 256);
     void* scratch = ws->take<uint8_t>(bytes);
-    dp::launch_evaluate(hist, n_nodes, nullptr, n_features, bin_stride, n_bins, node_sums, nullptr,
-                        exp_g, exp_h, *param, scratch, out, as_stream(stream));
+    dp::launch_evaluate(hist, n_nodes, n_features, bin_stride, n_bins, node_sums, exp_g, exp_h,
+                        *param, scratch, out, as_stream(stream));
   });
 }
 
@@ -756,8 +756,8 @@ int dp_evaluate_splits_noalloc(const int64_t* hist, int32_t n_nodes, int32_t n_f
     const size_t bytes =
         n_features > dp::kEvalNodeFeatures ? dp::evaluate_scratch_bytes(n_nodes, n_features) : 0;
     void* scratch = dp::noalloc_scratch(bytes);
-    dp::launch_evaluate(hist, n_nodes, nullptr, n_features, bin_stride, n_bins, node_sums, nullptr,
-                        exp_g, exp_h, *param, scratch, out, as_stream(stream));
+    dp::launch_evaluate(hist, n_nodes, n_features, bin_stride, n_bins, node_sums, exp_g, exp_h,
+                        *param, scratch, out, as_stream(stream));
   });
 }
 

@@ -354,12 +354,12 @@ void launch_hist(const uint8_t* bins, const dp_bin_layout& layout, const int32_t
 // from the column copy cols[f][row].
 void launch_bin_counts(const uint8_t* cols, int64_t n_rows, int32_t n_features,
                        unsigned int* counts, hipStream_t s);
-// Completes the histograms of launch_hist: sums partial tiles, writes built
-// and sibling node histograms.  accumulate: add the sums to hist instead of
-// storing them (then no job may rely on a direct item).
+// Completes the histograms of launch_hist (without fmaj; the booster's levels:
+// launch_reduce_evaluate_dense): sums the partial tiles of each job's node.
+// accumulate: add the sums to hist instead of storing them (then no job may rely
+// on a direct item).
 void launch_hist_reduce(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                        const int32_t* n_jobs_dev, int32_t n_tiles, int32_t n_features,
-                        int32_t bin_stride, const int64_t* parent_base, int64_t* hist,
+                        int32_t n_tiles, int32_t n_features, int32_t bin_stride, int64_t* hist,
                         bool accumulate, hipStream_t s);
 // Minimum rows per histogram chunk and the chunk size for `rows` rows when
 // each row chunk makes `groups` work items: at most `items` work items in all
@@ -435,29 +435,26 @@ void launch_subtract(const int64_t* parent, const int64_t* built, int64_t* sibli
                      hipStream_t s);
 
 
-// Split evaluation; scratch holds evaluate_scratch_bytes(n_nodes, n_features)
-// (the per-feature candidates, as FeatCand [node][feature]).  Returns whether
-// the split records were written: always with select; without it, only for
-// matrices few enough features for one workgroup per node -- otherwise the
-// caller selects from the candidates (SplitSelect in launch_partition).
-// With at most kEvalNodeFeatures features the evaluation writes the split
-// records itself (one workgroup per node) and uses no scratch.
+// Split evaluation of the operators; scratch holds evaluate_scratch_bytes(n_nodes,
+// n_features) (the per-feature candidates, as FeatCand [node][feature]).  With at
+// most kEvalNodeFeatures features one workgroup per node writes the split record
+// itself and uses no scratch.
 constexpr int kEvalNodeFeatures = 16;
 size_t evaluate_scratch_bytes(int32_t n_nodes, int32_t n_features);
-bool launch_evaluate(const int64_t* hist, int32_t n_nodes, const int32_t* n_nodes_dev,
-                     int32_t n_features, int32_t bin_stride, const int32_t* n_bins,
-                     const int64_t* node_sums, const int32_t* exps, int32_t exp_g, int32_t exp_h,
-                     const dp_train_param& param, void* scratch, dp_split_record* out,
-                     hipStream_t s, bool select = true, const uint32_t* fmask = nullptr,
-                     const uint8_t* skip_bins = nullptr);
+void launch_evaluate(const int64_t* hist, int32_t n_nodes, int32_t n_features, int32_t bin_stride,
+                     const int32_t* n_bins, const int64_t* node_sums, int32_t exp_g,
+                     int32_t exp_h, const dp_train_param& param, void* scratch,
+                     dp_split_record* out, hipStream_t s);
+// Reduce and evaluation of the booster's levels, in one launch: the node
+// histograms (built from the partial slots, sibling = parent - built; none stored
+// when !store) and the per-feature candidates, which the partition count selects
+// from (SplitSelect).
+// fmask: column samples (launch_colsample), or null.
 // skip_bins ([n_features] bytes, matrices without missing values): the
 // histograms leave each feature's skip bin at zero (launch_hist's skip); the
 // node's remaining sums (totals minus the bins) are that bin's.
-// Present-value layout (at most 64 bins, tiles of a multiple of 16 features):
-// launch_hist_reduce_flat and launch_evaluate(..., select = false) in one
-// launch -- the same node histograms (built and sibling) and the same
-// per-feature candidates in scratch.  exps: the quantiser exponents in device
-// memory.  skip_direct: jobs whose node was built by one direct item are left
+// Present-value layout with at most 64 bins.  exps: the quantiser exponents in
+// device memory.  skip_direct: jobs whose node was built by one direct item are left
 // alone (launch_hist_sparse's evaluation did them).
 void launch_reduce_evaluate_flat(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
                                  const int32_t* n_jobs_dev, int32_t n_tiles, int32_t tile_features,
@@ -467,18 +464,20 @@ void launch_reduce_evaluate_flat(const int64_t* partial, const HistReduce* jobs,
                                  const dp_train_param& param, const uint32_t* fmask,
                                  const uint8_t* skip_bins, void* scratch, bool store,
                                  hipStream_t s, bool skip_direct = false);
-// Feature counts from which the booster's dense levels below the root use
-// feature-major partial slots and launch_reduce_evaluate_dense, and from which
-// that launch takes four features per workgroup instead of one.
-constexpr int32_t kDenseFuseFeatures = 17;
+// The feature count from which launch_reduce_evaluate_dense takes four features
+// per workgroup instead of one.
 constexpr int32_t kDenseWideFeatures = 256;
-// Dense levels whose partial slots are feature-major (launch_hist's fmaj):
-// launch_hist_reduce and launch_evaluate(..., select = false) in one launch --
-// the same node histograms (built and sibling; none stored when !store) and the
-// same per-feature candidates in scratch.  At most 256 bins.
+// Feature-major partial slots, [tile_features][bin_stride][g, h] per tile: dense
+// levels (16-feature tiles, launch_hist's fmaj) and the present-value layout with
+// more than 64 bins.  Separate reduce and evaluation launches measured slower at
+// every width: on dense matrices of up to 16 features, whose evaluation also chose
+// the split, rounds of 10k x 8 took 186 against 167 us, 100k x 16 223 against 195,
+// 1M x 8 370 against 353, 3M x 5 the same 460; on present-value ones of 500k x 20
+// with 255 bins 306 against 292, 200k x 300 with 128 bins 271 against 262.
 void launch_reduce_evaluate_dense(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                                  const int32_t* n_jobs_dev, int32_t n_tiles, int32_t n_features,
-                                  int32_t bin_stride, const int64_t* parent_base, int64_t* hist,
+                                  const int32_t* n_jobs_dev, int32_t n_tiles,
+                                  int32_t tile_features, int32_t n_features, int32_t bin_stride,
+                                  const int64_t* parent_base, int64_t* hist,
                                   const int32_t* n_bins, const int64_t* node_sums,
                                   const int32_t* exps, const dp_train_param& param,
                                   const uint32_t* fmask, const uint8_t* skip_bins, void* scratch,
@@ -546,8 +545,8 @@ struct LastLevel {
 // launch_plan_scatter.  last: the last split level's margin update is done by
 // the count launch, and no scatter is launched or deferred (ridx_out is not
 // written; the count still writes work_left for the level's planner).
-// Per-feature candidates left by launch_evaluate(..., select = false): the
-// partition count selects each node's split from them and writes the records.
+// Per-feature candidates left by the reduce-and-evaluate launch: the partition
+// count selects each node's split from them and writes the records.
 struct SplitSelect {
   const FeatCand* cand = nullptr;
   int32_t n_features = 0;
@@ -775,7 +774,7 @@ void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_feature
                           hipStream_t s);
 // Histograms from the present-value layout: work items as for launch_hist,
 // with `tile` a sparse tile; partial slots of tile_features * bin_stride * 2
-// words in the node histogram's layout.  Finished by launch_hist_reduce_flat.
+// words in the node histogram's layout.
 // The evaluation a present-value pass does for the nodes it builds in one
 // chunk (HistWork::partial < 0; HistWork::parent names the sibling): the
 // node's and its sibling's words and per-feature candidates of
@@ -799,10 +798,7 @@ void launch_hist_sparse(const SparseBins& sp, int64_t n_rows, int32_t n_features
                         int32_t n_work, const int32_t* n_work_dev, int32_t bin_stride,
                         int64_t* hist, int64_t* partial, hipStream_t s,
                         const SparseEval* eval = nullptr);
-void launch_hist_reduce_flat(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                             const int32_t* n_jobs_dev, int32_t n_tiles, int32_t tile_features,
-                             int32_t n_features, int32_t bin_stride, const int64_t* parent_base,
-                             int64_t* hist, hipStream_t s);
+
 
 // rows[r * n_tiles * 16 + t * 16 + j] = tile t's byte j of row r; for the
 // first tile t of each of the layout's pairs, the pair's joint tile instead

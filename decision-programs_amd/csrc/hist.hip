@@ -747,39 +747,6 @@ __device__ __forceinline__ long long sum_slots(const long long* __restrict__ src
   return ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
 }
 
-// Reduce for the present-value path: partial slots hold a sparse tile in the
-// node histogram's layout, so word e of tile t is word t * tile_features *
-// bin_stride * 2 + e of the node histogram.  Otherwise as hist_reduce_kernel.
-__global__ __launch_bounds__(256) void hist_reduce_flat_kernel(
-    const long long* __restrict__ partial, const HistReduce* __restrict__ jobs,
-    int32_t n_jobs_host, const int32_t* __restrict__ n_jobs_dev, int32_t n_tiles,
-    int32_t tile_features, int32_t n_features, int32_t bin_stride,
-    const long long* __restrict__ parent_base, long long* __restrict__ hist) {
-  const int32_t n_jobs = n_jobs_dev ? *n_jobs_dev : n_jobs_host;
-  const int t = blockIdx.y;
-  const int32_t f0 = t * tile_features;
-  const int32_t nf = f0 + tile_features < n_features ? tile_features : n_features - f0;
-  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (e >= int64_t(nf) * bin_stride * 2) return;  // no barriers below
-  const int64_t slot_words = int64_t(tile_features) * bin_stride * 2;
-  const int64_t node_elems = int64_t(n_features) * bin_stride * 2;
-  const int64_t at = int64_t(f0) * bin_stride * 2 + e;
-  for (int32_t jb = blockIdx.z; jb < n_jobs; jb += gridDim.z) {
-    const HistReduce j = jobs[jb];
-    long long* built = hist + int64_t(j.slot) * node_elems + at;
-    long long sum;
-    if (j.nc == 1 && j.p0 < 0) {
-      sum = *built;  // written directly by the node's only chunk
-    } else {
-      sum = sum_slots(partial + (int64_t(j.p0) * n_tiles + t) * slot_words + e,
-                      int64_t(n_tiles) * slot_words, j.nc);
-      *built = sum;
-    }
-    if (j.sibling >= 0)
-      hist[int64_t(j.sibling) * node_elems + at] = parent_base[j.parent + at] - sum;
-  }
-}
-
 __global__ void zero_i64_dev_kernel(int64_t* __restrict__ p, const int32_t* __restrict__ n_dev,
                                     int64_t per) {
   const int64_t n = int64_t(*n_dev) * per;
@@ -801,12 +768,9 @@ __global__ void subtract_kernel(const int64_t* __restrict__ parent,
 // word over the job's partial slots and writes the built and sibling values in
 // the [feature][bin][g, h] layout.
 __global__ __launch_bounds__(256) void hist_reduce_kernel(
-    const long long* __restrict__ partial, const HistReduce* __restrict__ jobs,
-    int32_t n_jobs_host, const int32_t* __restrict__ n_jobs_dev, int32_t n_tiles,
-    int32_t n_features, int32_t bin_stride, const long long* __restrict__ parent_base,
-    long long* __restrict__ hist, int32_t accumulate) {
-  const HistReduce j_first = int32_t(blockIdx.z) < n_jobs_host ? jobs[blockIdx.z] : HistReduce{};
-  const int32_t n_jobs = n_jobs_dev ? *n_jobs_dev : n_jobs_host;
+    const long long* __restrict__ partial, const HistReduce* __restrict__ jobs, int32_t n_jobs,
+    int32_t n_tiles, int32_t n_features, int32_t bin_stride, long long* __restrict__ hist,
+    int32_t accumulate) {
   const int n_words = bin_stride * 32;
   const int e = blockIdx.x * 256 + threadIdx.x;
   const int t = blockIdx.y;
@@ -816,19 +780,13 @@ __global__ __launch_bounds__(256) void hist_reduce_kernel(
   const int64_t node_elems = int64_t(n_features) * bin_stride * 2;
   const int64_t at = (int64_t(f) * bin_stride + bin) * 2 + (within >> 4);
   for (int32_t jb = blockIdx.z; jb < n_jobs; jb += gridDim.z) {
-    const HistReduce j = jb == int32_t(blockIdx.z) ? j_first : jobs[jb];
+    const HistReduce j = jobs[jb];
+    if (j.nc == 1 && j.p0 < 0) continue;  // the node's only chunk wrote it
     long long* built = hist + int64_t(j.slot) * node_elems + at;
-    long long sum;
-    if (j.nc == 1 && j.p0 < 0) {
-      sum = *built;  // written directly by the node's only chunk
-    } else {
-      sum = sum_slots(partial + (int64_t(j.p0) * n_tiles + t) * n_words + e,
-                      int64_t(n_tiles) * n_words, j.nc);
-      if (accumulate) sum += *built;
-      *built = sum;
-    }
-    if (j.sibling >= 0)
-      hist[int64_t(j.sibling) * node_elems + at] = parent_base[j.parent + at] - sum;
+    long long sum = sum_slots(partial + (int64_t(j.p0) * n_tiles + t) * n_words + e,
+                              int64_t(n_tiles) * n_words, j.nc);
+    if (accumulate) sum += *built;
+    *built = sum;
   }
 }
 
@@ -840,10 +798,10 @@ __global__ __launch_bounds__(256) void hist_reduce_kernel(
 constexpr int kWideGroups = 4;
 __global__ __launch_bounds__(256 * kWideGroups) void hist_reduce_wide_kernel(
     const long long* __restrict__ partial, const HistReduce* __restrict__ jobs, int32_t n_tiles,
-    int32_t n_features, int32_t bin_stride, const long long* __restrict__ parent_base,
-    long long* __restrict__ hist, int32_t accumulate) {
+    int32_t n_features, int32_t bin_stride, long long* __restrict__ hist, int32_t accumulate) {
   __shared__ long long part[kWideGroups - 1][256];
   const HistReduce j = jobs[0];
+  if (j.nc == 1 && j.p0 < 0) return;  // the node's only chunk wrote it
   const int q = threadIdx.x >> 8, t = threadIdx.x & 255;
   const int n_words = bin_stride * 32;
   const int e = blockIdx.x * 256 + t;
@@ -851,9 +809,8 @@ __global__ __launch_bounds__(256 * kWideGroups) void hist_reduce_wide_kernel(
   const int within = e & 31, bin = e >> 5;
   const int f = tile * kTile + (within & 15);
   const bool live = e < n_words && f < n_features;
-  const bool direct = j.nc == 1 && j.p0 < 0;  // uniform: the node's only chunk wrote it
   long long sum = 0;
-  if (live && !direct && q < j.nc) {
+  if (live && q < j.nc) {
     const int32_t nq = (j.nc - q + kWideGroups - 1) / kWideGroups;  // slots q, q + 4, ...
     sum = sum_slots(partial + (int64_t(j.p0 + q) * n_tiles + tile) * n_words + e,
                     int64_t(kWideGroups) * n_tiles * n_words, nq);
@@ -864,15 +821,10 @@ __global__ __launch_bounds__(256 * kWideGroups) void hist_reduce_wide_kernel(
   const int64_t node_elems = int64_t(n_features) * bin_stride * 2;
   const int64_t at = (int64_t(f) * bin_stride + bin) * 2 + (within >> 4);
   long long* built = hist + int64_t(j.slot) * node_elems + at;
-  if (direct) {
-    sum = *built;
-  } else {
 #pragma unroll
-    for (int k = 0; k < kWideGroups - 1; ++k) sum += part[k][t];
-    if (accumulate) sum += *built;
-    *built = sum;
-  }
-  if (j.sibling >= 0) hist[int64_t(j.sibling) * node_elems + at] = parent_base[j.parent + at] - sum;
+  for (int k = 0; k < kWideGroups - 1; ++k) sum += part[k][t];
+  if (accumulate) sum += *built;
+  *built = sum;
 }
 
 }  // namespace
@@ -1114,28 +1066,22 @@ void launch_subtract(const int64_t* parent, const int64_t* built, int64_t* sibli
 }
 
 void launch_hist_reduce(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                        const int32_t* n_jobs_dev, int32_t n_tiles, int32_t n_features,
-                        int32_t bin_stride, const int64_t* parent_base, int64_t* hist,
+                        int32_t n_tiles, int32_t n_features, int32_t bin_stride, int64_t* hist,
                         bool accumulate, hipStream_t s) {
   if (n_jobs <= 0) return;
   need(bin_stride >= 1 && bin_stride <= kMaxBins, "histogram bin stride out of range");
-  if (n_jobs == 1 && !n_jobs_dev) {  // one node (a root pass): the wide reduce
-    hipLaunchKernelGGL(hist_reduce_wide_kernel,
-                       dim3(unsigned(bin_stride * 32 + 255) / 256, unsigned(n_tiles)),
-                       dim3(256 * kWideGroups), 0, s, reinterpret_cast<const long long*>(partial),
-                       jobs, n_tiles, n_features, bin_stride,
-                       reinterpret_cast<const long long*>(parent_base),
-                       reinterpret_cast<long long*>(hist), accumulate ? 1 : 0);
-    DP_HIP(hipGetLastError());
-    return;
-  }
-  const dim3 grid(unsigned(bin_stride * 32 + 255) / 256, unsigned(n_tiles),
-                  unsigned(n_jobs < 64 ? n_jobs : 64));
-  hipLaunchKernelGGL(hist_reduce_kernel, grid, dim3(256), 0, s,
-                     reinterpret_cast<const long long*>(partial), jobs, n_jobs, n_jobs_dev,
-                     n_tiles, n_features, bin_stride,
-                     reinterpret_cast<const long long*>(parent_base),
-                     reinterpret_cast<long long*>(hist), accumulate ? 1 : 0);
+  auto* out = reinterpret_cast<long long*>(hist);
+  const auto* in = reinterpret_cast<const long long*>(partial);
+  const unsigned words = unsigned(bin_stride * 32 + 255) / 256;
+  if (n_jobs == 1)  // one node (a root pass): the wide reduce
+    hipLaunchKernelGGL(hist_reduce_wide_kernel, dim3(words, unsigned(n_tiles)),
+                       dim3(256 * kWideGroups), 0, s, in, jobs, n_tiles, n_features, bin_stride,
+                       out, accumulate ? 1 : 0);
+  else
+    hipLaunchKernelGGL(hist_reduce_kernel,
+                       dim3(words, unsigned(n_tiles), unsigned(n_jobs < 64 ? n_jobs : 64)),
+                       dim3(256), 0, s, in, jobs, n_jobs, n_tiles, n_features, bin_stride, out,
+                       accumulate ? 1 : 0);
   DP_HIP(hipGetLastError());
 }
 
@@ -1185,22 +1131,6 @@ void launch_hist_sparse(const SparseBins& sp, int64_t n_rows, int32_t n_features
                      reinterpret_cast<unsigned long long*>(hist),
                      reinterpret_cast<unsigned long long*>(partial), ev,
                      rows ? sp.n_tiles : 1);
-  DP_HIP(hipGetLastError());
-}
-
-void launch_hist_reduce_flat(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                             const int32_t* n_jobs_dev, int32_t n_tiles, int32_t tile_features,
-                             int32_t n_features, int32_t bin_stride, const int64_t* parent_base,
-                             int64_t* hist, hipStream_t s) {
-  if (n_jobs <= 0) return;
-  const int64_t words = int64_t(tile_features) * bin_stride * 2;
-  const dim3 grid(unsigned((words + 255) / 256), unsigned(n_tiles),
-                  unsigned(n_jobs < 64 ? n_jobs : 64));
-  hipLaunchKernelGGL(hist_reduce_flat_kernel, grid, dim3(256), 0, s,
-                     reinterpret_cast<const long long*>(partial), jobs, n_jobs, n_jobs_dev,
-                     n_tiles, tile_features, n_features, bin_stride,
-                     reinterpret_cast<const long long*>(parent_base),
-                     reinterpret_cast<long long*>(hist));
   DP_HIP(hipGetLastError());
 }
 

@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void evaluate_features_seg_kernel(
 // only chunk wrote), writes the built and sibling words, and evaluates both
 // nodes' feature from its registers.  No barriers, and no second pass over the
 // level's histograms: the words and candidates are those of
-// hist_reduce_flat_kernel followed by evaluate_features_seg_kernel.  With
+// a reduce launch followed by evaluate_features_seg_kernel.  With
 // store == 0 (the tree's last split level, whose histograms no later level
 // reads) the built and sibling words are evaluated but not written.  With
 // skip_direct, jobs whose node was built by its only chunk are left alone:
@@ -304,36 +304,39 @@ __global__ __launch_bounds__(256) void reduce_evaluate_flat_kernel(
   }
 }
 
-// Reduce and evaluate in one launch for dense levels whose partial slots are
-// feature-major ([16 features][bin_stride][g, h] per tile: hist_kernel's fmaj
-// flush, so a feature's words in a slot are contiguous), for wide matrices
-// (many workgroups per job, nodes of few chunks).  One wavefront per
-// feature, four per 256-thread workgroup, lane l holding bins 4l .. 4l + 3 as
-// evaluate_features_kernel<4> does: the lane sums the job's partial slots of
-// its 64 contiguous bytes (or reads what the node's only chunk wrote), writes
-// the built and sibling words (with store), and evaluates both nodes' feature
-// from its registers -- the words and candidates of hist_reduce_kernel
-// followed by evaluate_features_kernel<4>, with one launch and one pass over
-// the level's histograms fewer.  Bins past bin_stride read the feature's last
+// Reduce and evaluate in one launch for levels whose partial slots are
+// feature-major ([tile_features][bin_stride][g, h] per tile: hist_kernel's fmaj
+// flush of 16 features, or the present-value tiles' of more, so a feature's words
+// in a slot are contiguous), for wide matrices (many workgroups per job, nodes of
+// few chunks).  One wavefront per feature, four per 256-thread workgroup, lane l
+// holding bins BPL l .. BPL l + BPL - 1 as evaluate_features_kernel does (BPL: the
+// fewest of 1, 2, 4 that hold bin_stride bins; idle lanes otherwise sum and
+// evaluate masked bins: 300k x 300 with 128 bins 334 -> 317 us a round, 1M x 20
+// with 64 bins 360 -> 337): the lane sums the job's partial slots of its 16 BPL
+// contiguous bytes (or reads what the node's only chunk wrote), writes the built
+// and sibling words (with store), and evaluates both nodes' feature from its
+// registers, with one launch and one pass over the level's histograms fewer than
+// separate launches.  Bins past bin_stride read the feature's last
 // bin and are masked (branch-free loads).  No barriers.
 constexpr int kDenseEvalFeatures = 4;  // features per workgroup (one per wavefront)
 constexpr int64_t kDenseOneRound = 1024;  // four-wave reduce-evaluate workgroups 256 CUs hold at once
+template <int BPL>
 __global__ __launch_bounds__(64 * kDenseEvalFeatures) void reduce_evaluate_dense_kernel(
     const long long* __restrict__ partial, const HistReduce* __restrict__ jobs,
     int32_t n_jobs_host, const int32_t* __restrict__ n_jobs_dev, int32_t n_tiles,
-    int32_t n_features, int32_t bin_stride, const long long* __restrict__ parent_base,
-    long long* __restrict__ hist, const int32_t* __restrict__ n_bins,
+    int32_t tile_features, int32_t n_features, int32_t bin_stride,
+    const long long* __restrict__ parent_base, long long* __restrict__ hist,
+    const int32_t* __restrict__ n_bins,
     const long long* __restrict__ node_sums, const int32_t* __restrict__ exps, Param p,
     const uint32_t* __restrict__ fmask, const uint8_t* __restrict__ skip_bins,
     FeatCand* __restrict__ cand, int32_t store) {
-  constexpr int BPL = 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int32_t f = int32_t(blockIdx.x) * kDenseEvalFeatures + wave;
   if (f >= n_features) return;  // wave-uniform; no barriers in this kernel
   const HistReduce j_first = int32_t(blockIdx.y) < n_jobs_host ? jobs[blockIdx.y] : HistReduce{};
   const int32_t n_jobs = n_jobs_dev ? *n_jobs_dev : n_jobs_host;
-  const int32_t tile = f >> 4, fl = f & 15;
-  const int64_t slot_words = int64_t(bin_stride) * 32;  // a tile's partial slot
+  const int32_t tile = f / tile_features, fl = f - tile * tile_features;
+  const int64_t slot_words = int64_t(bin_stride) * tile_features * 2;  // a tile's partial slot
   const int64_t node_elems = int64_t(n_features) * bin_stride * 2;
   bool ok[BPL];
   int64_t at[BPL], pat[BPL];  // word of bin (g; h is + 1): node histogram, partial slot
@@ -427,43 +430,37 @@ __global__ __launch_bounds__(64 * kDenseEvalFeatures) void reduce_evaluate_dense
   }
 }
 
-// Reduce and evaluate in one launch for dense levels whose partial slots are
-// feature-major ([16 features][bin_stride][g, h] per tile: hist_kernel's fmaj
-// flush, so a feature's words in a slot are contiguous), for narrower
-// matrices (fewer workgroups per job, nodes of many chunks).  One 256-thread
-// workgroup per (reduce job, feature); every lane holds bins 4l .. 4l + 3 of
-// the feature, as evaluate_features_kernel<4> does.  Wavefront w sums the
-// job's partial slots w, w + 4, ... of its lane's 64 contiguous bytes (or
-// wavefront 0 reads what the node's only chunk wrote), the sums meet in LDS,
-// and then wavefront 0 writes (with store) and evaluates the node while
-// wavefront 1 derives, writes and evaluates the sibling from the parent's
-// words -- the words and candidates of hist_reduce_kernel followed by
-// evaluate_features_kernel<4>, with one launch and one pass over the level's
-// histograms fewer.  Bins past bin_stride read the feature's last bin and are
+// The same for narrower matrices (fewer workgroups per job, nodes of many
+// chunks).  One 256-thread workgroup per (reduce job, feature); every lane holds
+// BPL bins of the feature as above.  Wavefront w sums the job's partial slots w,
+// w + 4, ... of its lane's contiguous bytes (or wavefront 0 reads what the node's
+// only chunk wrote), the sums meet in LDS, and then wavefront 0 writes (with
+// store) and evaluates the node while wavefront 1 derives, writes and evaluates
+// the sibling from the parent's words.  Bins past bin_stride read the feature's last bin and are
 // masked (branch-free loads).  W wavefronts per workgroup: 4, or 2 (the node
 // and the sibling only) when the launch has more workgroups than the chip holds
 // at once with four wavefronts each (the kernel's registers allow four
 // wavefronts per SIMD, 1,024 such workgroups on 256 CUs): two-wave workgroups
 // fit twice as many, and such levels have mostly one chunk per node (C2's last
 // split level: 12.0 -> 10.0 us; with fewer workgroups two waves measured slower).
-template <int W>
+template <int W, int BPL>
 __global__ __launch_bounds__(64 * W) void reduce_evaluate_dense_split_kernel(
     const long long* __restrict__ partial, const HistReduce* __restrict__ jobs,
     int32_t n_jobs_host, const int32_t* __restrict__ n_jobs_dev, int32_t n_tiles,
-    int32_t n_features, int32_t bin_stride, const long long* __restrict__ parent_base,
-    long long* __restrict__ hist, const int32_t* __restrict__ n_bins,
+    int32_t tile_features, int32_t n_features, int32_t bin_stride,
+    const long long* __restrict__ parent_base, long long* __restrict__ hist,
+    const int32_t* __restrict__ n_bins,
     const long long* __restrict__ node_sums, const int32_t* __restrict__ exps, Param p,
     const uint32_t* __restrict__ fmask, const uint8_t* __restrict__ skip_bins,
     FeatCand* __restrict__ cand, int32_t store) {
-  constexpr int BPL = 4;
   __shared__ long long part[W][2 * BPL][64];  // each wavefront's sums; [0] then the node's
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int32_t f = int32_t(blockIdx.x);
   const HistReduce j_first = int32_t(blockIdx.y) < n_jobs_host ? jobs[blockIdx.y] : HistReduce{};
   const int32_t n_jobs = n_jobs_dev ? *n_jobs_dev : n_jobs_host;
-  const int32_t tile = f >> 4, fl = f & 15;
-  const int64_t slot_words = int64_t(bin_stride) * 32;  // a tile's partial slot
+  const int32_t tile = f / tile_features, fl = f - tile * tile_features;
+  const int64_t slot_words = int64_t(bin_stride) * tile_features * 2;  // a tile's partial slot
   const int64_t node_elems = int64_t(n_features) * bin_stride * 2;
   bool ok[BPL];
   int64_t at[BPL], pat[BPL];  // word of bin (g; h is + 1): node histogram, partial slot
@@ -754,13 +751,11 @@ size_t evaluate_scratch_bytes(int32_t n_nodes, int32_t n_features) {
   return sizeof(FeatCand) * size_t(n_nodes > 0 ? n_nodes : 0) * size_t(n_features);
 }
 
-bool launch_evaluate(const int64_t* hist, int32_t n_nodes, const int32_t* n_nodes_dev,
-                     int32_t n_features, int32_t bin_stride, const int32_t* n_bins,
-                     const int64_t* node_sums, const int32_t* exps, int32_t exp_g, int32_t exp_h,
-                     const dp_train_param& param, void* scratch, dp_split_record* out,
-                     hipStream_t s, bool select, const uint32_t* fmask,
-                     const uint8_t* skip_bins) {
-  if (n_nodes <= 0) return true;
+void launch_evaluate(const int64_t* hist, int32_t n_nodes, int32_t n_features, int32_t bin_stride,
+                     const int32_t* n_bins, const int64_t* node_sums, int32_t exp_g,
+                     int32_t exp_h, const dp_train_param& param, void* scratch,
+                     dp_split_record* out, hipStream_t s) {
+  if (n_nodes <= 0) return;
   need(bin_stride >= 1 && bin_stride <= kMaxBins, "split bin stride out of range");
   need(n_features >= 1, "split evaluation needs at least one feature");
   Param p{double(param.lambda), double(param.alpha), double(param.min_child_weight),
@@ -770,50 +765,36 @@ bool launch_evaluate(const int64_t* hist, int32_t n_nodes, const int32_t* n_node
   if (n_features <= kNodeFeatures) {
     const dim3 grid(n_nodes < 2048 ? n_nodes : 2048), block(64 * kNodeWaves);
     if (bin_stride <= 64)
-      hipLaunchKernelGGL(evaluate_nodes_kernel<1>, grid, block, 0, s, h, n_nodes, n_nodes_dev,
-                         n_features, bin_stride, n_bins, sums, exps, exp_g, exp_h, p, fmask, skip_bins, out);
+      hipLaunchKernelGGL(evaluate_nodes_kernel<1>, grid, block, 0, s, h, n_nodes, nullptr,
+                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
     else if (bin_stride <= 128)
-      hipLaunchKernelGGL(evaluate_nodes_kernel<2>, grid, block, 0, s, h, n_nodes, n_nodes_dev,
-                         n_features, bin_stride, n_bins, sums, exps, exp_g, exp_h, p, fmask, skip_bins, out);
+      hipLaunchKernelGGL(evaluate_nodes_kernel<2>, grid, block, 0, s, h, n_nodes, nullptr,
+                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
     else
-      hipLaunchKernelGGL(evaluate_nodes_kernel<4>, grid, block, 0, s, h, n_nodes, n_nodes_dev,
-                         n_features, bin_stride, n_bins, sums, exps, exp_g, exp_h, p, fmask, skip_bins, out);
+      hipLaunchKernelGGL(evaluate_nodes_kernel<4>, grid, block, 0, s, h, n_nodes, nullptr,
+                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
     DP_HIP(hipGetLastError());
-    return true;
+    return;
   }
   auto* cand = static_cast<FeatCand*>(scratch);
   if (bin_stride <= 64) {
     const int64_t items = int64_t(n_nodes) * ((n_features + kSegFeatures - 1) / kSegFeatures);
     hipLaunchKernelGGL(evaluate_features_seg_kernel, dim3(items < 2048 ? items : 2048), dim3(256),
-                       0, s, h, n_nodes, n_nodes_dev, n_features, bin_stride, n_bins, sums, exps,
-                       exp_g, exp_h, p, fmask, skip_bins, cand);
-    DP_HIP(hipGetLastError());
-    if (!select) return false;
-    hipLaunchKernelGGL(select_splits_kernel, dim3(n_nodes < 1024 ? n_nodes : 1024),
-                       dim3(kSelectThreads), 0, s, cand, n_nodes, n_nodes_dev, n_features,
-                       double(param.gamma), out);
-    DP_HIP(hipGetLastError());
-    return true;
+                       0, s, h, n_nodes, nullptr, n_features, bin_stride, n_bins, sums, nullptr,
+                       exp_g, exp_h, p, nullptr, nullptr, cand);
+  } else {
+    const int64_t groups = (n_features + kFeatWaves - 1) / kFeatWaves;
+    const int64_t items = int64_t(n_nodes) * groups;
+    hipLaunchKernelGGL(bin_stride <= 128 ? evaluate_features_kernel<2> : evaluate_features_kernel<4>,
+                       dim3(int(items < 2048 ? items : 2048)), dim3(64 * kFeatWaves), 0, s, h,
+                       n_nodes, nullptr, n_features, bin_stride, n_bins, sums, nullptr, exp_g,
+                       exp_h, p, nullptr, nullptr, cand);
   }
-  const int64_t groups = (n_features + kFeatWaves - 1) / kFeatWaves;
-  const int64_t items = int64_t(n_nodes) * groups;
-  const int grid = int(items < 2048 ? items : 2048);
-  const dim3 block(64 * kFeatWaves);
-  if (bin_stride <= 128)
-    hipLaunchKernelGGL(evaluate_features_kernel<2>, dim3(grid), block, 0, s, h, n_nodes,
-                       n_nodes_dev, n_features, bin_stride, n_bins, sums, exps, exp_g, exp_h, p,
-                       fmask, skip_bins, cand);
-  else
-    hipLaunchKernelGGL(evaluate_features_kernel<4>, dim3(grid), block, 0, s, h, n_nodes,
-                       n_nodes_dev, n_features, bin_stride, n_bins, sums, exps, exp_g, exp_h, p,
-                       fmask, skip_bins, cand);
   DP_HIP(hipGetLastError());
-  if (!select) return false;
   hipLaunchKernelGGL(select_splits_kernel, dim3(n_nodes < 1024 ? n_nodes : 1024),
-                     dim3(kSelectThreads), 0, s, cand, n_nodes, n_nodes_dev, n_features,
+                     dim3(kSelectThreads), 0, s, cand, n_nodes, nullptr, n_features,
                      double(param.gamma), out);
   DP_HIP(hipGetLastError());
-  return true;
 }
 
 void launch_reduce_evaluate_flat(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
@@ -846,14 +827,16 @@ void launch_reduce_evaluate_flat(const int64_t* partial, const HistReduce* jobs,
 }
 
 void launch_reduce_evaluate_dense(const int64_t* partial, const HistReduce* jobs, int32_t n_jobs,
-                                  const int32_t* n_jobs_dev, int32_t n_tiles, int32_t n_features,
-                                  int32_t bin_stride, const int64_t* parent_base, int64_t* hist,
+                                  const int32_t* n_jobs_dev, int32_t n_tiles,
+                                  int32_t tile_features, int32_t n_features, int32_t bin_stride, const int64_t* parent_base, int64_t* hist,
                                   const int32_t* n_bins, const int64_t* node_sums,
                                   const int32_t* exps, const dp_train_param& param,
                                   const uint32_t* fmask, const uint8_t* skip_bins, void* scratch,
                                   bool store, hipStream_t s) {
   if (n_jobs <= 0 || n_features <= 0) return;
   need(bin_stride >= 1 && bin_stride <= 64 * 4, "dense reduce-evaluate needs at most 256 bins");
+  need(tile_features >= 1 && n_tiles == (n_features + tile_features - 1) / tile_features,
+       "tile count");
   need(exps && scratch && n_bins && node_sums,
        "reduce-evaluate needs the quantiser exponents, the bin counts and candidate scratch");
   Param p{double(param.lambda), double(param.alpha), double(param.min_child_weight),
@@ -867,12 +850,23 @@ void launch_reduce_evaluate_dense(const int64_t* partial, const HistReduce* jobs
   const dim3 grid(unsigned(wide ? (n_features + kDenseEvalFeatures - 1) / kDenseEvalFeatures
                                 : n_features),
                   unsigned(n_jobs < 256 ? n_jobs : 256));
-  hipLaunchKernelGGL(wide   ? reduce_evaluate_dense_kernel
-                     : many ? reduce_evaluate_dense_split_kernel<2>
-                            : reduce_evaluate_dense_split_kernel<4>,
-                     grid, dim3(many ? 128 : 256), 0, s,
+  // Bins per lane: the fewest that hold the feature in 64 lanes.
+  const auto kernel = [&] {
+    if (bin_stride <= 64)
+      return wide   ? reduce_evaluate_dense_kernel<1>
+             : many ? reduce_evaluate_dense_split_kernel<2, 1>
+                    : reduce_evaluate_dense_split_kernel<4, 1>;
+    if (bin_stride <= 128)
+      return wide   ? reduce_evaluate_dense_kernel<2>
+             : many ? reduce_evaluate_dense_split_kernel<2, 2>
+                    : reduce_evaluate_dense_split_kernel<4, 2>;
+    return wide   ? reduce_evaluate_dense_kernel<4>
+           : many ? reduce_evaluate_dense_split_kernel<2, 4>
+                  : reduce_evaluate_dense_split_kernel<4, 4>;
+  }();
+  hipLaunchKernelGGL(kernel, grid, dim3(many ? 128 : 256), 0, s,
                      reinterpret_cast<const long long*>(partial), jobs, n_jobs, n_jobs_dev,
-                     n_tiles, n_features, bin_stride,
+                     n_tiles, tile_features, n_features, bin_stride,
                      reinterpret_cast<const long long*>(parent_base),
                      reinterpret_cast<long long*>(hist), n_bins,
                      reinterpret_cast<const long long*>(node_sums), exps, p, fmask, skip_bins,

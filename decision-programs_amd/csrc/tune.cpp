@@ -128,8 +128,8 @@ double time_dense(const Pass& p, const HistConfig& cfg, hipStream_t s) {
         // sums are discarded, its time stands for the levels' reduce.
         launch_hist(p.bins, *p.L, p.gpair, p.ridx, dw.p, int32_t(w.size()), nullptr,
                     p.bin_stride, p.out, partial.p, s, p.rows_major, cfg, p.skip, p.fmaj);
-        launch_hist_reduce(partial.p, dj.p, p.nodes, nullptr, p.L->n_tiles, p.L->n_features,
-                           p.bin_stride, nullptr, p.out, false, s);
+        launch_hist_reduce(partial.p, dj.p, p.nodes, p.L->n_tiles, p.L->n_features,
+                           p.bin_stride, p.out, false, s);
       },
       s);
   DP_HIP(hipStreamSynchronize(s));  // before the buffers are freed
@@ -223,15 +223,14 @@ const HistTuning& tune_dense_hist(const dp_bin_layout& L, const uint8_t* bins, b
       }
       return it->second.p;
     };
-    // The levels' flush layout: feature-major where the booster fuses the
-    // reduce and the evaluation (it costs more per item than the LDS image).
-    const bool fmaj = L.n_features >= kDenseFuseFeatures && bin_stride <= 256;
+    // The levels' flush layout: feature-major, as the booster's reduce and
+    // evaluation read it (it costs more per item than the LDS image).
     report += ",";
     t.level = pick(
         dense_candidates(L.n_tiles, false),
         [&](const HistConfig& c) {
           Pass level{&L,  bins,   rows_for(c), skip, ridx.p, per, kNodes, bin_stride,
-                     gpair, out.p, fmaj};
+                     gpair, out.p, true};
           return time_dense(level, c, s);
         },
         report, "gathered", kTieShareGathered);
@@ -263,24 +262,22 @@ const HistTuning& tune_sparse_hist(const SparseBins& sp, int64_t n_rows, int32_t
   std::vector<HistConfig> cands;
   for (int32_t items : {512, 1024, 2048}) cands.push_back(HistConfig{1, 2, items});
   DeviceBuffer<int64_t> out(size_t(n_features) * size_t(bin_stride) * 2);
-  // The booster sums the root's partial slots in the launch that also
-  // evaluates them (reduce_evaluate_flat_kernel) whenever the bins allow it;
-  // its reduce runs one workgroup per 16 features, so its time grows with the
-  // slots far more than the reduce-only launch's.  The timed pass runs that
+  // The booster sums the root's partial slots in the launch that also evaluates
+  // them; with at most 64 bins its reduce runs one workgroup per 16 features
+  // (reduce_evaluate_flat_kernel), so its time grows with the slots far more than
+  // a reduce-only launch's.  The timed pass runs that
   // launch, with node sums of zero (every candidate is refused at once, the
   // same small evaluation for each candidate count).
   const bool fused = bin_stride <= 64 && sp.tile_features % 16 == 0;  // as the booster decides
-  DeviceBuffer<int32_t> nbins(fused ? size_t(n_features) : 0);
-  DeviceBuffer<int64_t> sums(fused ? 2 : 0);
-  DeviceBuffer<int32_t> exps(fused ? 2 : 0);
-  DeviceBuffer<FeatCand> feat(fused ? size_t(n_features) : 0);
-  std::vector<int32_t> nb;  // alive until the stream has read it (synchronised below)
-  if (fused) {
-    nb.assign(size_t(n_features), bin_stride);
-    DP_HIP(hipMemcpyAsync(nbins.p, nb.data(), nbins.bytes(), hipMemcpyHostToDevice, s));
-    DP_HIP(hipMemsetAsync(sums.p, 0, sums.bytes(), s));
-    DP_HIP(hipMemsetAsync(exps.p, 0, exps.bytes(), s));
-  }
+  DeviceBuffer<int32_t> nbins(static_cast<size_t>(n_features));
+  DeviceBuffer<int64_t> sums(2);
+  DeviceBuffer<int32_t> exps(2);
+  DeviceBuffer<FeatCand> feat(static_cast<size_t>(n_features));
+  // alive until the stream has read it (synchronised below)
+  const std::vector<int32_t> nb(static_cast<size_t>(n_features), bin_stride);
+  DP_HIP(hipMemcpyAsync(nbins.p, nb.data(), nbins.bytes(), hipMemcpyHostToDevice, s));
+  DP_HIP(hipMemsetAsync(sums.p, 0, sums.bytes(), s));
+  DP_HIP(hipMemsetAsync(exps.p, 0, exps.bytes(), s));
   const dp_train_param zero{};
   dp_bin_layout L{};
   L.n_rows = n_rows;
@@ -311,9 +308,10 @@ const HistTuning& tune_sparse_hist(const SparseBins& sp, int64_t n_rows, int32_t
                                             out.p, nbins.p, sums.p, exps.p, zero, nullptr,
                                             nullptr, feat.p, true, s);
               else
-                launch_hist_reduce_flat(partial.p, dj.p, 1, nullptr, sp.n_tiles,
-                                        sp.tile_features, n_features, bin_stride, nullptr, out.p,
-                                        s);
+                launch_reduce_evaluate_dense(partial.p, dj.p, 1, nullptr, sp.n_tiles,
+                                             sp.tile_features, n_features, bin_stride, nullptr,
+                                             out.p, nbins.p, sums.p, exps.p, zero, nullptr,
+                                             nullptr, feat.p, true, s);
             },
             s);
         DP_HIP(hipStreamSynchronize(s));
