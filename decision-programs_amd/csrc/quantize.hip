@@ -21,7 +21,9 @@ namespace {
 // A lane's feature is lane & 15: a load takes 4 rows' 64-byte runs.  Lane group
 // lane >> 4 owns kBinRows adjacent rows, whose searches run side by side; its
 // bytes are then adjacent in the column copy, and four lanes exchange theirs so
-// that each stores a 4-feature word of one row of the tile.  One workgroup takes
+// that each stores a 4-feature word of one row of the tile.  Packing the few
+// present values of mostly missing steps before the search, as the cut sketch
+// does, gained nothing here: the stores bound those.  One workgroup takes
 // a chunk of rows; those of one XCD take adjacent tiles of the same rows, which
 // share 128-byte lines.
 //
@@ -29,13 +31,13 @@ namespace {
 // 16 bytes per value with 65-256 bins, bound it.  The row-per-thread kernel it
 // replaced (16 strided loads, 8 binary steps of one word each) took 0.70 ms for
 // 1M x 100 and 12.9 ms for 2M x 1,000 with 95 % missing, and the column copy a
-// pass of its own (0.71 ms at the latter); now 0.20 and 4.6 ms, copy included.
+// pass of its own (0.71 ms at the latter); now 0.20 and 4.0 ms, copy included.
 constexpr int32_t kBinFeatures = 1 << 20;
 constexpr int kBinRows = 8;
 constexpr int kBinThreads = 256;
 
-struct __attribute__((packed)) PackedWords {
-  uint32_t w[kBinRows / 4];
+struct __attribute__((packed)) UnalignedWords {  // 8 bytes at any address
+  uint32_t w[2];
 };
 
 template <bool WIDE>
@@ -45,6 +47,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
     int32_t missing_bin, int32_t tiles, int32_t chunks, int64_t chunk_rows,
     uint8_t* __restrict__ bins, uint8_t* __restrict__ cols, uint16_t* __restrict__ cols16) {
   __shared__ uint4 tree[search_nodes(4) * kTile];
+  __shared__ uint2 s_cols[kTile][kBinThreads / 16 + 1];  // [feature][8 rows each]
   const int32_t per = (tiles * chunks + 7) / 8;
   const int32_t item = int32_t(blockIdx.x % 8) * per + int32_t(blockIdx.x / 8);
   if (int32_t(blockIdx.x / 8) >= per || item >= tiles * chunks) return;
@@ -72,7 +75,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
   // arithmetic, so all are in flight before the first wait.
   const uint32_t offset = (uint32_t((lane >> 4) * kBinRows) * uint32_t(n_features) +
                            uint32_t(min(f, n_features - 1))) * 4u;
-  for (int64_t w0 = chunk * chunk_rows + wave * kWaveRows; w0 < r1;
+  // Every wavefront takes part in each step (the columns' barriers), also past r1.
+  for (int64_t w0 = chunk * chunk_rows + wave * kWaveRows; w0 - wave * kWaveRows < r1;
        w0 += kBinThreads / 64 * kWaveRows) {
     const int64_t r0 = w0 + (lane >> 4) * kBinRows;
     const float* base = values + w0 * n_features;
@@ -118,19 +122,28 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
       const int64_t r = r0 + u + k;
       if (r < r1) *reinterpret_cast<uint32_t*>(tile + r * kTile + (j & ~3)) = v;
     }
-    if (!cols || !live) continue;
-    uint8_t* c = cols + int64_t(f) * n_rows + r0;
-    if (r0 + kBinRows <= r1) {
-      PackedWords w;
-#pragma unroll
-      for (int q = 0; q < kBinRows / 4; ++q)
-        w.w[q] = uint32_t(bin[4 * q]) | uint32_t(bin[4 * q + 1]) << 8 |
-                 uint32_t(bin[4 * q + 2]) << 16 | uint32_t(bin[4 * q + 3]) << 24;
-      *reinterpret_cast<PackedWords*>(c) = w;
-    } else {
-#pragma unroll
-      for (int u = 0; u < kBinRows; ++u)
-        if (r0 + u < r1) c[u] = uint8_t(bin[u]);
+    if (!cols) continue;
+    // The workgroup's 128 rows of a feature meet in LDS, so that the copy's columns
+    // are stored in 128-byte runs (a lane's own 8 rows: 32-byte runs per wavefront,
+    // half-written sectors; 2M x 1,000 4.6 ms against 4.0).
+    uint2 mine;
+    mine.x = uint32_t(bin[0]) | uint32_t(bin[1]) << 8 | uint32_t(bin[2]) << 16 | uint32_t(bin[3]) << 24;
+    mine.y = uint32_t(bin[4]) | uint32_t(bin[5]) << 8 | uint32_t(bin[6]) << 16 | uint32_t(bin[7]) << 24;
+    static_assert(kBinRows == 8, "a lane's rows of a column are 8 bytes");
+    __syncthreads();  // the last step's columns are stored
+    s_cols[j][wave * 4 + (lane >> 4)] = mine;
+    __syncthreads();
+    const int c = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;  // feature, 8 rows
+    const int64_t rc = w0 - wave * kWaveRows + part * kBinRows;
+    if (f0 + c < n_features && rc < r1) {
+      const uint2 v = s_cols[c][part];
+      uint8_t* to = cols + int64_t(f0 + c) * n_rows + rc;
+      if (rc + kBinRows <= r1) {
+        *reinterpret_cast<UnalignedWords*>(to) = {{v.x, v.y}};
+      } else {
+        for (int u = 0; u < int(r1 - rc); ++u)
+          to[u] = uint8_t((u < 4 ? v.x >> (8 * u) : v.y >> (8 * (u - 4))));
+      }
     }
   }
 }
