@@ -32,13 +32,14 @@
 // Two reads of the matrix and its binary searches bound it.  Sorting every
 // feature (a radix sort each) moved 8 to 10 times the bytes in 4 to 21 launches
 // per feature.  Device time before and now: 1M x 100, 20 % missing, 255 bins
-// 19.0 -> 0.84 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 8.4 ms; 1M x 28 4.2
+// 19.0 -> 0.84 ms; 2M x 1,000, 95 % missing, 64 bins 178 -> 5.0 ms; 1M x 28 4.2
 // -> 0.3 ms; 10k x 8 0.22 -> 0.06 ms.
 #include "dp_internal.hpp"
 #include "search.hpp"
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace dp {
 namespace {
@@ -52,10 +53,11 @@ __device__ __forceinline__ float end_cut(float v) { return v + (fabsf(v) + 1e-5f
 // levels (search.hpp) and as many counters.
 constexpr int kLevels = 5;
 constexpr int kBuckets = 1 << (2 * kLevels);
-constexpr size_t kBucketLds = sizeof(uint4) * search_nodes(kLevels) * kTile +
-                              sizeof(uint32_t) * kBuckets * kTile;
 constexpr int kSample = 8192;
 constexpr int kThreads = 1024;
+constexpr size_t kBucketLds = sizeof(uint4) * search_nodes(kLevels) * kTile +
+                              sizeof(uint32_t) * kBuckets * kTile +
+                              sizeof(PackedKey) * 64 * (kThreads / 64);
 // Rows up to which a feature is sorted whole in LDS (68 KiB padded): one
 // launch instead of six and a host read-back.
 constexpr int kSortRows = 16384;
@@ -249,14 +251,16 @@ struct FeaturePlan {
 // that repeats in the sample makes its bucket exactly that value.
 //   at most kBuckets / 2 - 1 distinct sample values: all of them;
 //   more: kBuckets - 1 evenly spaced ones.
-// used[f]: entries in use; many[f]: the sample alone has over max_bin values.
+// used[f]: entries in use; many[f]: the sample alone has over max_bin values;
+// valid[f]: present values of the sample.
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ values,
                                                           int64_t n_rows, int32_t n_features,
                                                           int32_t f_begin, int32_t f_count,
                                                           int32_t max_bin,
                                                           uint32_t* __restrict__ bounds,
                                                           int32_t* __restrict__ used,
-                                                          int32_t* __restrict__ many) {
+                                                          int32_t* __restrict__ many,
+                                                          int32_t* __restrict__ valid) {
   __shared__ uint32_t s[sort_words(kSample)];
   __shared__ uint32_t part[kThreads / 64];
   // 16 adjacent features (one 64-byte run of a row) on one XCD, whose L2 then
@@ -305,6 +309,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
   if (threadIdx.x == 0) {
     used[j] = int32_t(total) + 1;
     many[j] = distinct > uint32_t(max_bin) ? 1 : 0;
+    valid[j] = n;
   }
 }
 
@@ -316,14 +321,15 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 //   gather  slots holds each (chunk, bucket)'s offset in its segment and
 //           seg[tile][bucket][16] the segment's in the feature (kNanKey: not
 //           wanted); the keys go to out[plan.base + segment + offset].
-// Trees (85 KiB) and counters (64 KiB) leave one workgroup per CU.
+// Trees (85 KiB), counters (64 KiB) and the wavefronts' packed keys (8 KiB) leave
+// one workgroup per CU.
 constexpr int kRows = 8;
 template <bool GATHER>
 __global__ __launch_bounds__(kThreads) void bucket_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features, int32_t f_begin,
     int32_t f_end, int32_t tiles, int32_t chunks, int64_t chunk_rows,
-    const uint32_t* __restrict__ bounds,
-    const int32_t* __restrict__ used, uint32_t* __restrict__ slots,
+    const uint32_t* __restrict__ bounds, const int32_t* __restrict__ used,
+    const int32_t* __restrict__ valid, uint32_t* __restrict__ slots,
     const uint32_t* __restrict__ seg, const FeaturePlan* __restrict__ plans,
     uint32_t* __restrict__ out) {
   extern __shared__ uint4 tree[];  // [search_nodes(kLevels)][16]
@@ -348,15 +354,28 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
       s_count[e] = 0u;
     }
   }
-  int32_t widest = 1;
-  for (int k = 0; k < kTile && f_begin + tile * kTile + k < f_end; ++k)
+  int32_t widest = 1, features = 0, sampled = 0;
+  for (int k = 0; k < kTile && f_begin + tile * kTile + k < f_end; ++k) {
     widest = max(widest, used[tile * kTile + k]);
+    sampled += valid[tile * kTile + k];
+    ++features;
+  }
+  // Steps of few present values are worth looking for when at most a fifth are
+  // (a step of 512 values packs up to 64); looking costs dense tiles 6 %.
+  const bool few = int64_t(sampled) * 5 <= int64_t(features) * kSample;
   const int levels = search_levels(widest);
   search_fill(tree, levels, [&](int k, int p) {
     return f_begin + tile * kTile + k < f_end ? tb[p * kTile + k] : kNanKey;
   });
+  PackedKey* queue = reinterpret_cast<PackedKey*>(s_count + kBuckets * kTile) +
+                     int(threadIdx.x >> 6) * 64;
+  // Where the keys of each feature go.
+  __shared__ uint32_t* s_base[kTile];
   uint32_t* keys = nullptr;
-  if constexpr (GATHER) keys = live ? out + plans[tile * kTile + j].base : nullptr;
+  if constexpr (GATHER) {
+    keys = live ? out + plans[tile * kTile + j].base : nullptr;
+    if (threadIdx.x < kTile) s_base[threadIdx.x] = keys;
+  }
   __syncthreads();
   const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
   // Loads from wave-uniform bases and one 32-bit byte offset per lane: no branches
@@ -365,7 +384,15 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const uint32_t offset =
       (uint32_t(lane4) * uint32_t(n_features) + uint32_t(min(f, n_features - 1))) * 4u;
-  auto step = [&](const float* base, int64_t rows) {  // rows: of this step, 64 * kRows or fewer
+  auto add = [&](uint32_t key, int bucket, int k, uint32_t* to) {
+    uint32_t* c = &s_count[bucket * kTile + k];
+    if constexpr (GATHER) {
+      if (*c != kNanKey) to[atomicAdd(c, 1u)] = key;
+    } else {
+      atomicAdd(c, 1u);
+    }
+  };
+  auto step = [&](const float* base, int64_t rows, auto packed) {  // rows: of this step, or more
     float x[kRows];
     uint32_t key[kRows];
     int pos[kRows];
@@ -382,20 +409,28 @@ __global__ __launch_bounds__(kThreads) void bucket_kernel(
     }
 #pragma unroll
     for (int u = 0; u < kRows; ++u) key[u] = order_key(x[u]) | (live ? 0u : ~0u);
-    search<kRows>(tree, levels, j, key, pos);
-#pragma unroll
-    for (int u = 0; u < kRows; ++u) {
-      if (key[u] == kNanKey) continue;
-      uint32_t* c = &s_count[pos[u] * kTile + j];
-      if constexpr (GATHER) {
-        if (*c != kNanKey) keys[atomicAdd(c, 1u)] = key[u];
-      } else {
-        atomicAdd(c, 1u);
+    if constexpr (packed.value) {
+      const int present = present_keys<kRows>(key);
+      if (present <= 64) {
+        const PackedKey p = pack_keys<kRows>(key, j, queue);
+        const int k = int(p.at & (kTile - 1));
+        search<1>(tree, levels, k, &p.key, pos);
+        if ((int(threadIdx.x) & 63) < present) add(p.key, pos[0], k, GATHER ? s_base[k] : nullptr);
+        return;
       }
     }
+    search<kRows>(tree, levels, j, key, pos);
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      if (key[u] != kNanKey) add(key[u], pos[u], j, keys);
   };
-  for (int64_t r0 = chunk * chunk_rows; r0 < r1; r0 += 64 * kRows)
-    step(values + r0 * n_features, r1 - r0);
+  if (few) {
+    for (int64_t r0 = chunk * chunk_rows; r0 < r1; r0 += 64 * kRows)
+      step(values + r0 * n_features, r1 - r0, std::true_type{});
+  } else {
+    for (int64_t r0 = chunk * chunk_rows; r0 < r1; r0 += 64 * kRows)
+      step(values + r0 * n_features, r1 - r0, std::false_type{});
+  }
   if constexpr (!GATHER) {
     __syncthreads();
     for (int e = threadIdx.x; e < kBuckets * kTile; e += kThreads) slot[e] = s_count[e];
@@ -792,19 +827,19 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
       totals.reserve(table);
       seg.reserve(table);
       slots.reserve(table * size_t(chunks));
-      used.reserve(size_t(fc) * 2);
+      used.reserve(size_t(fc) * 3);
       rank_bucket.reserve(size_t(fc) * size_t(max_bin + 1));
       cand.reserve(size_t(fc) * size_t(max_bin + 1));
       plans.reserve(size_t(fc));
       gathered.reserve(1);
-      int32_t* many = used.p + fc;
+      int32_t *many = used.p + fc, *valid = many + fc;
       launch_fill_u8(reinterpret_cast<uint8_t*>(gathered.p), sizeof(unsigned long long), 0, s);
       hipLaunchKernelGGL(sample_kernel, dim3((fc + 127) / 128 * 128), dim3(kThreads), 0, s, values,
-                         n_rows, n_features, f0, fc, max_bin, bounds.p, used.p, many);
+                         n_rows, n_features, f0, fc, max_bin, bounds.p, used.p, many, valid);
       DP_HIP(hipGetLastError());
       const dim3 grid(unsigned((tiles * chunks + 7) / 8 * 8));
       hipLaunchKernelGGL(bucket_kernel<false>, grid, dim3(kThreads), kBucketLds, s, values, n_rows,
-                         n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, slots.p,
+                         n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, valid, slots.p,
                          nullptr, nullptr, nullptr);
       DP_HIP(hipGetLastError());
       hipLaunchKernelGGL(offsets_kernel, dim3(unsigned((table + 255) / 256)), dim3(256), 0, s,
@@ -822,7 +857,7 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
         while (cap < n_keys) cap += std::max<size_t>(1 << 16, cap / 8);
         if (keys.n < cap) keys.resize(cap);
         hipLaunchKernelGGL(bucket_kernel<true>, grid, dim3(kThreads), kBucketLds, s, values, n_rows,
-                           n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, slots.p,
+                           n_features, f0, f0 + fc, tiles, chunks, chunk_rows, bounds.p, used.p, valid, slots.p,
                            seg.p, plans.p, keys.p);
         DP_HIP(hipGetLastError());
       }
