@@ -13,17 +13,22 @@
 //     batch by batch.
 //   predict_trees_kernel  fewer rows than the chip has threads, wide rows, or
 //     large trees: R rows per workgroup, its other threads spread over the trees.
-//     Their leaf values meet in LDS, where one thread per row adds them in order.
+//     Their leaf values meet in LDS, where each of a row's threads adds those of
+//     one output in order.  (One thread per row adding all outputs' made its
+//     wavefront the last at every barrier, and the softmax went over global
+//     memory: whole calls of 60k x 784 x 500 trees 455 us against 284 now, 100k x
+//     400 x 160 trees 255 against 196, 9,000 x 600 x 200 trees 83 against 70.)
 //     Nodes come from global memory (a batch is walked by too few rows to be
 //     worth staging).
 //
 // One thread per row over global memory, the form these replaced, took 7,140 us
 // for 1M x 28 rows through 100 trees of depth 8, 2,700 us for 60k x 784 through
-// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 360, 410 and 12 us.
+// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 360, 240 and 12 us.
 // The first is bound by its vector instructions (11 per visit) and LDS reads (8
 // bytes of node from random banks, 4 of value), the second by the node loads of
 // its lanes, which rarely share a line.  Staging the second's nodes in LDS too
-// took 548 us: a batch has too few trees for a wide-row workgroup's lanes.
+// took 590 us a call, the next batch's loaded ahead into registers: beside 32 wide
+// rows a batch is 32 trees, one walk per lane, and a chain with a barrier at each.
 #include "predict.hpp"
 
 #include <algorithm>
@@ -215,9 +220,77 @@ __global__ __launch_bounds__(R) void predict_rows_kernel(
   sum.finish();
 }
 
+// m + leaves[0] + leaves[R] + ... in that order, n of them, with the LDS reads of
+// a block in flight before its additions.
+__device__ __forceinline__ float add_leaves(float m, const float* leaves, int32_t n, int R) {
+  constexpr int kBlock = 16;
+  float y[kBlock];
+  int32_t i = 0;
+  for (; i + kBlock <= n; i += kBlock) {
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) y[k] = leaves[(i + k) * R];
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) m += y[k];
+  }
+  if (i < n) {
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) y[k] = leaves[min(i + k, n - 1) * R];
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) m = i + k < n ? m + y[k] : m;
+  }
+  return m;
+}
+
+// The outputs of `rows` rows from their margins in LDS, part[row * stride + g], with
+// two places after them per row.  Every thread of the workgroup calls it.
+__device__ __forceinline__ void store_outputs(float* part, int stride, int rows, int32_t groups,
+                                              int32_t transform, float* out) {
+  __syncthreads();
+  if (transform == kPredArgmax) {
+    for (int q = threadIdx.x; q < rows; q += blockDim.x) {
+      RowOutput row{out + q, groups, transform, true};
+      for (int32_t g = 0; g < groups; ++g) row.margin(g, part[q * stride + g]);
+      row.finish();
+    }
+    return;
+  }
+  if (transform == kPredSoftmax) {
+    for (int q = threadIdx.x; q < rows; q += blockDim.x) {
+      float mx = -INFINITY;
+      for (int32_t g = 0; g < groups; ++g) mx = fmaxf(mx, part[q * stride + g]);
+      part[q * stride + groups] = mx;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < rows * groups; i += blockDim.x) {
+      float* p = part + i / groups * stride;
+      p[i % groups] = pred_expf(p[i % groups] - p[groups]);
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < rows; q += blockDim.x) {
+      float sum = 0.0f;
+      for (int32_t g = 0; g < groups; ++g) sum += part[q * stride + g];
+      part[q * stride + groups + 1] = sum;
+    }
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < rows * groups; i += blockDim.x) {
+    const float* p = part + i / groups * stride;
+    const float m = p[i % groups];
+    out[i] = transform == kPredSoftmax   ? m / p[groups + 1]
+             : transform == kPredSigmoid ? 1.0f / (1.0f + pred_expf(-m))
+                                         : m;
+  }
+}
+
 // R rows (a power of two) x blockDim.x / R tree lanes per workgroup.  STAGE: the
 // rows in LDS, x[row * (n_features | 1) + f] (coalesced loads; the odd stride
-// spreads the rows over the banks).
+// spreads the rows over the banks).  With at most kPredOutputs outputs a row's lanes
+// add up different outputs, whose margins meet in LDS; with more, its first lane
+// adds all and keeps them in global memory.
+constexpr int kPredOutputs = 64;
+__host__ __device__ constexpr int part_stride(int32_t groups) {  // odd: rows on different banks
+  return groups <= kPredOutputs ? (groups + 2) | 1 : 0;
+}
 template <class Node, bool STAGE>
 __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features, int64_t row_stride,
@@ -225,8 +298,10 @@ __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
     const int32_t* __restrict__ tree_ptr, const int32_t* __restrict__ tree_base,
     const int32_t* __restrict__ group_ptr, int32_t groups, int32_t trees, int32_t depth,
     const float* __restrict__ base, int32_t transform, int R, float* __restrict__ out) {
-  extern __shared__ float s_leaf[];  // [2][kWalk * blockDim.x], then the rows
-  float* x = s_leaf + 2 * kWalk * blockDim.x;
+  extern __shared__ float s_leaf[];  // [2][kWalk * blockDim.x], the margins, the rows
+  const int margins = part_stride(groups);
+  float* part = s_leaf + 2 * kWalk * blockDim.x;
+  float* x = part + R * margins;
   const int row = threadIdx.x & (R - 1), lane = int(threadIdx.x) / R, lanes = blockDim.x / R;
   const int64_t r0 = int64_t(blockIdx.x) * R, r = r0 + row;
   const int64_t rc = min(r, n_rows - 1);
@@ -250,7 +325,25 @@ __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
   }
   const int32_t outputs = transform == kPredArgmax ? 1 : groups;
   const float* v = values + rc * row_stride;
-  const bool adds = lane == 0 && r < n_rows;
+  const bool adds = margins == 0 && lane == 0 && r < n_rows;
+  // The output this lane adds up, its trees [a, b) and its margin so far.
+  int32_t g = lane, a = trees, b = trees;
+  float m = 0.0f;
+  auto open = [&] {
+    if (g >= groups) {
+      a = trees;
+      return;
+    }
+    a = group_ptr[g];
+    b = group_ptr[g + 1];
+    m = base[g];
+  };
+  auto close = [&] {
+    part[row * margins + g] = m;
+    g += lanes;
+    open();
+  };
+  if (margins) open();
   Margins sum(group_ptr, base, {out + rc * outputs, groups, transform, adds});
   const float* xr = x + row * stride;
   auto value = [&](int32_t f) { return STAGE ? xr[f] : or_nan(v[f], missing); };
@@ -288,17 +381,23 @@ __global__ __launch_bounds__(kPredThreads) void predict_trees_kernel(
       }
     }
     __syncthreads();  // the next round writes the other buffer
-    if (adds) {
-      const int32_t m = min(per_round, trees - t0);
-      for (int32_t i = 0; i < m; i += 8) {  // eight LDS reads in flight
-        float y[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) y[k] = leaves[min(i + k, m - 1) * R + row];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (i + k < m) sum.add(y[k]);
+    const int32_t end = min(t0 + per_round, trees);
+    if (margins) {
+      while (a < end) {
+        const int32_t lo = max(a, t0), hi = min(b, end);
+        m = add_leaves(m, leaves + (lo - t0) * R + row, hi - lo, R);
+        if (b > end) break;
+        close();
       }
+    } else if (adds) {
+      for (int32_t i = 0; i < end - t0; ++i) sum.add(leaves[i * R + row]);
     }
+  }
+  if (margins) {
+    while (g < groups) close();  // outputs without trees at the end
+    store_outputs(part, margins, int(min(int64_t(R), n_rows - r0)), groups, transform,
+                  out + r0 * outputs);
+    return;
   }
   if (adds) sum.finish();
 }
@@ -450,7 +549,9 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   // while another walks; all of it for rows too wide for that.
   bool stage = int64_t(forest.trees) * 128 >= n_features;
   auto lds_of = [&](int rows, int threads) {
-    return sizeof(float) * (2 * kWalk * size_t(threads) + size_t(rows) * size_t(n_features | 1));
+    return sizeof(float) * (2 * kWalk * size_t(threads) +
+                            size_t(rows) * size_t(part_stride(forest.groups) +
+                                                  (n_features | 1)));
   };
   int most = kPredThreads;
   if (stage) {
@@ -468,8 +569,8 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   int threads = 64;
   while (threads < most && threads < int64_t(forest.trees) * rows) threads *= 2;
   threads = std::max(threads, rows);
-  const size_t leaf_lds = sizeof(float) * 2 * kWalk * size_t(threads);
-  const size_t lds = leaf_lds + (stage ? sizeof(float) * size_t(rows) * size_t(n_features | 1) : 0);
+  const size_t lds =
+      lds_of(rows, threads) - (stage ? 0 : sizeof(float) * size_t(rows) * size_t(n_features | 1));
   const dim3 grid(unsigned((n_rows + rows - 1) / rows));
   auto run = [&](auto kernel, const auto* nodes) {
     allow_lds(reinterpret_cast<const void*>(kernel));

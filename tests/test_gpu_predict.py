@@ -29,13 +29,13 @@ def _forest(rng, trees, depth, features, full):
     return out
 
 
-def _model(forest, features, classes):
+def _model(forest, features, classes, objective=None):
     trees = [{"left_children": left.tolist(),
               "right_children": np.where(left < 0, -1, left + 1).tolist(),
               "split_indices": feature.tolist(),
               "split_conditions": [float(c) for c in cond], "default_left": default.tolist()}
              for left, feature, cond, default in forest]
-    objective = "reg:squarederror" if classes == 1 else "multi:softprob"
+    objective = objective or ("reg:squarederror" if classes == 1 else "multi:softprob")
     return json.dumps({"learner": {
         "gradient_booster": {"model": {
             "iteration_indptr": list(range(0, len(trees) + 1, classes)),
@@ -70,6 +70,8 @@ def _margins(forest, x, classes):
     (270001, 9, 37, 7, 0.97, 1),     # 1,024 rows, several batches
     (70000, 20, 5, 13, 1.0, 1),      # trees beyond a batch (16,383 nodes)
     (9000, 784, 120, 6, 1.0, 10),    # wide rows, nodes and rows in LDS
+    (700, 9, 3, 4, 1.0, 11),         # outputs spread over a row's lanes, several passes
+    (300, 12, 2, 3, 1.0, 65),        # more outputs than are spread
     (2000, 5000, 12, 7, 1.0, 1),     # rows too wide for many in LDS
     (40, 17000, 3, 4, 1.0, 1),       # features beyond the packed nodes
     (300, 7, 2, 17, 0.995, 1),       # trees beyond the packed nodes
@@ -97,3 +99,23 @@ def test_margins_match_a_numpy_walk(dp, device, rows, features, trees, depth, fu
     got = bst.predict(torch.as_tensor(y, device=device), margin=True, missing=-999.0)
     np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32),
                                   _margins(forest, x, classes).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,classes", [(1, 3), (2049, 10), (77, 64), (77, 65)])
+def test_outputs_of_the_margins(dp, device, rows, classes):
+    """Probabilities and class ids follow from the margins: each operation of the softmax rounds
+    once (2^-24), a sum of K positive terms at most K times, the exponential within 2 ulp."""
+    import torch
+
+    rng = np.random.default_rng(rows * classes)
+    forest = _forest(rng, 3 * classes, 4, 6, 0.9)
+    x = torch.as_tensor(rng.normal(size=(rows, 6)).astype(np.float32), device=device)
+    margins = _margins(forest, x.cpu().numpy(), classes)
+    p = np.exp(margins.astype(np.float64) - margins.max(axis=1, keepdims=True))
+    p /= p.sum(axis=1, keepdims=True)
+    bst = dp.Booster.from_buffer(_model(forest, 6, classes))
+    np.testing.assert_allclose(bst.predict(x).cpu().numpy().reshape(rows, classes), p,
+                               rtol=(classes + 8) * 2.0 ** -23)
+    bst = dp.Booster.from_buffer(_model(forest, 6, classes, "multi:softmax"))
+    np.testing.assert_array_equal(bst.predict(x).cpu().numpy().reshape(rows),
+                                  margins.argmax(axis=1).astype(np.float32))
