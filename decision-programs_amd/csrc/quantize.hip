@@ -168,6 +168,41 @@ __global__ void copy_matrix_kernel(const float* __restrict__ src, int64_t row_st
   if (__ballot(inf) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
+// The same for rows without gaps and 16-byte aligned: kCopyLoads 128-bit loads of a
+// thread in flight and no division of an element's place into row and feature.
+// Memory bounds it (8 B per value): 2M x 1,000 3.67 -> 3.05 ms (5.2 TB/s), 1M x 28
+// 57 -> 40 us.
+constexpr int kCopyLoads = 4;
+constexpr int kCopyThreads = 256;
+__global__ __launch_bounds__(kCopyThreads) void copy_flat_kernel(
+    const float4* __restrict__ src, int64_t n, float missing, float4* __restrict__ dst,
+    int32_t* __restrict__ bad) {
+  constexpr int64_t kStep = int64_t(kCopyLoads) * kCopyThreads;
+  const int64_t quads = (n + 3) / 4, whole = n / 4;
+  bool inf = false;
+  auto fix = [&](float x) {
+    inf = inf || isinf(x);
+    return x == missing ? __builtin_nanf("") : x;
+  };
+  for (int64_t q0 = int64_t(blockIdx.x) * kStep; q0 < quads; q0 += kStep * gridDim.x) {
+    float4 v[kCopyLoads];
+    const int64_t q = q0 + threadIdx.x;
+    if (q0 + kStep <= whole) {  // uniform
+#pragma unroll
+      for (int k = 0; k < kCopyLoads; ++k) v[k] = src[q + k * kCopyThreads];
+#pragma unroll
+      for (int k = 0; k < kCopyLoads; ++k)
+        dst[q + k * kCopyThreads] = make_float4(fix(v[k].x), fix(v[k].y), fix(v[k].z), fix(v[k].w));
+    } else {
+      const float* from = reinterpret_cast<const float*>(src);
+      float* to = reinterpret_cast<float*>(dst);
+      for (int64_t i = q0 * 4 + threadIdx.x; i < min(n, (q0 + kStep) * 4); i += kCopyThreads)
+        to[i] = fix(from[i]);
+    }
+  }
+  if (__ballot(inf) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
+}
+
 // Joint tiles of the paired tiles (dp_bin_layout::paired_tiles): joint tile
 // n_tiles + k, for the k-th pair (tiles t, t + 1; blockIdx.y = k), holds per
 // row and feature slot i the byte (tile t's bin << 4) | (tile t + 1's bin &
@@ -519,6 +554,15 @@ void launch_copy_matrix(const float* src, int64_t row_stride, int64_t n_rows, in
   launch_fill_u8(reinterpret_cast<uint8_t*>(bad), 4, 0, s);
   const int64_t total = n_rows * n_features;
   if (total <= 0) return;
+  if (row_stride == n_features && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(dst) % 16 == 0) {
+    const int64_t per = int64_t(kCopyLoads) * kCopyThreads * 4;
+    const int64_t blocks = std::min<int64_t>((total + per - 1) / per, 16384);
+    hipLaunchKernelGGL(copy_flat_kernel, dim3(unsigned(blocks)), dim3(kCopyThreads), 0, s, reinterpret_cast<const float4*>(src), total,
+                       missing, reinterpret_cast<float4*>(dst), bad);
+    DP_HIP(hipGetLastError());
+    return;
+  }
   hipLaunchKernelGGL(copy_matrix_kernel, dim3(grid_for(total, 256, 16384)), dim3(256), 0, s, src,
                      row_stride, n_rows, n_features, missing, dst, bad);
   DP_HIP(hipGetLastError());

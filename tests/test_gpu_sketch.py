@@ -55,3 +55,34 @@ def test_cuts_match_the_oracle(dp, oracle, ws, device, n, max_bin):
             np.testing.assert_array_equal(ops.from_tiles(bins.cpu().numpy(), lay),
                                           oracle.bin_matrix(part, o_ptr, o_cuts, 255))
         assert missing == bool(np.isnan(part).any())
+
+
+@pytest.mark.parametrize("rows,features", [(1, 1), (3, 5), (256, 16), (256, 17), (241, 1003)])
+def test_matrices_are_copied_whole(dp, device, rows, features):
+    """With at most 256 rows the cuts are the distinct values above the smallest: the copy is
+    checked value by value, from aligned rows (128-bit loads) and others; infinities are refused
+    wherever they stand."""
+    import torch
+
+    rng = np.random.default_rng(rows * features)
+    x = rng.normal(size=(rows, features)).astype(np.float32)
+    x[rng.random(x.shape) < 0.1] = -999.0
+    want = []
+    for f in range(features):
+        u = np.unique(x[:, f][x[:, f] != -999.0])
+        top = u[-1] if u.size else np.float32(0.0)
+        want.append(np.append(u[1:], top + (np.abs(top) + np.float32(1e-5))))
+    want = np.concatenate(want).astype(np.float32)
+    flat = torch.zeros(rows * features + 1, device=device)
+    views = [torch.empty((rows, features), device=device), flat[1:].view(rows, features)]
+    for v in views:
+        v.copy_(torch.as_tensor(x))
+        d = dp.DMatrix(v, torch.arange(rows, device=device).float(), missing=-999.0)
+        dp.Booster({"objective": "reg:squarederror", "tree_method": "hist", "device": "cuda:0",
+                    "max_depth": 1, "max_bin": 256}, [d]).update(d, 0)
+        np.testing.assert_array_equal(d.cuts(256)[1], want)
+        for at in {0, rows * features // 2, rows * features - 1}:
+            v[at // features, at % features] = float("inf")
+            with pytest.raises(Exception, match="inf"):
+                dp.DMatrix(v, missing=-999.0)
+            v.copy_(torch.as_tensor(x))
