@@ -422,13 +422,20 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
     total += t.nodes.size();
     packed = packed && t.nodes.size() <= (size_t(1) << 16);
     batched = batched && t.nodes.size() <= size_t(kPredBatchNodes);
-    std::vector<int32_t> level(t.nodes.size(), 0);  // children follow their parents
+    // Nodes that rows reach (children follow their parents; pruned models keep
+    // nodes that no parent names).  Packed, a pair of children has one order, its
+    // parent's: a pair that two parents name takes the general form.
+    std::vector<int32_t> level(t.nodes.size(), -1);
+    level[0] = 0;
     for (size_t i = 0; i < t.nodes.size(); ++i) {
       const PredNode& n = t.nodes[i];
-      if (n.left < 0) continue;
+      if (n.left < 0 || level[i] < 0) continue;
       packed = packed && !std::isnan(n.cond) && (n.flags & 1 || n.cond != -INFINITY);
-      level[size_t(n.left)] = level[size_t(n.left) + 1] = level[i] + 1;
-      out.depth = std::max(out.depth, level[i] + 1);
+      for (size_t c = size_t(n.left); c <= size_t(n.left) + 1; ++c) {
+        packed = packed && level[c] < 0;
+        level[c] = std::max(level[c], level[i] + 1);
+        out.depth = std::max(out.depth, level[c]);
+      }
     }
   }
   need(total < size_t(INT32_MAX), "forest has too many nodes");
@@ -449,9 +456,12 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
       if (!packed) general.insert(general.end(), t->nodes.begin(), t->nodes.end());
       if (packed) {
         // Node i's place: children that missing values enter on the right swap.
-        std::vector<int32_t> place(static_cast<size_t>(size), 0);
-        for (const PredNode& nd : t->nodes) {
-          if (nd.left < 0) continue;
+        // -1: no row reaches it.
+        std::vector<int32_t> place(static_cast<size_t>(size), -1);
+        place[0] = 0;
+        for (int32_t i = 0; i < size; ++i) {
+          const PredNode& nd = t->nodes[size_t(i)];
+          if (nd.left < 0 || place[size_t(i)] < 0) continue;
           const int32_t second = nd.flags & 1 ? 1 : 0;  // the right child's place in the pair
           place[size_t(nd.left)] = nd.left + 1 - second;
           place[size_t(nd.left) + 1] = nd.left + second;
@@ -460,6 +470,7 @@ void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>
         leaves.resize(small.size());
         const uint32_t at = uint32_t(n - batch);
         for (int32_t i = 0; i < size; ++i) {
+          if (place[size_t(i)] < 0) continue;
           const PredNode& nd = t->nodes[size_t(i)];
           PackedNode& out_node = small[size_t(n + place[size_t(i)])];
           leaves[size_t(n + place[size_t(i)])] = nd.left < 0 ? nd.cond : 0.0f;

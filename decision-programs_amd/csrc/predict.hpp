@@ -34,8 +34,8 @@ struct PredNode {
 //                   -x >= cond exactly when x < t
 //   leaf            its own index, cond NaN: every row stays; its value is in
 //                   Forest::leaf_values
-// Forests of at most 16,384 features, 65,536 nodes a tree and no threshold that
-// would make a NaN take it.
+// Forests of at most 16,384 features, 65,536 nodes a tree, one parent for each
+// node that rows reach and no threshold that would make a NaN take it.
 struct alignas(8) PackedNode {
   float cond;
   uint32_t word;

@@ -119,3 +119,46 @@ def test_outputs_of_the_margins(dp, device, rows, classes):
     bst = dp.Booster.from_buffer(_model(forest, 6, classes, "multi:softmax"))
     np.testing.assert_array_equal(bst.predict(x).cpu().numpy().reshape(rows),
                                   margins.argmax(axis=1).astype(np.float32))
+
+
+def _pruned(forest, rng):
+    """A fifth of the inner nodes become leaves: the nodes below them stay, unreached."""
+    out = []
+    for left, feature, cond, default in forest:
+        cut = (left >= 0) & (rng.random(len(left)) < 0.2)
+        out.append((np.where(cut, -1, left), np.where(cut, 0, feature), cond,
+                    np.where(cut, 0, default)))
+    return out
+
+
+def _shared(forest):
+    """In each tree two inner nodes name one pair, missing values going opposite ways."""
+    out = []
+    for left, feature, cond, default in forest:
+        left, default = left.copy(), default.copy()
+        a, b = np.flatnonzero(left >= 0)[1:3]
+        left[a] = left[b]
+        default[a], default[b] = 0, 1
+        out.append((left, feature, cond, default))
+    return out
+
+
+@pytest.mark.parametrize("rows,trees", [(300, 30), (70001, 30), (1000, 1)])
+@pytest.mark.parametrize("shape", ["pruned", "shared"])
+def test_nodes_without_or_with_two_parents(dp, device, rows, trees, shape):
+    """Pruned models keep nodes that no parent names; nothing forbids two parents of a pair."""
+    import torch
+
+    rng = np.random.default_rng(rows + trees)
+    forest = _forest(rng, trees, 5, 9, 1.0)
+    forest = _pruned(forest, rng) if shape == "pruned" else _shared(forest)
+    # a root leaf before two unreached leaves, and before an unreached inner node
+    for tail in ([-1, -1, -1], [-1, 2, -1, -1]) if shape == "pruned" else ():
+        n = len(tail)
+        forest.append((np.array(tail), np.zeros(n, dtype=np.int64),
+                       np.arange(n, dtype=np.float32) + 10, np.zeros(n, dtype=np.int64)))
+    bst = dp.Booster.from_buffer(_model(forest, 9, 1))
+    x = rng.normal(size=(rows, 9)).astype(np.float32)
+    x[rng.random(x.shape) < 0.2] = np.nan
+    got = bst.predict(torch.as_tensor(x, device=device), margin=True).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), _margins(forest, x, 1).view(np.uint32))
