@@ -180,9 +180,10 @@ __global__ __launch_bounds__(kCopyThreads) void copy_flat_kernel(
   constexpr int64_t kStep = int64_t(kCopyLoads) * kCopyThreads;
   const int64_t quads = (n + 3) / 4, whole = n / 4;
   bool inf = false;
-  auto fix = [&](float x) {
+  auto fix = [&](float x) {  // the value that stands for missing may be an infinity
+    x = x == missing ? __builtin_nanf("") : x;
     inf = inf || isinf(x);
-    return x == missing ? __builtin_nanf("") : x;
+    return x;
   };
   for (int64_t q0 = int64_t(blockIdx.x) * kStep; q0 < quads; q0 += kStep * gridDim.x) {
     float4 v[kCopyLoads];

@@ -58,18 +58,21 @@ def test_cuts_match_the_oracle(dp, oracle, ws, device, n, max_bin):
 
 
 @pytest.mark.parametrize("rows,features", [(1, 1), (3, 5), (256, 16), (256, 17), (241, 1003)])
-def test_matrices_are_copied_whole(dp, device, rows, features):
+@pytest.mark.parametrize("missing", [-999.0, np.inf, -np.inf])
+def test_matrices_are_copied_whole(dp, device, rows, features, missing):
     """With at most 256 rows the cuts are the distinct values above the smallest: the copy is
-    checked value by value, from aligned rows (128-bit loads) and others; infinities are refused
-    wherever they stand."""
+    checked value by value, from aligned rows (128-bit loads) and others; infinities other than
+    the value that stands for missing are refused wherever they stand."""
     import torch
 
+    missing = np.float32(missing)
+    refused = -np.inf if missing > 0 else np.inf
     rng = np.random.default_rng(rows * features)
     x = rng.normal(size=(rows, features)).astype(np.float32)
-    x[rng.random(x.shape) < 0.1] = -999.0
+    x[rng.random(x.shape) < 0.1] = missing
     want = []
     for f in range(features):
-        u = np.unique(x[:, f][x[:, f] != -999.0])
+        u = np.unique(x[:, f][x[:, f] != missing])
         top = u[-1] if u.size else np.float32(0.0)
         want.append(np.append(u[1:], top + (np.abs(top) + np.float32(1e-5))))
     want = np.concatenate(want).astype(np.float32)
@@ -77,12 +80,12 @@ def test_matrices_are_copied_whole(dp, device, rows, features):
     views = [torch.empty((rows, features), device=device), flat[1:].view(rows, features)]
     for v in views:
         v.copy_(torch.as_tensor(x))
-        d = dp.DMatrix(v, torch.arange(rows, device=device).float(), missing=-999.0)
+        d = dp.DMatrix(v, torch.arange(rows, device=device).float(), missing=float(missing))
         dp.Booster({"objective": "reg:squarederror", "tree_method": "hist", "device": "cuda:0",
                     "max_depth": 1, "max_bin": 256}, [d]).update(d, 0)
         np.testing.assert_array_equal(d.cuts(256)[1], want)
         for at in {0, rows * features // 2, rows * features - 1}:
-            v[at // features, at % features] = float("inf")
+            v[at // features, at % features] = refused
             with pytest.raises(Exception, match="inf"):
-                dp.DMatrix(v, missing=-999.0)
+                dp.DMatrix(v, missing=float(missing))
             v.copy_(torch.as_tensor(x))
