@@ -1553,7 +1553,9 @@ void Booster::upload_forest(int32_t tree_begin, int32_t tree_end) {
     const float b = base_score_.empty() ? 0.0f : base_score_[k < base_score_.size() ? k : 0];
     base[k] = objective_id_ == DP_OBJ_LOGISTIC ? float(std::log(double(b) / (1.0 - double(b)))) : b;
   }
-  build_forest(trees, base, n_features_, forest_);
+  Forest forest;  // forest_ stays that of its range if this one finds no memory
+  build_forest(trees, base, n_features_, forest);
+  forest_ = std::move(forest);
   forest_begin_ = tree_begin;
   forest_end_ = tree_end;
   forest_trees_ = trees_.size();

@@ -1,0 +1,103 @@
+"""Who owns which device memory when, without a GPU: the library runs on a HIP runtime in host
+memory (tests/native/fake_hip.cpp), in a process of its own, whose kernels do nothing."""
+import json
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes, json, sys
+fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL({lib!r})
+lib.XGBGetLastError.restype = fake.fake_launches.restype = ctypes.c_char_p
+fake.fake_live_bytes.restype = fake.fake_arg.restype = ctypes.c_uint64
+fake.fake_synchronised.restype = ctypes.c_long
+fake.fake_fail_after.argtypes = [ctypes.c_long]
+
+def ok(status):
+    assert status == 0, lib.XGBGetLastError().decode()
+
+def device_array(shape, strides=None, device=0):
+    ok(fake.hipSetDevice(device))
+    n, p = 4, ctypes.c_void_p()
+    for d in shape:
+        n *= d
+    ok(fake.hipMalloc(ctypes.byref(p), ctypes.c_size_t(n)))
+    return json.dumps(dict(data=[p.value, True], shape=list(shape), strides=strides,
+                           typestr="<f4", version=3, stream=1)).encode()
+
+def matrix(rows, features, device=0):
+    h = ctypes.c_void_p()
+    a = device_array((rows, features), device=device)
+    ok(lib.XGDMatrixCreateFromCudaArrayInterface(a, b'{{"missing": NaN}}', ctypes.byref(h)))
+    return h
+"""
+
+
+@pytest.fixture(scope="session")
+def host(dp, tmp_path_factory):
+    """Runs code (after PRELUDE) on the host-memory runtime; returns what it printed as JSON."""
+    fake = str(tmp_path_factory.mktemp("hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-o", fake,
+                    os.path.join(HERE, "native", "fake_hip.cpp")], check=True)
+
+    def run(code):
+        text = PRELUDE.format(fake=fake, lib=dp.LIB_PATH) + textwrap.dedent(code)
+        p = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True,
+                           timeout=120)
+        assert p.returncode == 0, p.stderr
+        return json.loads(p.stdout)
+
+    return run
+
+
+def _model(trees, splits):
+    """Chains of `splits` splits: 2 * splits + 1 nodes a tree, one tree a round."""
+    n = 2 * splits + 1
+    left = [i + 1 if i % 2 == 0 and i < 2 * splits else -1 for i in range(n)]
+    tree = {"left_children": left, "right_children": [c + 1 if c > 0 else -1 for c in left],
+            "split_indices": [0] * n, "split_conditions": [0.5] * n, "default_left": [1] * n}
+    return json.dumps({"learner": {
+        "gradient_booster": {"model": {"iteration_indptr": list(range(trees + 1)),
+                                       "tree_info": [0] * trees, "trees": [tree] * trees}},
+        "learner_model_param": {"base_score": "[0]", "num_class": "0", "num_feature": "3"},
+        "objective": {"name": "reg:squarederror"}}})
+
+
+def test_a_failed_upload_leaves_the_last_forest(host):
+    """A prediction whose forest finds no memory fails; the next one of the range before must
+    not launch on what the failure left."""
+    out = host(f"""
+        text = {_model(40, 30)!r}.encode()
+        b = ctypes.c_void_p()
+        ok(lib.XGBoosterCreate(None, 0, ctypes.byref(b)))
+        ok(lib.XGBoosterLoadModelFromBuffer(b, text, ctypes.c_uint64(len(text))))
+        x = device_array((50, 3))
+        shape, dim, res = ctypes.c_void_p(), ctypes.c_uint64(), ctypes.c_void_p()
+        def predict(end):
+            cfg = json.dumps(dict(type=1, training=False, iteration_begin=0, iteration_end=end,
+                                  strict_shape=True, cache_id=0, missing=float("nan"))).encode()
+            return lib.XGBoosterPredictFromCudaArray(b, x, cfg, None, ctypes.byref(shape),
+                                                     ctypes.byref(dim), ctypes.byref(res))
+        seen = []
+        for fail in range(1, 12):  # the allocations that the larger forest is given
+            ok(predict(2))
+            before = [fake.fake_arg(i) for i in (5, 6)]
+            fake.fake_fail_after(fail - 1)
+            failed = predict(40)
+            fake.fake_fail_after(-1)
+            fake.fake_forget_launches()
+            ok(predict(2))
+            seen.append([failed, before, [fake.fake_arg(i) for i in (5, 6)]])
+        print(json.dumps(seen))
+    """)
+    assert out[0][0] != 0  # without any allocation it cannot succeed
+    for failed, before, after in out:
+        assert all(before) and all(after)
+        if failed:
+            assert after == before
