@@ -21,6 +21,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <limits>
+#include <set>
 
 #include "json.hpp"
 #include "tune.hpp"
@@ -770,7 +771,14 @@ void DMatrix::release_pending() {
     }
   }
   pending.clear();
-  (void)hipDeviceSynchronize();
+  std::set<int> devices{values.dev, labels.dev};
+  for (const auto& q : quantized) devices.insert(q.second->d_nbins.dev);
+  for (int device : devices) {
+    try {
+      synchronize_device(device);
+    } catch (...) {  // freed regardless
+    }
+  }
 }
 
 Booster::~Booster() {

@@ -70,7 +70,7 @@ struct DMatrix {
   std::map<int32_t, std::unique_ptr<Quantized>> quantized;  // by requested max_bin
   Quantized& quantize(int32_t max_bin, hipStream_t s);
   // Boosters with a round in flight on this matrix.  Freeing the matrix
-  // collects those rounds first (release_pending) and waits for the device.
+  // collects those rounds first (release_pending) and waits for its devices.
   std::vector<const Booster*> pending;
   void release_pending();
 };

@@ -257,7 +257,7 @@ int XGDMatrixSetInfoFromInterface(DMatrixHandle handle, const char* field, const
     dp::DMatrix& m = dm(handle);
     dp::need(field && std::string(field) == "label", "only the label field is supported");
     ArrayInterface a = parse_array(data);
-    if (m.labels.p) DP_HIP(hipDeviceSynchronize());  // rounds in flight may read the old labels
+    if (m.labels.p) dp::synchronize_device(m.labels.dev);  // rounds in flight may read the old ones
     m.labels.resize(size_t(m.n_rows));
     copy_float_array(a, m.n_rows, 1, m.labels.p);
     m.has_labels = true;

@@ -163,4 +163,12 @@ void pinned_pool_put(void* p, size_t bytes) {
   give(pinned_cache(), -1, p, rounded(bytes), true);
 }
 
+void synchronize_device(int device) {
+  const int now = current_device();
+  if (device != now) DP_HIP(hipSetDevice(device));
+  const hipError_t status = hipDeviceSynchronize();
+  if (device != now) DP_HIP(hipSetDevice(now));
+  DP_HIP(status);
+}
+
 }  // namespace dp

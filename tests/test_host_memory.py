@@ -101,3 +101,25 @@ def test_a_failed_upload_leaves_the_last_forest(host):
         assert all(before) and all(after)
         if failed:
             assert after == before
+
+
+def test_a_matrix_waits_for_its_own_device(host):
+    """Its blocks go back to the pool of the device they are on: that device must be idle, not
+    the one that happens to be current."""
+    out = host("""
+        h = matrix(100, 5, device=1)
+        ok(lib.XGDMatrixSetInfoFromInterface(h, b"label", device_array((100,), device=1)))
+        label = device_array((100,), device=1)
+        ok(fake.hipSetDevice(0))
+        counts = [fake.fake_synchronised(1)]
+        ok(lib.XGDMatrixSetInfoFromInterface(h, b"label", label))  # the old labels are given back
+        counts.append(fake.fake_synchronised(1))
+        ok(lib.XGDMatrixFree(h))
+        counts.append(fake.fake_synchronised(1))
+        now = ctypes.c_int()
+        ok(fake.hipGetDevice(ctypes.byref(now)))
+        print(json.dumps([counts, now.value]))
+    """)
+    (start, labels, freed), device = out
+    assert start < labels < freed
+    assert device == 0
