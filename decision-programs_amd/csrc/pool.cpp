@@ -2,10 +2,11 @@
 //
 // Blocks are kept by (device, size), sizes rounded up to 256 bytes and above 1
 // MiB to a sixteenth of their power of two, so that buffers whose size follows
-// the data (present values, gathered keys) meet the next matrix's.  At most
-// kCachedBytes per kind stay cached: a block that would exceed it first evicts
-// the blocks handed back longest ago, and blocks above kLargestBlock are never
-// cached.  So a process that trains many models, also on new data of the same
+// the data (present values, gathered keys) meet the next matrix's.  Each kind has
+// its limits: a block that would exceed the total, over all devices, first evicts
+// the blocks handed back longest ago, and larger blocks than the largest are never
+// cached.  Pinned host memory, which the whole machine shares, keeps little: it
+// holds readbacks and staged tables of at most some MB.  So a process that trains many models, also on new data of the same
 // kind, reuses the same blocks.  A fit of 2M x 1,000 values takes 14 GB, which the
 // driver maps and clears anew each time: back-to-back fits 30 ms without the
 // cache for matrices, 25 with it; between other large allocations 248 and 25.
@@ -21,9 +22,6 @@
 namespace dp {
 namespace {
 
-constexpr size_t kCachedBytes = size_t(24) << 30;
-constexpr size_t kLargestBlock = size_t(12) << 30;
-
 struct Block {
   void* p;
   int dev;
@@ -31,21 +29,23 @@ struct Block {
 };
 
 struct Cache {
+  const size_t total, largest;  // bytes kept, and of one block
   std::mutex m;
   // Blocks by when they were handed back, and their places by device and size.
   std::map<uint64_t, Block> blocks;
   std::map<std::pair<int, size_t>, std::vector<uint64_t>> by_size;
   uint64_t clock = 0;
   size_t cached = 0;
+  Cache(size_t t, size_t l) : total(t), largest(l) {}
 };
 
 Cache& device_cache() {
-  static Cache* c = new Cache();  // never destroyed
+  static Cache* c = new Cache(size_t(24) << 30, size_t(12) << 30);  // never destroyed
   return *c;
 }
 
 Cache& pinned_cache() {
-  static Cache* c = new Cache();  // never destroyed
+  static Cache* c = new Cache(size_t(2) << 30, size_t(512) << 20);  // never destroyed
   return *c;
 }
 
@@ -107,8 +107,8 @@ void give(Cache& c, int dev, void* p, size_t bytes, bool pinned) {
   std::vector<void*> out;  // freed outside the lock: the driver may wait for the device
   {
     std::lock_guard<std::mutex> lock(c.m);
-    if (bytes <= kLargestBlock) {
-      while (c.cached + bytes > kCachedBytes) {
+    if (bytes <= c.largest) {
+      while (c.cached + bytes > c.total) {
         const auto oldest = c.blocks.begin();
         out.push_back(oldest->second.p);
         forget(c, oldest->first, oldest->second);

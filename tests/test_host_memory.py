@@ -123,3 +123,38 @@ def test_a_matrix_waits_for_its_own_device(host):
     (start, labels, freed), device = out
     assert start < labels < freed
     assert device == 0
+
+
+POOL = """
+lib._ZN2dp15device_pool_getEmPi.restype = lib._ZN2dp15pinned_pool_getEm.restype = ctypes.c_void_p
+dev = ctypes.c_int()
+def get(n, pinned=False):
+    if pinned:
+        return lib._ZN2dp15pinned_pool_getEm(ctypes.c_size_t(n))
+    return lib._ZN2dp15device_pool_getEmPi(ctypes.c_size_t(n), ctypes.byref(dev))
+def put(p, n, pinned=False):
+    if pinned:
+        lib._ZN2dp15pinned_pool_putEPvm(ctypes.c_void_p(p), ctypes.c_size_t(n))
+    else:
+        lib._ZN2dp15device_pool_putEPvmi(ctypes.c_void_p(p), ctypes.c_size_t(n), dev)
+MB = 1 << 20
+"""
+
+
+@pytest.mark.parametrize("pinned,total,largest", [(False, 24 << 30, 12 << 30),
+                                                  (True, 2 << 30, 512 << 20)])
+def test_what_the_pool_keeps_is_bounded(host, pinned, total, largest):
+    """Device memory up to 24 GiB; host memory, which is never much, far less."""
+    out = host(POOL + f"""
+kind, pinned = ({-1 if pinned else 0}, {pinned})
+live = []
+for block in ({total // 64}, {largest}, {largest} + MB):
+    held = [get(block, pinned) for _ in range(70)] if block < MB * 512 else [get(block, pinned)]
+    for p in held: put(p, block, pinned)
+    live.append(fake.fake_live_bytes(kind))
+print(json.dumps(live))
+""")
+    many, one, larger = out
+    assert many == total  # 64 of 70 blocks stay
+    assert one == total   # the largest evicts as much as it brings
+    assert larger <= total  # a larger one is never kept
