@@ -49,10 +49,12 @@ Cache& pinned_cache() {
   return *c;
 }
 
-size_t rounded(size_t bytes) {
-  size_t unit = 256;
-  if (bytes > (size_t(1) << 20)) unit = (size_t(1) << (63 - __builtin_clzll(bytes))) / 16;
-  return (bytes + unit - 1) / unit * unit;
+// Blocks that are never cached get what they ask for: a sixteenth of a matrix of
+// 100 GiB is more than the device may have left.
+size_t rounded(const Cache& c, size_t bytes) {
+  auto up = [&](size_t unit) { return (bytes + unit - 1) / unit * unit; };
+  if (bytes <= (size_t(1) << 20) || bytes > c.largest) return up(256);
+  return up((size_t(1) << (63 - __builtin_clzll(bytes))) / 16);
 }
 
 int current_device() {
@@ -128,7 +130,7 @@ void give(Cache& c, int dev, void* p, size_t bytes, bool pinned) {
 }  // namespace
 
 void* device_pool_get(size_t bytes, int* device) {
-  bytes = rounded(bytes);
+  bytes = rounded(device_cache(), bytes);
   const int dev = current_device();
   *device = dev;
   if (void* p = take(device_cache(), dev, bytes)) return p;
@@ -143,11 +145,11 @@ void* device_pool_get(size_t bytes, int* device) {
 
 void device_pool_put(void* p, size_t bytes, int device) {
   if (!p) return;
-  give(device_cache(), device, p, rounded(bytes), false);
+  give(device_cache(), device, p, rounded(device_cache(), bytes), false);
 }
 
 void* pinned_pool_get(size_t bytes) {
-  bytes = rounded(bytes);
+  bytes = rounded(pinned_cache(), bytes);
   if (void* p = take(pinned_cache(), -1, bytes)) return p;
   void* p = nullptr;
   if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
@@ -160,7 +162,7 @@ void* pinned_pool_get(size_t bytes) {
 
 void pinned_pool_put(void* p, size_t bytes) {
   if (!p) return;
-  give(pinned_cache(), -1, p, rounded(bytes), true);
+  give(pinned_cache(), -1, p, rounded(pinned_cache(), bytes), true);
 }
 
 void synchronize_device(int device) {

@@ -158,3 +158,16 @@ print(json.dumps(live))
     assert many == total  # 64 of 70 blocks stay
     assert one == total   # the largest evicts as much as it brings
     assert larger <= total  # a larger one is never kept
+
+
+@pytest.mark.parametrize("size", [1, 256, 257, 1 << 20, (1 << 20) + 1, (9 << 30) + 1, 12 << 30,
+                                  (12 << 30) + 1, (17 << 30) + 255])
+def test_blocks_that_are_not_kept_are_not_rounded_up(host, size):
+    """Kept blocks come in sizes that later ones can share, at most a sixteenth larger; a block
+    too large to be kept takes 256-byte units, as the driver's own allocations do."""
+    got = host(POOL + f"""
+p = get({size})
+print(json.dumps(fake.fake_live_bytes(0)))
+""")
+    assert size <= got and got % 256 == 0
+    assert got <= (size + 255 if size <= 1 << 20 or size > 12 << 30 else size * 17 // 16)
