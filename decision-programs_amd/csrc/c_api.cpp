@@ -514,6 +514,10 @@ int DPDMatrixGetCuts(DMatrixHandle handle, int32_t max_bin, int32_t* cut_ptr, fl
   });
 }
 
+int DPReleaseCachedMemory(void) {
+  return guarded([&] { dp::release_pools(); });
+}
+
 // ===========================================================================
 // Kernel-level operator API
 // ===========================================================================

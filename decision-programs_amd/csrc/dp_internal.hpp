@@ -40,6 +40,8 @@ void* device_pool_get(size_t bytes, int* device);
 void device_pool_put(void* p, size_t bytes, int device);
 void* pinned_pool_get(size_t bytes);
 void pinned_pool_put(void* p, size_t bytes);
+// Hands every cached block back to the driver.
+void release_pools();
 // Waits for everything queued on `device`, whichever is current: before buffers
 // that launches of unknown streams may still read go back to the pool.
 void synchronize_device(int device);

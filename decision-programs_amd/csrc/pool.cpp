@@ -10,8 +10,8 @@
 // kind, reuses the same blocks.  A fit of 2M x 1,000 values takes 14 GB, which the
 // driver maps and clears anew each time: back-to-back fits 30 ms without the
 // cache for matrices, 25 with it; between other large allocations 248 and 25.
-// The cache lives until the process ends (no destructor runs at exit, when
-// the runtime may already be gone).
+// DPReleaseCachedMemory hands all of it back; what is left lives until the process
+// ends (no destructor runs at exit, when the runtime may already be gone).
 #include <map>
 #include <mutex>
 #include <utility>
@@ -87,13 +87,14 @@ void free_block(void* p, bool pinned) {
   else (void)hipFree(p);
 }
 
-// Hands every cached block of `dev` back to the driver.
+// Hands every cached block of `dev` (kAllDevices: of every one) back to the driver.
+constexpr int kAllDevices = -2;
 void drain(Cache& c, int dev, bool pinned) {
   std::vector<void*> out;
   {
     std::lock_guard<std::mutex> lock(c.m);
     for (auto it = c.blocks.begin(); it != c.blocks.end();) {
-      if (it->second.dev != dev) {
+      if (dev != kAllDevices && it->second.dev != dev) {
         ++it;
         continue;
       }
@@ -163,6 +164,11 @@ void* pinned_pool_get(size_t bytes) {
 void pinned_pool_put(void* p, size_t bytes) {
   if (!p) return;
   give(pinned_cache(), -1, p, rounded(pinned_cache(), bytes), true);
+}
+
+void release_pools() {
+  drain(device_cache(), kAllDevices, false);
+  drain(pinned_cache(), kAllDevices, true);
 }
 
 void synchronize_device(int device) {

@@ -115,6 +115,7 @@ def load():
         "DPBoosterGetLastPositions": (c_int, [H, c_void_p, c_uint64]),
         "DPBoosterGetTuning": (c_int, [H, POINTER(c_uint64), POINTER(c_char_p)]),
         "DPDMatrixGetCuts": (c_int, [H, c_int32, c_void_p, c_void_p, c_uint64, POINTER(c_int32)]),
+        "DPReleaseCachedMemory": (c_int, []),
         "dp_workspace_create": (c_int, [POINTER(H)]),
         "dp_workspace_free": (c_int, [H]),
         "dp_layout_init": (c_int, [c_int64, c_int32, c_int32, c_int32, POINTER(BinLayout)]),
@@ -172,6 +173,11 @@ def build_info():
     out = c_char_p()
     check(load().XGBuildInfo(ctypes.byref(out)))
     return json.loads(out.value.decode())
+
+
+def release_cached_memory():
+    """Hands the memory kept of freed matrices and boosters back to the driver."""
+    check(load().DPReleaseCachedMemory())
 
 
 def array_interface(t):

@@ -197,6 +197,12 @@ int DPValidateHyperparameters(const char* hyperparameters, uint32_t classes, bst
 int DPDMatrixGetCuts(DMatrixHandle handle, int32_t max_bin, int32_t* cut_ptr,
                      float* cut_values, bst_ulong capacity, int32_t* missing_bin);
 
+/* Hands the memory that the library keeps for later matrices and boosters back
+ * to the driver: up to 24 GiB of device memory and 2 GiB of pinned host memory
+ * of freed ones, which other allocators of the process cannot use meanwhile.
+ * Live matrices and boosters keep theirs.  Any thread may call it at any time. */
+int DPReleaseCachedMemory(void);
+
 /* ======================================================================= */
 /* 2. Kernel-level operator API                                             */
 /* ======================================================================= */

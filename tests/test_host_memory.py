@@ -171,3 +171,22 @@ print(json.dumps(fake.fake_live_bytes(0)))
 """)
     assert size <= got and got % 256 == 0
     assert got <= (size + 255 if size <= 1 << 20 or size > 12 << 30 else size * 17 // 16)
+
+
+def test_kept_memory_can_be_handed_back(host):
+    """Freed matrices' blocks stay for the next ones until the program asks for them."""
+    out = host("""
+        h = matrix(1000, 50)
+        second = matrix(10, 5, device=1)
+        before = [fake.fake_live_bytes(d) for d in (0, 1)]
+        ok(lib.XGDMatrixFree(h))
+        freed = fake.fake_live_bytes(0)
+        ok(lib.DPReleaseCachedMemory())
+        after = [fake.fake_live_bytes(d) for d in (0, 1)]
+        ok(lib.DPReleaseCachedMemory())
+        print(json.dumps([before, freed, after]))
+    """)
+    before, freed, after = out
+    assert freed == before[0]
+    assert after[0] == 4 * 1000 * 50  # the program's own array
+    assert 4 * 10 * 5 * 2 <= after[1] <= before[1]  # a live matrix keeps its copy
