@@ -32,7 +32,9 @@ namespace {
 // replaced (16 strided loads, 8 binary steps of one word each) took 0.70 ms for
 // 1M x 100 and 12.9 ms for 2M x 1,000 with 95 % missing, and the column copy a
 // pass of its own (0.71 ms at the latter); now 0.20 and 4.0 ms, copy included.
-constexpr int32_t kBinFeatures = 1 << 20;
+// Features up to which a lane's byte offset (24 rows and a row's end) fits 32 bits;
+// matrices of more take 64-bit ones.
+constexpr int32_t kBinFeatures = 1 << 25;
 constexpr int kBinRows = 8;
 constexpr int kBinThreads = 256;
 
@@ -40,7 +42,7 @@ struct __attribute__((packed)) UnalignedWords {  // 8 bytes at any address
   uint32_t w[2];
 };
 
-template <bool WIDE>
+template <bool WIDE, class Offset>
 __global__ __launch_bounds__(kBinThreads) void bin_kernel(
     const float* __restrict__ values, int64_t n_rows, int32_t n_features,
     const int32_t* __restrict__ cut_ptr, const float* __restrict__ cut_values,
@@ -70,11 +72,10 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
   uint8_t* tile = WIDE ? nullptr : bins + int64_t(f0 / kTile) * n_rows * kTile;
   const int64_t r1 = min(n_rows, (chunk + 1) * chunk_rows);
   constexpr int kWaveRows = 4 * kBinRows;
-  // Loads from wave-uniform bases and one 32-bit byte offset per lane (below 2^32
-  // for the 2^20 features a matrix may have): no branches and no address
-  // arithmetic, so all are in flight before the first wait.
-  const uint32_t offset = (uint32_t((lane >> 4) * kBinRows) * uint32_t(n_features) +
-                           uint32_t(min(f, n_features - 1))) * 4u;
+  // Loads from wave-uniform bases and one byte offset per lane: no branches and no
+  // address arithmetic, so all are in flight before the first wait.
+  const Offset offset = (Offset((lane >> 4) * kBinRows) * Offset(n_features) +
+                         Offset(min(f, n_features - 1))) * 4u;
   // Every wavefront takes part in each step (the columns' barriers), also past r1.
   for (int64_t w0 = chunk * chunk_rows + wave * kWaveRows; w0 - wave * kWaveRows < r1;
        w0 += kBinThreads / 64 * kWaveRows) {
@@ -580,9 +581,10 @@ void launch_bin_values(const float* values, const dp_bin_layout& layout, const i
                        const float* cut_values, uint8_t* bins, uint8_t* cols, hipStream_t s) {
   if (layout.n_rows <= 0) return;
   need(layout.tile_width == kTile, "binning needs 16-feature tiles");
-  need(layout.n_features <= kBinFeatures, "too many features to bin");
   const int32_t chunks = bin_chunks(layout.n_rows, layout.n_tiles);
-  hipLaunchKernelGGL(bin_kernel<false>, dim3(unsigned((layout.n_tiles * chunks + 7) / 8 * 8)),
+  const auto kernel = layout.n_features <= kBinFeatures ? bin_kernel<false, uint32_t>
+                                                        : bin_kernel<false, uint64_t>;
+  hipLaunchKernelGGL(kernel, dim3(unsigned((layout.n_tiles * chunks + 7) / 8 * 8)),
                      dim3(kBinThreads), 0, s, values, layout.n_rows, layout.n_features, cut_ptr,
                      cut_values, layout.missing_bin, layout.n_tiles, chunks,
                      (layout.n_rows + chunks - 1) / chunks, bins, cols,
@@ -594,12 +596,13 @@ void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_feature
                           const int32_t* cut_ptr, const float* cut_values, uint16_t* cols,
                           hipStream_t s) {
   if (n_rows <= 0 || n_features <= 0) return;
-  need(n_features <= kBinFeatures, "too many features to bin");
   const int32_t tiles = (n_features + kTile - 1) / kTile, chunks = bin_chunks(n_rows, tiles);
-  hipLaunchKernelGGL(bin_kernel<true>, dim3(unsigned((tiles * chunks + 7) / 8 * 8)),
-                     dim3(kBinThreads), 0, s, values, n_rows, n_features, cut_ptr, cut_values,
-                     kWideMissing, tiles, chunks, (n_rows + chunks - 1) / chunks,
-                     static_cast<uint8_t*>(nullptr), static_cast<uint8_t*>(nullptr), cols);
+  const auto kernel =
+      n_features <= kBinFeatures ? bin_kernel<true, uint32_t> : bin_kernel<true, uint64_t>;
+  hipLaunchKernelGGL(kernel, dim3(unsigned((tiles * chunks + 7) / 8 * 8)), dim3(kBinThreads), 0, s,
+                     values, n_rows, n_features, cut_ptr, cut_values, kWideMissing, tiles, chunks,
+                     (n_rows + chunks - 1) / chunks, static_cast<uint8_t*>(nullptr),
+                     static_cast<uint8_t*>(nullptr), cols);
   DP_HIP(hipGetLastError());
 }
 

@@ -32,7 +32,8 @@ __device__ __forceinline__ float key_value(uint32_t k) {
 // *(base + byte offset) with a wave-uniform base: one load with a scalar base and a
 // 32-bit vector offset (the empty asm keeps the compiler from folding the two into
 // 64-bit vector additions per load).
-__device__ __forceinline__ float load_at(const float* base, uint32_t offset) {
+template <class Offset>
+__device__ __forceinline__ float load_at(const float* base, Offset offset) {
   uint64_t b = reinterpret_cast<uint64_t>(base);
   asm("" : "+s"(b));
   const auto* p = reinterpret_cast<const __attribute__((address_space(1))) char*>(b) + offset;

@@ -89,3 +89,23 @@ def test_matrices_are_copied_whole(dp, device, rows, features, missing):
             with pytest.raises(Exception, match="inf"):
                 dp.DMatrix(v, missing=float(missing))
             v.copy_(torch.as_tensor(x))
+
+
+@pytest.mark.parametrize("rows,features", [(64, (1 << 20) + 17), (40, (1 << 25) + 5)])
+def test_bins_of_very_wide_matrices(dp, device, rows, features):
+    """More features than a lane's 32-bit offset reaches, and than the widest matrices of
+    practice; one cut at 0 and the last one."""
+    import torch
+    from dpgbdt import ops
+
+    x = torch.randn((rows, features), device=device,
+                    generator=torch.Generator(device).manual_seed(features))
+    x[1, features - 1] = float("nan")
+    lay = ops.layout(rows, features, 0, 255)
+    ptr = np.arange(features + 1, dtype=np.int32) * 2
+    bins = ops.bin_values(x, lay, ptr, np.tile(np.float32([0.0, 9.0]), features))
+    tiles = bins.view(lay.n_tiles, rows, 16)
+    want = torch.where(torch.isnan(x), 255, (x >= 0).to(torch.uint8)).to(torch.uint8)
+    pad = torch.zeros((rows, lay.n_tiles * 16 - features), dtype=torch.uint8, device=device)
+    want = torch.cat([want, pad], dim=1).view(rows, lay.n_tiles, 16)
+    assert torch.equal(tiles, want.transpose(0, 1))
