@@ -134,7 +134,7 @@ __device__ __forceinline__ bool row_kept(const RowSample& rs, uint64_t prefix, i
 
 __global__ __launch_bounds__(kQuantThreads) void absmax_kernel(
     const float* __restrict__ grad, const float* __restrict__ hess, int64_t n_rows,
-    int n_classes, unsigned* __restrict__ max_slots, RowSample rs) {
+    int n_classes, uint2* __restrict__ max_slots, RowSample rs) {
   const int k = blockIdx.y;
   const uint64_t prefix = row_prefix(rs, k);
   unsigned mg = 0, mh = 0;
@@ -145,11 +145,7 @@ __global__ __launch_bounds__(kQuantThreads) void absmax_kernel(
     mh = max(mh, __float_as_uint(fabsf(hess[r * n_classes + k])));
   }
   block_max2(mg, mh);
-  if (threadIdx.x == 0) {
-    unsigned* slot = max_slots + (int64_t(k) * gridDim.x + blockIdx.x) * 2;
-    slot[0] = mg;
-    slot[1] = mh;
-  }
+  if (threadIdx.x == 0) max_slots[int64_t(k) * gridDim.x + blockIdx.x] = make_uint2(mg, mh);
 }
 
 __device__ __forceinline__ int quant_exp(unsigned bits) {
@@ -164,16 +160,16 @@ __device__ __forceinline__ int quant_exp(unsigned bits) {
 // workgroup's sums to the sum slots.
 __global__ __launch_bounds__(kQuantThreads) void quantise_kernel(
     const float* __restrict__ grad, const float* __restrict__ hess, int64_t n_rows,
-    int n_classes, const unsigned* __restrict__ max_slots, int32_t* __restrict__ exps,
+    int n_classes, const uint2* __restrict__ max_slots, int n_max, int32_t* __restrict__ exps,
     int2* __restrict__ gpair, long long* __restrict__ sum_slots, RowSample rs) {
   __shared__ long long wave_sum[2][kQuantThreads / 64];
   __shared__ int s_exp[2];
   const int k = blockIdx.y;
   unsigned mg = 0, mh = 0;
-  const unsigned* slots = max_slots + int64_t(k) * gridDim.x * 2;
-  for (int b = threadIdx.x; b < int(gridDim.x); b += kQuantThreads) {
-    mg = max(mg, slots[2 * b]);
-    mh = max(mh, slots[2 * b + 1]);
+  const uint2* slots = max_slots + int64_t(k) * n_max;
+  for (int b = threadIdx.x; b < n_max; b += kQuantThreads) {
+    mg = max(mg, slots[b].x);
+    mh = max(mh, slots[b].y);
   }
   block_max2(mg, mh);
   if (threadIdx.x == 0) {
@@ -410,7 +406,7 @@ __host__ __device__ __forceinline__ int quant_rows(int n_classes) {
 
 __global__ __launch_bounds__(kQuantThreads) void class_quantise_kernel(
     const float* __restrict__ grad, const float* __restrict__ hess, int64_t n_rows,
-    int n_classes, const uint2* __restrict__ max_slots, int32_t* __restrict__ exps,
+    int n_classes, const uint2* __restrict__ max_slots, int n_max, int32_t* __restrict__ exps,
     int2* __restrict__ gpair, long long* __restrict__ sum_slots, RowSample rs) {
   __shared__ __attribute__((aligned(16))) int2 s[kQuantPairs];
   __shared__ int2 s_exp[kQuantThreads];
@@ -418,9 +414,9 @@ __global__ __launch_bounds__(kQuantThreads) void class_quantise_kernel(
   const int lane = threadIdx.x & 63;
   // Every workgroup reduces the classes' maxima slots, a wavefront per class.
   for (int k = int(threadIdx.x) >> 6; k < n_classes; k += kQuantThreads / 64) {
-    const uint2* slots = max_slots + int64_t(k) * gridDim.x;
+    const uint2* slots = max_slots + int64_t(k) * n_max;
     unsigned a = 0, b = 0;
-    for (int i = lane; i < int(gridDim.x); i += 64) {
+    for (int i = lane; i < n_max; i += 64) {
       const uint2 v = slots[i];
       a = max(a, v.x);
       b = max(b, v.y);
@@ -534,19 +530,54 @@ static bool flat_classes(int32_t n_classes) {
   return n_classes >= 2 && n_classes <= kQuantThreads;
 }
 
-// One output: at least four rows per thread, since every quantise workgroup
-// re-reads all the maxima slots: a 1M-row pass keeps about 1,000 of them (four per
-// CU; eight rows per thread measured 0.8 % slower on C2's trees), a 10M-row one
-// 2048.  Several: a tile of rows each, at most 1,024 workgroups and, again for
-// the slots every one of them reads, at most 16,384 slots.
-int quantise_blocks(int64_t n_rows, int32_t n_classes) {
-  if (!flat_classes(n_classes)) return grid_for(n_rows, kQuantThreads * 4, kQuantBlocks);
+// Where the flat quantiser is the faster: arrays too large for the L2s to serve the
+// other one's strided passes (from about 2.5M elements; us, strided and flat: 300k x
+// 10 40 and 29, 100k x 32 79 and 38, but 100k x 10 8 and 16, 30k x 32 12 and 28).
+// With more classes a workgroup's tile has few rows and its reduction of all their
+// maxima weighs more: 100k x 128 411 and 303 but 30k x 128 44 and 112, and 100k x
+// 200 626 and 1,109.  Two classes waste half of a strided line only: 1M x 2 12 and 21.
+static bool flat_quantise(int64_t n_rows, int32_t n_classes) {
+  const int64_t n = n_rows * n_classes;
+  return n_classes >= 3 && (n_classes <= 64 ? n >= 2'500'000 : n_classes <= 128 && n >= 8'000'000);
+}
+
+// The flat maxima pass has no such cost; strided it is the faster for few classes
+// of arrays below 1M elements (100k x 2 3.4 and 5.0 us, 1M x 2 8.1 and 7.1).
+static bool flat_absmax(int64_t n_rows, int32_t n_classes) {
+  return flat_classes(n_classes) && (n_classes >= 6 || n_rows * n_classes >= 1'000'000);
+}
+
+// Workgroups of the flat kernels: a tile of rows each, at most 1,024 workgroups and,
+// for the maxima slots every quantise workgroup reads, at most 16,384 slots.
+static int flat_blocks(int64_t n_rows, int32_t n_classes) {
   return grid_for(n_rows, quant_rows(n_classes), std::clamp(16384 / n_classes, 64, 1024));
+}
+
+// The other kernels, per class: at least four rows per thread, since every quantise
+// workgroup re-reads all the maxima slots: a 1M-row pass keeps about 1,000 of them
+// (four per CU; eight rows per thread measured 0.8 % slower on C2's trees), a 10M-row
+// one 2048.
+int quantise_blocks(int64_t n_rows, int32_t n_classes) {
+  if (flat_quantise(n_rows, n_classes)) return flat_blocks(n_rows, n_classes);
+  return grid_for(n_rows, kQuantThreads * 4, kQuantBlocks);
+}
+
+// Maxima slots per class.
+static int maxima_blocks(int64_t n_rows, int32_t n_classes) {
+  return flat_classes(n_classes) ? flat_blocks(n_rows, n_classes)
+                                 : quantise_blocks(n_rows, n_classes);
+}
+
+// The quantiser's scratch: the maxima slots, then the sum slots.
+static size_t sum_slots_at(int64_t n_rows, int32_t n_classes) {
+  const size_t slots = size_t(n_classes) * size_t(std::max(maxima_blocks(n_rows, n_classes),
+                                                           quantise_blocks(n_rows, n_classes)));
+  return (slots * sizeof(uint2) + 255) & ~size_t(255);
 }
 
 size_t quantise_scratch_bytes(int64_t n_rows, int32_t n_classes) {
   const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows, n_classes));
-  return slots * 2 * sizeof(uint32_t) + 256 + slots * 2 * sizeof(int64_t);
+  return sum_slots_at(n_rows, n_classes) + slots * 2 * sizeof(int64_t);
 }
 
 void launch_init_margin(float* margin, int64_t n_rows, int32_t n_outputs, const float* base,
@@ -564,9 +595,12 @@ bool launch_gradients(int32_t objective, float* margin, const float* label,
   need(objective == DP_OBJ_LOGISTIC || objective == DP_OBJ_SOFTPROB ||
            objective == DP_OBJ_SQUARED,
        "unknown objective id");
-  if (objective == DP_OBJ_SOFTPROB && flat_classes(n_classes)) {
+  // Without maxima to leave, a row of two or three outputs is the faster with a
+  // thread of its own (1M x 2 9.8 us against 15.2, x 3 14.3 against 18.7).
+  if (objective == DP_OBJ_SOFTPROB && flat_classes(n_classes) &&
+      (quant_scratch || n_classes > 3)) {
     const auto kernel = quant_scratch ? softprob_kernel<true> : softprob_kernel<false>;
-    const int blocks = quant_scratch ? quantise_blocks(n_rows, n_classes)
+    const int blocks = quant_scratch ? maxima_blocks(n_rows, n_classes)
                                      : grid_for(n_rows, soft_rows(n_classes), 4096);
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kQuantThreads), 0, s, margin, label, n_rows,
                        n_classes, grad, hess, static_cast<uint2*>(quant_scratch), values);
@@ -574,8 +608,8 @@ bool launch_gradients(int32_t objective, float* margin, const float* label,
     return quant_scratch != nullptr;
   }
   if (quant_scratch && n_classes == 1) {
-    hipLaunchKernelGGL(gradients_kernel<true>, dim3(quantise_blocks(n_rows, n_classes)), dim3(kQuantThreads),
-                       0, s, objective, margin, label, n_rows, n_classes, grad, hess,
+    hipLaunchKernelGGL(gradients_kernel<true>, dim3(maxima_blocks(n_rows, n_classes)),
+                       dim3(kQuantThreads), 0, s, objective, margin, label, n_rows, n_classes, grad, hess,
                        static_cast<unsigned*>(quant_scratch), values);
     DP_HIP(hipGetLastError());
     return true;
@@ -602,29 +636,28 @@ void launch_quantise(const float* grad, const float* hess, int64_t n_rows, int32
   need(n_classes >= 1 && n_classes <= 65535, "class count out of range");
   need(n_rows >= 1, "quantiser needs at least one row");
   const int blocks = quantise_blocks(n_rows, n_classes);
-  const size_t slots = size_t(n_classes) * size_t(blocks);
-  auto* max_slots = static_cast<unsigned*>(scratch);
+  // The strided maxima pass leaves a slot per workgroup of the strided quantiser.
+  const bool few_slots = !maxima_ready && !flat_absmax(n_rows, n_classes);
+  const int n_max = few_slots ? blocks : maxima_blocks(n_rows, n_classes);
+  auto* max_slots = static_cast<uint2*>(scratch);
   auto* sum_slots = reinterpret_cast<long long*>(static_cast<uint8_t*>(scratch) +
-                                                 ((slots * 2 * sizeof(uint32_t) + 255) & ~size_t(255)));
-  const bool flat = flat_classes(n_classes);
-  auto* pair_slots = reinterpret_cast<uint2*>(max_slots);
+                                                 sum_slots_at(n_rows, n_classes));
+  auto* pairs = reinterpret_cast<int2*>(gpair);
   if (!maxima_ready) {
-    if (flat)
-      hipLaunchKernelGGL(class_absmax_kernel, dim3(blocks), dim3(kQuantThreads), 0, s, grad, hess,
-                         n_rows, n_classes, pair_slots, rows);
+    if (!few_slots)
+      hipLaunchKernelGGL(class_absmax_kernel, dim3(n_max), dim3(kQuantThreads), 0, s, grad, hess,
+                         n_rows, n_classes, max_slots, rows);
     else
-      hipLaunchKernelGGL(absmax_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
+      hipLaunchKernelGGL(absmax_kernel, dim3(n_max, n_classes), dim3(kQuantThreads), 0, s, grad,
                          hess, n_rows, n_classes, max_slots, rows);
     DP_HIP(hipGetLastError());
   }
-  if (flat)
+  if (flat_quantise(n_rows, n_classes))
     hipLaunchKernelGGL(class_quantise_kernel, dim3(blocks), dim3(kQuantThreads), 0, s, grad, hess,
-                       n_rows, n_classes, pair_slots, exps, reinterpret_cast<int2*>(gpair),
-                       sum_slots, rows);
+                       n_rows, n_classes, max_slots, n_max, exps, pairs, sum_slots, rows);
   else
     hipLaunchKernelGGL(quantise_kernel, dim3(blocks, n_classes), dim3(kQuantThreads), 0, s, grad,
-                     hess, n_rows, n_classes, max_slots, exps, reinterpret_cast<int2*>(gpair),
-                     sum_slots, rows);
+                       hess, n_rows, n_classes, max_slots, n_max, exps, pairs, sum_slots, rows);
   DP_HIP(hipGetLastError());
   if (!sums) return;  // the caller reduces the sum slots itself
   hipLaunchKernelGGL(finish_sums_kernel, dim3(n_classes), dim3(kQuantThreads), 0, s, sum_slots,
@@ -633,9 +666,8 @@ void launch_quantise(const float* grad, const float* hess, int64_t n_rows, int32
 }
 
 const int64_t* quantise_sum_slots(const void* scratch, int64_t n_rows, int32_t n_classes) {
-  const size_t slots = size_t(n_classes) * size_t(quantise_blocks(n_rows, n_classes));
   return reinterpret_cast<const int64_t*>(static_cast<const uint8_t*>(scratch) +
-                                          ((slots * 2 * sizeof(uint32_t) + 255) & ~size_t(255)));
+                                          sum_slots_at(n_rows, n_classes));
 }
 
 }  // namespace dp

@@ -7,7 +7,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,k", [(1, 2), (3, 256), (255, 3), (257, 10), (1000, 64), (999, 65),
-                                 (70001, 7), (2100, 255), (2100, 256), (300, 257), (300, 300)])
+                                 (70001, 7), (2100, 255), (2100, 256), (300, 257), (300, 300),
+                                 # the quantisers and maxima passes change over
+                                 (500000, 2), (499999, 2), (833333, 3), (833334, 3),
+                                 (250000, 10), (249999, 10), (39063, 64), (62500, 128),
+                                 (62499, 128), (124100, 65), (6000, 200)])
 def test_softprob_and_quantiser_match_the_oracle(dp, oracle, ws, device, n, k):
     import torch
     from dpgbdt import ops
@@ -45,3 +49,18 @@ def test_rounds_add_leaf_values_in_the_gradients(dp, oracle, device, k):
         bst.update(d, r)
     np.testing.assert_array_equal(bst.margins(n, k).view(np.uint32),
                                   bst.predict(x, margin=True).cpu().numpy().view(np.uint32))
+
+
+@pytest.mark.parametrize("n,k", [(250000, 10), (3000, 10), (3000, 3), (400, 130)])
+def test_row_samples_of_several_outputs(dp, oracle, device, n, k):
+    """Sampled rows' maxima and pairs, a draw per output, in each quantiser."""
+    import torch
+    from test_gpu_booster import _compare, _train_both
+
+    rng = np.random.default_rng(n + k)
+    x = torch.as_tensor(rng.integers(0, 20, (n, 3)).astype(np.float32), device=device)
+    y = torch.as_tensor(rng.integers(0, k, n).astype(np.float32), device=device)
+    bst, _, o_trees, o_margin, pos, _ = _train_both(
+        dp, oracle, device, 0, n, 3, 1, k, {"max_depth": 2, "eta": 0.3}, 2, 0,
+        values_labels=(x, y), sample={"seed": 5, "subsample": 0.7})
+    _compare(bst, o_trees, o_margin, pos, n, k)
