@@ -49,20 +49,22 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
     int32_t missing_bin, int32_t tiles, int32_t chunks, int64_t chunk_rows,
     uint8_t* __restrict__ bins, uint8_t* __restrict__ cols, uint16_t* __restrict__ cols16) {
   __shared__ uint4 tree[search_nodes(4) * kTile];
+  __shared__ int32_t s_ptr[kTile + 1];
   __shared__ uint2 s_cols[kTile][kBinThreads / 16 + 1];  // [feature][8 rows each]
   const int32_t per = (tiles * chunks + 7) / 8;
   const int32_t item = int32_t(blockIdx.x % 8) * per + int32_t(blockIdx.x / 8);
   if (int32_t(blockIdx.x / 8) >= per || item >= tiles * chunks) return;
   const int32_t chunk = item / tiles, f0 = item % tiles * kTile;
+  if (threadIdx.x <= kTile) s_ptr[threadIdx.x] = cut_ptr[min(f0 + int(threadIdx.x), n_features)];
+  __syncthreads();
   int widest = 1;
-  for (int k = 0; k < kTile && f0 + k < n_features; ++k)
-    widest = max(widest, cut_ptr[f0 + k + 1] - cut_ptr[f0 + k]);
+#pragma unroll
+  for (int k = 0; k < kTile; ++k) widest = max(widest, s_ptr[k + 1] - s_ptr[k]);
   const int levels = search_levels(min(widest, kMaxBins));
   // bin(x) = cuts <= x, the last cut left out: the clamp to the last bin.
   search_fill(tree, levels, [&](int j, int p) {
-    const int f = f0 + j;
-    if (f >= n_features || p >= cut_ptr[f + 1] - cut_ptr[f]) return kNanKey;
-    return order_key(cut_values[cut_ptr[f] + p - 1]);
+    if (p >= s_ptr[j + 1] - s_ptr[j]) return kNanKey;
+    return order_key(cut_values[s_ptr[j] + p - 1]);
   });
   __syncthreads();
   const int lane = threadIdx.x & 63;
@@ -146,6 +148,59 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(
           to[u] = uint8_t((u < 4 ? v.x >> (8 * u) : v.y >> (8 * (u - 4))));
       }
     }
+  }
+}
+
+// The same for matrices of few features, whose tile would leave most of bin_kernel's
+// lanes without one: a thread per row, its features' binary searches side by side.
+// Cuts past a feature's last are NaN, which no value reaches.  1M rows with 255 bins,
+// bin_kernel and here: x 1 37 and 11 us, x 5 38 and 21, x 8 39 and 32 (2 bins: 20 and
+// 22), about 4 us more per feature.
+constexpr int kNarrow = 8;
+template <bool WIDE>
+__global__ __launch_bounds__(kBinThreads) void bin_narrow_kernel(
+    const float* __restrict__ values, int64_t n_rows, int32_t n_features,
+    const int32_t* __restrict__ cut_ptr, const float* __restrict__ cut_values,
+    int32_t missing_bin, uint8_t* __restrict__ bins, uint8_t* __restrict__ cols,
+    uint16_t* __restrict__ cols16) {
+  __shared__ float s_cuts[kNarrow][kMaxBins];
+  int widest = 1;  // cuts searched: all but the last, the clamp to the last bin
+#pragma unroll
+  for (int k = 0; k < kNarrow; ++k) {
+    const int at = cut_ptr[min(k, n_features)];
+    const int n = min(cut_ptr[min(k + 1, n_features)] - at, kMaxBins) - 1;
+    widest = max(widest, n);
+    for (int b = threadIdx.x; b < kMaxBins; b += kBinThreads)
+      s_cuts[k][b] = b < n ? cut_values[at + b] : __builtin_nanf("");
+  }
+  const int top = 1 << (31 - __builtin_clz(widest));
+  __syncthreads();
+  for (int64_t r = int64_t(blockIdx.x) * kBinThreads + threadIdx.x; r < n_rows;
+       r += int64_t(gridDim.x) * kBinThreads) {
+    const float* row = values + r * n_features;
+    float x[kNarrow];
+    int bin[kNarrow];
+#pragma unroll
+    for (int k = 0; k < kNarrow; ++k) {
+      x[k] = row[min(k, n_features - 1)];
+      bin[k] = 0;
+    }
+    for (int step = top; step > 0; step >>= 1) {
+#pragma unroll
+      for (int k = 0; k < kNarrow; ++k)
+        if (k < n_features) bin[k] += s_cuts[k][bin[k] + step - 1] <= x[k] ? step : 0;
+    }
+    uint32_t word[2] = {0u, 0u};
+#pragma unroll
+    for (int k = 0; k < kNarrow; ++k) {
+      if (k >= n_features) break;
+      if (x[k] != x[k]) bin[k] = WIDE ? kWideMissing : missing_bin & 0xff;
+      word[k >> 2] |= uint32_t(bin[k]) << (8 * (k & 3));
+      if constexpr (WIDE) cols16[int64_t(k) * n_rows + r] = uint16_t(bin[k]);
+      else if (cols) cols[int64_t(k) * n_rows + r] = uint8_t(bin[k]);
+    }
+    if constexpr (!WIDE)
+      *reinterpret_cast<uint4*>(bins + r * kTile) = make_uint4(word[0], word[1], 0u, 0u);
   }
 }
 
@@ -570,24 +625,38 @@ void launch_copy_matrix(const float* src, int64_t row_stride, int64_t n_rows, in
   DP_HIP(hipGetLastError());
 }
 
-// Row chunks of the binning grid: about eight workgroups per CU, of at least
-// 1,024 rows so that the tile's tables are worth their fill.
-static int32_t bin_chunks(int64_t n_rows, int32_t tiles) {
-  const int64_t chunks = std::min<int64_t>((n_rows + 1023) / 1024, (2048 + tiles - 1) / tiles);
-  return int32_t(std::max<int64_t>(chunks, 1));
+// Row chunks of the binning grid: as many workgroups as the chip holds at once (six
+// per CU by their LDS), of whole steps.  (At least 1,024 rows each left small
+// matrices to a few workgroups: 20k x 30 with 255 bins 23 us against 11.)
+struct BinChunks {
+  int32_t n;
+  int64_t rows;
+};
+static BinChunks bin_chunks(int64_t n_rows, int32_t tiles) {
+  constexpr int32_t kStep = kBinThreads / 16 * kBinRows, kHeld = 6 * 256;
+  const int64_t steps = (n_rows + kStep - 1) / kStep, most = std::max(1, kHeld / tiles);
+  const int64_t each = (steps + most - 1) / most;
+  return {int32_t((steps + each - 1) / each), each * kStep};
 }
 
 void launch_bin_values(const float* values, const dp_bin_layout& layout, const int32_t* cut_ptr,
                        const float* cut_values, uint8_t* bins, uint8_t* cols, hipStream_t s) {
   if (layout.n_rows <= 0) return;
   need(layout.tile_width == kTile, "binning needs 16-feature tiles");
-  const int32_t chunks = bin_chunks(layout.n_rows, layout.n_tiles);
+  if (layout.n_features <= kNarrow) {
+    hipLaunchKernelGGL(bin_narrow_kernel<false>, dim3(grid_for(layout.n_rows, kBinThreads, 2048)),
+                       dim3(kBinThreads), 0, s, values, layout.n_rows, layout.n_features, cut_ptr,
+                       cut_values, layout.missing_bin, bins, cols, nullptr);
+    DP_HIP(hipGetLastError());
+    return;
+  }
+  const BinChunks chunks = bin_chunks(layout.n_rows, layout.n_tiles);
   const auto kernel = layout.n_features <= kBinFeatures ? bin_kernel<false, uint32_t>
                                                         : bin_kernel<false, uint64_t>;
-  hipLaunchKernelGGL(kernel, dim3(unsigned((layout.n_tiles * chunks + 7) / 8 * 8)),
+  hipLaunchKernelGGL(kernel, dim3(unsigned((layout.n_tiles * chunks.n + 7) / 8 * 8)),
                      dim3(kBinThreads), 0, s, values, layout.n_rows, layout.n_features, cut_ptr,
-                     cut_values, layout.missing_bin, layout.n_tiles, chunks,
-                     (layout.n_rows + chunks - 1) / chunks, bins, cols,
+                     cut_values, layout.missing_bin, layout.n_tiles, chunks.n, chunks.rows, bins,
+                     cols,
                      static_cast<uint16_t*>(nullptr));
   DP_HIP(hipGetLastError());
 }
@@ -596,12 +665,20 @@ void launch_bin_columns16(const float* values, int64_t n_rows, int32_t n_feature
                           const int32_t* cut_ptr, const float* cut_values, uint16_t* cols,
                           hipStream_t s) {
   if (n_rows <= 0 || n_features <= 0) return;
-  const int32_t tiles = (n_features + kTile - 1) / kTile, chunks = bin_chunks(n_rows, tiles);
+  if (n_features <= kNarrow) {
+    hipLaunchKernelGGL(bin_narrow_kernel<true>, dim3(grid_for(n_rows, kBinThreads, 2048)),
+                       dim3(kBinThreads), 0, s, values, n_rows, n_features, cut_ptr, cut_values,
+                       kWideMissing, nullptr, nullptr, cols);
+    DP_HIP(hipGetLastError());
+    return;
+  }
+  const int32_t tiles = (n_features + kTile - 1) / kTile;
+  const BinChunks chunks = bin_chunks(n_rows, tiles);
   const auto kernel =
       n_features <= kBinFeatures ? bin_kernel<true, uint32_t> : bin_kernel<true, uint64_t>;
-  hipLaunchKernelGGL(kernel, dim3(unsigned((tiles * chunks + 7) / 8 * 8)), dim3(kBinThreads), 0, s,
-                     values, n_rows, n_features, cut_ptr, cut_values, kWideMissing, tiles, chunks,
-                     (n_rows + chunks - 1) / chunks, static_cast<uint8_t*>(nullptr),
+  hipLaunchKernelGGL(kernel, dim3(unsigned((tiles * chunks.n + 7) / 8 * 8)), dim3(kBinThreads), 0,
+                     s, values, n_rows, n_features, cut_ptr, cut_values, kWideMissing, tiles,
+                     chunks.n, chunks.rows, static_cast<uint8_t*>(nullptr),
                      static_cast<uint8_t*>(nullptr), cols);
   DP_HIP(hipGetLastError());
 }

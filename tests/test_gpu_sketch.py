@@ -109,3 +109,46 @@ def test_bins_of_very_wide_matrices(dp, device, rows, features):
     pad = torch.zeros((rows, lay.n_tiles * 16 - features), dtype=torch.uint8, device=device)
     want = torch.cat([want, pad], dim=1).view(rows, lay.n_tiles, 16)
     assert torch.equal(tiles, want.transpose(0, 1))
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 3000, 530001])
+@pytest.mark.parametrize("features", [1, 5, 8, 9])
+def test_bins_of_narrow_matrices(dp, oracle, ws, device, n, features):
+    """A thread per row up to 8 features, more threads than rows and fewer (2,048 workgroups)."""
+    import torch
+    from dpgbdt import ops
+
+    rng = np.random.default_rng(n + features)
+    x = rng.normal(size=(n, features)).astype(np.float32)
+    x[:, -1] = rng.integers(-2, 2, n)
+    x[rng.random(x.shape) < 0.05] = np.nan
+    x[rng.random(x.shape) < 0.05] = -0.0
+    for max_bin in (2, 16, 17, 255):
+        ptr, cuts, _ = oracle.compute_cuts(x, max_bin)
+        y = x.copy()
+        y[rng.random(x.shape) < 0.05] *= 100.0  # above the last cut
+        lay = ops.layout(n, features, 0, 255)
+        bins = ops.bin_values(torch.as_tensor(y, device=device), lay, ptr, cuts)
+        np.testing.assert_array_equal(ops.from_tiles(bins.cpu().numpy(), lay),
+                                      oracle.bin_matrix(y, ptr, cuts, 255))
+        tile = bins.view(-1, n, 16)[-1].cpu().numpy()
+        assert not tile[:, (features - 1) % 16 + 1:].any()  # the tile's padding
+
+
+@pytest.mark.parametrize("features", [1, 8, 9])
+@pytest.mark.parametrize("max_bin", [200, 256])
+def test_training_on_narrow_matrices_with_missing_values(dp, oracle, device, features, max_bin):
+    """The column copies made with the bins: bytes, and 16-bit symbols for 256 bins."""
+    import torch
+    from test_gpu_booster import _compare, _train_both
+
+    rng = np.random.default_rng(features + max_bin)
+    n = 5000
+    x = rng.normal(size=(n, features)).astype(np.float32)
+    x[rng.random(x.shape) < 0.1] = np.nan
+    y = (rng.random(n) < 0.5).astype(np.float32)
+    bst, _, o_trees, o_margin, pos, _ = _train_both(
+        dp, oracle, device, 0, n, features, 0, 1, {"max_depth": 5, "eta": 0.3}, 2, 0,
+        max_bin=max_bin, values_labels=(torch.as_tensor(x, device=device),
+                                        torch.as_tensor(y, device=device)))
+    _compare(bst, o_trees, o_margin, pos, n, 1)
