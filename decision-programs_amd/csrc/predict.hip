@@ -20,6 +20,7 @@
 //     400 x 160 trees 255 against 196, 9,000 x 600 x 200 trees 83 against 70.)
 //     Nodes come from global memory (a batch is walked by too few rows to be
 //     worth staging).
+//   predict_direct_kernel  small forests: a row per thread, nothing in LDS.
 //
 // One thread per row over global memory, the form these replaced, took 7,140 us
 // for 1M x 28 rows through 100 trees of depth 8, 2,700 us for 60k x 784 through
@@ -33,6 +34,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace dp {
 namespace {
@@ -59,21 +61,21 @@ __device__ __forceinline__ float pred_expf(float x) {
 constexpr int kPredThreads = 1024;
 constexpr int kWalk = 4;  // trees a lane walks side by side
 
-// Walks kWalk trees of packed nodes from the nodes at[w] (a leaf walks in place)
-// to their leaves, which at[w] then names.  fetch(w, i): node i of tree w;
+// Walks W trees of packed nodes from the nodes at[w] (a leaf walks in place) to
+// their leaves, which at[w] then names.  fetch(w, i): node i of tree w;
 // value(word): the row's value of the feature in bits 17-30.  Every step is
 // straight-line code; whether all lanes are at leaves is asked every fourth.
-template <class Fetch, class Value>
+template <int W = kWalk, class Fetch, class Value>
 __device__ __forceinline__ void walk(uint32_t* at, int32_t depth, Fetch fetch, Value value) {
-  PackedNode node[kWalk];
+  PackedNode node[W];
 #pragma unroll
-  for (int w = 0; w < kWalk; ++w) node[w] = fetch(w, at[w]);
+  for (int w = 0; w < W; ++w) node[w] = fetch(w, at[w]);
   for (int32_t d = 1; d <= depth; ++d) {
-    float x[kWalk];
+    float x[W];
 #pragma unroll
-    for (int w = 0; w < kWalk; ++w) x[w] = value(node[w].word);
+    for (int w = 0; w < W; ++w) x[w] = value(node[w].word);
 #pragma unroll
-    for (int w = 0; w < kWalk; ++w) {
+    for (int w = 0; w < W; ++w) {
       const float y = __uint_as_float(__float_as_uint(x[w]) ^ (node[w].word & 0x80000000u));
       at[w] = (node[w].word & 0xffffu) + (y >= node[w].cond ? 1u : 0u);
       node[w] = fetch(w, at[w]);
@@ -81,7 +83,7 @@ __device__ __forceinline__ void walk(uint32_t* at, int32_t depth, Fetch fetch, V
     if ((d & 3) == 0) {
       bool inner = false;
 #pragma unroll
-      for (int w = 0; w < kWalk; ++w) inner = inner || node[w].cond == node[w].cond;
+      for (int w = 0; w < W; ++w) inner = inner || node[w].cond == node[w].cond;
       if (!__any(inner)) break;
     }
   }
@@ -218,6 +220,54 @@ __global__ __launch_bounds__(R) void predict_rows_kernel(
     }
   }
   sum.finish();
+}
+
+// Small forests: a thread per row, nodes and values from global memory; kWalk trees
+// side by side, then two (`pairs`), then one.
+constexpr int kDirectThreads = 256;
+template <class Node>
+__global__ __launch_bounds__(kDirectThreads) void predict_direct_kernel(
+    const float* __restrict__ values, int64_t n_rows, int64_t row_stride, float missing,
+    const Node* __restrict__ nodes, const float* __restrict__ leaf_values,
+    const int32_t* __restrict__ tree_ptr, const int32_t* __restrict__ tree_base,
+    const int32_t* __restrict__ group_ptr, int32_t groups, int32_t trees, int32_t depth,
+    const float* __restrict__ base, int32_t transform, bool pairs, float* __restrict__ out) {
+  const int32_t outputs = transform == kPredArgmax ? 1 : groups;
+  for (int64_t r = int64_t(blockIdx.x) * kDirectThreads + threadIdx.x; r < n_rows;
+       r += int64_t(gridDim.x) * kDirectThreads) {
+    const float* v = values + r * row_stride;
+    Margins sum(group_ptr, base, {out + r * outputs, groups, transform, true});
+    auto value = [&](int32_t f) { return or_nan(v[f], missing); };
+    if constexpr (sizeof(Node) == sizeof(PackedNode)) {
+      auto some = [&](int32_t t, auto count) {  // `count` trees from t on
+        constexpr int W = decltype(count)::value;
+        uint32_t at[W];
+        int32_t origin[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+          origin[w] = tree_base[t + w];
+          at[w] = uint32_t(tree_ptr[t + w] - origin[w]);
+        }
+        walk<W>(at, depth, [&](int w, uint32_t i) { return nodes[origin[w] + int32_t(i)]; },
+                [&](uint32_t word) { return value(int32_t(word >> 17 & 0x3fffu)); });
+        float leaf[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) leaf[w] = leaf_values[origin[w] + int32_t(at[w])];
+#pragma unroll
+        for (int w = 0; w < W; ++w) sum.add(leaf[w]);
+      };
+      int32_t t = 0;
+      for (; t + kWalk <= trees; t += kWalk) some(t, std::integral_constant<int, kWalk>{});
+      if (pairs && t + 2 <= trees) {
+        some(t, std::integral_constant<int, 2>{});
+        t += 2;
+      }
+      for (; t < trees; ++t) some(t, std::integral_constant<int, 1>{});
+    } else {
+      for (int32_t t = 0; t < trees; ++t) sum.add(walk(nodes + tree_ptr[t], value));
+    }
+    sum.finish();
+  }
 }
 
 // m + leaves[0] + leaves[R] + ... in that order, n of them, with the LDS reads of
@@ -528,14 +578,48 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   DP_HIP(hipGetDevice(&dev));
   DP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const auto* packed = reinterpret_cast<const PackedNode*>(forest.nodes.p);
-  // A row per thread when the rows fill the chip with workgroups of at least 256
-  // and their values fit LDS beside a batch of nodes.
+  const auto* general = reinterpret_cast<const PredNode*>(forest.nodes.p);
+  // A row per thread in LDS when the rows fill the chip with workgroups of at least
+  // 256 and their values fit LDS beside a batch of nodes.
   int R = kPredThreads;
   auto rows_lds = [&](int rows) {
     return sizeof(PackedNode) * kPredBatchNodes + sizeof(float) * size_t(rows) * n_features;
   };
   while (R > 256 && (rows_lds(R) > kPredLds || n_rows < int64_t(R) * cus)) R /= 2;
-  if (forest.batches > 0 && n_rows >= int64_t(R) * cus && rows_lds(R) <= kPredLds) {
+  const bool in_rows =
+      forest.batches > 0 && n_rows >= int64_t(R) * cus && rows_lds(R) <= kPredLds;
+  // Small forests straight from global memory: copying rows to LDS costs more than the
+  // few values they read (us, in LDS and direct: 1M x 120 x 1 tree of depth 1 378 and
+  // 22, 1M x 28 x 4 of depth 1 53 and 20 but x 8 of depth 6 66 and 112; 60k x 28 x 4 of
+  // depth 6 16 and 6; 1,000 x 28 x 4 6.2 and 5.2, x 16 6.1 and 13).
+  // What decides is the chain of dependent reads, kWalk trees at a time (general nodes
+  // one): more rows hide a longer one, wider rows make the copy it spares larger; and
+  // for rows in plenty that are too wide for a row per thread, the values read.
+  const int64_t visits = int64_t(forest.trees) * std::max(forest.depth, 1);
+  const int64_t extra = forest.groups - 1;
+  const int64_t chain = int64_t(forest.packed ? (forest.trees + kWalk - 1) / kWalk : forest.trees) *
+                        (forest.depth + 1);
+  const bool direct = !forest.packed || n_rows <= 8192 ? chain + 2 * extra <= 12
+                      : in_rows ? chain <= (n_rows < 500000 ? 7 : 4) + n_features / 20
+                      : n_rows < 100000                ? chain + extra <= 20
+                                                       : visits + extra <= 30 + n_features / 18;
+  if (direct) {
+    // Two walks at once evict each other's lines of wide rows: 200k x 120 x 2 trees of
+    // depth 9 58 us against 49 one by one; 1M x 28 85 against 229.
+    const bool pairs = n_rows < 100000 || n_features < 100;
+    auto run = [&](auto kernel, const auto* nodes) {
+      hipLaunchKernelGGL(kernel, dim3(grid_for(n_rows, kDirectThreads, 16384)),
+                         dim3(kDirectThreads), 0, s, values, n_rows, row_stride, missing, nodes,
+                         forest.leaf_values.p, forest.tree_ptr.p, forest.tree_base.p,
+                         forest.group_ptr.p, forest.groups, forest.trees, forest.depth,
+                         forest.base.p, transform, pairs, out);
+      DP_HIP(hipGetLastError());
+    };
+    if (forest.packed) run(predict_direct_kernel<PackedNode>, packed);
+    else run(predict_direct_kernel<PredNode>, general);
+    return;
+  }
+  if (in_rows) {
     const auto kernel = R == 1024  ? predict_rows_kernel<1024>
                         : R == 512 ? predict_rows_kernel<512>
                                    : predict_rows_kernel<256>;
@@ -555,10 +639,11 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   while (rows < 256 && n_rows > int64_t(rows) * cus * 2 &&
          (rows < 32 || int64_t(forest.trees) * rows < int64_t(kPredThreads) * kWalk))
     rows *= 2;
-  // Values in LDS where they fit, unless the few trees read fewer of them than a
-  // row holds: half a CU's LDS and threads, so that one workgroup stages its rows
-  // while another walks; all of it for rows too wide for that.
-  bool stage = int64_t(forest.trees) * 128 >= n_features;
+  // Values in LDS where they fit, unless the trees read few of a row's (every one
+  // its own line; 20k x 5,000 x 64 trees of depth 1 29 us against 295): half a CU's
+  // LDS and threads, so that one workgroup stages its rows while another walks; all
+  // of it for rows too wide for that.
+  bool stage = visits * 8 >= n_features;
   auto lds_of = [&](int rows, int threads) {
     return sizeof(float) * (2 * kWalk * size_t(threads) +
                             size_t(rows) * size_t(part_stride(forest.groups) +
@@ -577,8 +662,12 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
       rows = full;
     }
   }
+  // Threads for every tree and row, and for staging a row's pieces in one pass each
+  // (one wavefront per 64 rows took 143 us for 60k x 784 x 8 trees, enough of them 69).
+  const int64_t pieces = stage ? int64_t(rows) * ((n_features + 511) / 512) : 0;
   int threads = 64;
-  while (threads < most && threads < int64_t(forest.trees) * rows) threads *= 2;
+  while (threads < most && threads < std::max<int64_t>(int64_t(forest.trees) * rows, 64 * pieces))
+    threads *= 2;
   threads = std::max(threads, rows);
   const size_t lds =
       lds_of(rows, threads) - (stage ? 0 : sizeof(float) * size_t(rows) * size_t(n_features | 1));
@@ -591,7 +680,6 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
                        forest.depth, forest.base.p, transform, rows, out);
     DP_HIP(hipGetLastError());
   };
-  const auto* general = reinterpret_cast<const PredNode*>(forest.nodes.p);
   if (forest.packed && stage) run(predict_trees_kernel<PackedNode, true>, packed);
   else if (forest.packed) run(predict_trees_kernel<PackedNode, false>, packed);
   else if (stage) run(predict_trees_kernel<PredNode, true>, general);

@@ -72,10 +72,22 @@ def _margins(forest, x, classes):
     (9000, 784, 120, 6, 1.0, 10),    # wide rows, nodes and rows in LDS
     (700, 9, 3, 4, 1.0, 11),         # outputs spread over a row's lanes, several passes
     (300, 12, 2, 3, 1.0, 65),        # more outputs than are spread
-    (2000, 5000, 12, 7, 1.0, 1),     # rows too wide for many in LDS
+    (2000, 5000, 100, 7, 1.0, 1),    # rows too wide for many in LDS
+    (2000, 5000, 12, 7, 1.0, 1),     # rows not worth staging
+    (20000, 9, 40, 5, 1.0, 1),       # more threads to stage the rows than to walk them
     (40, 17000, 3, 4, 1.0, 1),       # features beyond the packed nodes
     (300, 7, 2, 17, 0.995, 1),       # trees beyond the packed nodes
-    (50, 60000, 1, 2, 1.0, 1),       # rows not worth staging
+    (50, 60000, 1, 2, 1.0, 1),       # small forests, general nodes
+    (9000, 17000, 2, 3, 1.0, 1),
+    (8192, 28, 11, 3, 1.0, 1),       # small forests: quads, a pair and a single tree
+    (8193, 28, 7, 6, 0.9, 1),
+    (8192, 28, 12, 3, 1.0, 1),       # and the first that is not one
+    (66000, 120, 2, 6, 1.0, 3),      # against rows in LDS
+    (66000, 20, 4, 4, 1.0, 1),
+    (66000, 20, 5, 4, 1.0, 1),
+    (100000, 130, 3, 6, 1.0, 1),     # a pair one by one
+    (99999, 130, 16, 4, 1.0, 1),     # the longest chain that is direct
+    (5000000, 3, 1, 3, 1.0, 1),      # more rows than the grid has threads
 ])
 def test_margins_match_a_numpy_walk(dp, device, rows, features, trees, depth, full, classes):
     import torch
@@ -101,14 +113,17 @@ def test_margins_match_a_numpy_walk(dp, device, rows, features, trees, depth, fu
                                   _margins(forest, x, classes).view(np.uint32))
 
 
-@pytest.mark.parametrize("rows,classes", [(1, 3), (2049, 10), (77, 64), (77, 65)])
-def test_outputs_of_the_margins(dp, device, rows, classes):
+@pytest.mark.parametrize("rows,classes,rounds,depth", [
+    (1, 3, 3, 4), (2049, 10, 3, 4), (77, 64, 3, 4), (77, 65, 3, 4),
+    (300, 3, 1, 2),      # a small forest
+    (70001, 3, 12, 4)])  # a row per thread in LDS
+def test_outputs_of_the_margins(dp, device, rows, classes, rounds, depth):
     """Probabilities and class ids follow from the margins: each operation of the softmax rounds
     once (2^-24), a sum of K positive terms at most K times, the exponential within 2 ulp."""
     import torch
 
     rng = np.random.default_rng(rows * classes)
-    forest = _forest(rng, 3 * classes, 4, 6, 0.9)
+    forest = _forest(rng, rounds * classes, depth, 6, 0.9)
     x = torch.as_tensor(rng.normal(size=(rows, 6)).astype(np.float32), device=device)
     margins = _margins(forest, x.cpu().numpy(), classes)
     p = np.exp(margins.astype(np.float64) - margins.max(axis=1, keepdims=True))
@@ -162,3 +177,17 @@ def test_nodes_without_or_with_two_parents(dp, device, rows, trees, shape):
     x[rng.random(x.shape) < 0.2] = np.nan
     got = bst.predict(torch.as_tensor(x, device=device), margin=True).cpu().numpy()
     np.testing.assert_array_equal(got.view(np.uint32), _margins(forest, x, 1).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,trees", [(500, 3), (500, 60), (70001, 60)])
+def test_logistic_outputs_of_the_margins(dp, device, rows, trees):
+    """1 / (1 + exp(-margin)) in each kernel: three roundings and an exponential within 2 ulp."""
+    import torch
+
+    rng = np.random.default_rng(rows + trees)
+    forest = _forest(rng, trees, 4, 6, 0.9)
+    x = torch.as_tensor(rng.normal(size=(rows, 6)).astype(np.float32), device=device)
+    bst = dp.Booster.from_buffer(_model(forest, 6, 1, "binary:logistic"))
+    m = bst.predict(x, margin=True).cpu().numpy().astype(np.float64).reshape(rows)
+    np.testing.assert_allclose(bst.predict(x).cpu().numpy().reshape(rows), 1 / (1 + np.exp(-m)),
+                               rtol=8 * 2.0 ** -24)
