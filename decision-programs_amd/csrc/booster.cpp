@@ -1545,16 +1545,11 @@ void Booster::upload_forest(int32_t tree_begin, int32_t tree_end) {
   if (forest_begin_ == tree_begin && forest_end_ == tree_end && forest_trees_ == trees_.size())
     return;
   std::vector<ForestTree> trees;
+  trees.reserve(size_t(tree_end - tree_begin));
   for (int32_t t = tree_begin; t < tree_end; ++t) {
     const Tree& tr = trees_[size_t(t)];
-    ForestTree f;
-    f.group = tree_info_[size_t(t)];
-    for (int32_t i = 0; i < tr.size(); ++i) {
-      const bool leaf = tr.left[size_t(i)] == -1;
-      f.nodes.push_back({leaf ? -1 : tr.left[size_t(i)], leaf ? 0 : tr.feature[size_t(i)],
-                         tr.cond[size_t(i)], leaf ? 0 : int32_t(tr.default_left[size_t(i)])});
-    }
-    trees.push_back(std::move(f));
+    trees.push_back({tr.left.data(), tr.feature.data(), tr.cond.data(), tr.default_left.data(),
+                     tr.size(), tree_info_[size_t(t)]});
   }
   std::vector<float> base(size_t(std::max(n_groups_, 1)));
   for (size_t k = 0; k < base.size(); ++k) {

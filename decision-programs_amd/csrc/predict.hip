@@ -34,6 +34,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <memory>
 #include <type_traits>
 
 namespace dp {
@@ -460,114 +462,191 @@ void allow_lds(const void* kernel) {
 
 }  // namespace
 
+namespace {
+
+// What pack_tree knows of a node, in a word (a tree's stay in the L1 or L2): bits 0-13
+// its parent's feature, 14-28 its level (a tree of 65,536 nodes has at most 32,768),
+// 29 and 30 whether it changes places with the node before or after it, 31 set once
+// its parent is seen.
+constexpr uint32_t kReached = 1u << 31, kUp = 1u << 30, kDown = 1u << 29;
+constexpr int kLevelShift = 14;
+
+// The float above x (not +infinity, not NaN).
+float float_above(float x) {
+  uint32_t b;
+  std::memcpy(&b, &x, sizeof b);
+  b = (b & 0x7fffffffu) == 0u ? 1u : b + 1u - 2u * (b >> 31);  // no branch: signs are random
+  std::memcpy(&x, &b, sizeof b);
+  return x;
+}
+
+// A tree's packed nodes and leaf values, indices counted from `at`; false where it
+// takes the general form.  Children follow their parents.  Pruned models keep nodes
+// that no parent names: no row reaches them.  A pair of children has one order, its
+// parent's, so two parents must not name one.
+bool pack_tree(const ForestTree& t, uint32_t at, std::vector<uint32_t>& state, PackedNode* nodes,
+               float* leaves, int32_t& depth) {
+  std::fill_n(state.begin(), t.size, 0u);
+  state[0] = kReached;
+  uint32_t deepest = 0;
+  for (int32_t i = 0; i < t.size; ++i) {
+    const uint32_t s = state[size_t(i)];
+    const int32_t left = t.left[i];
+    const int32_t place = i + int32_t(s >> 30 & 1) - int32_t(s >> 29 & 1);
+    if (left == -1 || !(s & kReached)) {
+      nodes[place] = {std::nanf(""), (at + uint32_t(place)) | (s & 0x3fffu) << 17};
+      leaves[place] = t.cond[i];
+      continue;
+    }
+    const float cond = t.cond[i];
+    const bool swap = !(t.default_left[i] & 1);  // missing values go right: that child first
+    uint32_t *a = &state[size_t(left)], *b = a + 1;
+    if (std::isnan(cond) || (swap && cond == -INFINITY) || (*a | *b) & kReached) return false;
+    const uint32_t feature = uint32_t(t.feature[i]);
+    const uint32_t child =
+        kReached | ((s & (0x7fffu << kLevelShift)) + (1u << kLevelShift)) | feature;
+    *a = child | (swap ? kUp : 0u);
+    *b = child | (swap ? kDown : 0u);
+    deepest = std::max(deepest, child);
+    nodes[place] = {swap ? float_above(-cond) : cond,
+                    (at + uint32_t(left)) | feature << 17 | (swap ? 0x80000000u : 0u)};
+    leaves[place] = 0.0f;
+  }
+  depth = std::max(depth, int32_t(deepest >> kLevelShift & 0x7fffu));
+  return true;
+}
+
+void copy_tree(const ForestTree& t, std::vector<uint32_t>& level, PredNode* nodes,
+               int32_t& depth) {
+  std::fill_n(level.begin(), t.size, 0u);
+  for (int32_t i = 0; i < t.size; ++i) {
+    const bool leaf = t.left[i] == -1;
+    nodes[i] = {leaf ? -1 : t.left[i], leaf ? 0 : t.feature[i], t.cond[i],
+                leaf ? 0 : int32_t(t.default_left[i] & 1)};
+    if (leaf) continue;
+    const uint32_t below = level[size_t(i)] + 1;
+    for (int32_t c = t.left[i]; c <= t.left[i] + 1; ++c)
+      level[size_t(c)] = std::max(level[size_t(c)], below);
+    depth = std::max(depth, int32_t(below));
+  }
+}
+
+}  // namespace
+
+// Host work and transfers decide a first prediction: every table's size is known
+// before the nodes are looked at, so they are written once, into one buffer that one
+// copy takes.  First predictions of a loaded model with vectors per tree and table and
+// ten copies, and now (us): 64 rows, 100 trees of depth 8 727 and 341; 30 of depth 13
+// 3,584 and 1,600; one row, 10 of depth 6 257 and 101.
 void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>& base,
                   int32_t n_features, Forest& out) {
-  const int32_t groups = int32_t(base.size());
-  std::vector<std::vector<const ForestTree*>> by_group(static_cast<size_t>(groups));
+  const size_t n_trees = trees.size(), groups = base.size();
+  std::vector<int32_t> group_ptr(groups + 1, 0), order(n_trees);
   size_t total = 0;
-  bool packed = n_features <= (1 << 14), batched = true;
-  out.depth = 0;
+  int32_t largest = 1;
   for (const ForestTree& t : trees) {
-    by_group[size_t(t.group)].push_back(&t);
-    total += t.nodes.size();
-    packed = packed && t.nodes.size() <= (size_t(1) << 16);
-    batched = batched && t.nodes.size() <= size_t(kPredBatchNodes);
-    // Nodes that rows reach (children follow their parents; pruned models keep
-    // nodes that no parent names).  Packed, a pair of children has one order, its
-    // parent's: a pair that two parents name takes the general form.
-    std::vector<int32_t> level(t.nodes.size(), -1);
-    level[0] = 0;
-    for (size_t i = 0; i < t.nodes.size(); ++i) {
-      const PredNode& n = t.nodes[i];
-      if (n.left < 0 || level[i] < 0) continue;
-      packed = packed && !std::isnan(n.cond) && (n.flags & 1 || n.cond != -INFINITY);
-      for (size_t c = size_t(n.left); c <= size_t(n.left) + 1; ++c) {
-        packed = packed && level[c] < 0;
-        level[c] = std::max(level[c], level[i] + 1);
-        out.depth = std::max(out.depth, level[c]);
-      }
-    }
+    ++group_ptr[size_t(t.group) + 1];
+    total += size_t(t.size);
+    largest = std::max(largest, t.size);
   }
   need(total < size_t(INT32_MAX), "forest has too many nodes");
-  packed = packed && total < (size_t(1) << 29);
-  std::vector<int32_t> tree_ptr{0}, tree_base, group_ptr{0}, batch_tree{0};
-  std::vector<PackedNode> small;
-  std::vector<PredNode> general;
-  std::vector<float> leaves;
-  int32_t n = 0, batch = 0;  // nodes so far; the first node of the batch
-  for (const auto& group : by_group) {
-    for (const ForestTree* t : group) {
-      const int32_t size = int32_t(t->nodes.size());
-      // Packed indices count from the batch (a large tree: from itself).
-      if (n > batch && n + size - batch > kPredBatchNodes) {
-        batch = n;
-        batch_tree.push_back(int32_t(tree_ptr.size()) - 1);
-      }
-      if (!packed) general.insert(general.end(), t->nodes.begin(), t->nodes.end());
-      if (packed) {
-        // Node i's place: children that missing values enter on the right swap.
-        // -1: no row reaches it.
-        std::vector<int32_t> place(static_cast<size_t>(size), -1);
-        place[0] = 0;
-        for (int32_t i = 0; i < size; ++i) {
-          const PredNode& nd = t->nodes[size_t(i)];
-          if (nd.left < 0 || place[size_t(i)] < 0) continue;
-          const int32_t second = nd.flags & 1 ? 1 : 0;  // the right child's place in the pair
-          place[size_t(nd.left)] = nd.left + 1 - second;
-          place[size_t(nd.left) + 1] = nd.left + second;
-        }
-        small.resize(size_t(n) + size_t(size));
-        leaves.resize(small.size());
-        const uint32_t at = uint32_t(n - batch);
-        for (int32_t i = 0; i < size; ++i) {
-          if (place[size_t(i)] < 0) continue;
-          const PredNode& nd = t->nodes[size_t(i)];
-          PackedNode& out_node = small[size_t(n + place[size_t(i)])];
-          leaves[size_t(n + place[size_t(i)])] = nd.left < 0 ? nd.cond : 0.0f;
-          if (nd.left < 0)
-            out_node = {std::nanf(""), at + uint32_t(place[size_t(i)])};
-          else
-            out_node = {nd.flags & 1 ? nd.cond : std::nextafterf(-nd.cond, INFINITY),
-                        (at + uint32_t(nd.left)) | uint32_t(nd.feature) << 17 |
-                            (nd.flags & 1 ? 0u : 0x80000000u)};
-        }
-      }
-      tree_base.push_back(batch);
-      n += size;
-      tree_ptr.push_back(n);
+  for (size_t g = 0; g < groups; ++g) group_ptr[g + 1] += group_ptr[g];
+  {
+    std::vector<int32_t> next(group_ptr);
+    for (size_t t = 0; t < n_trees; ++t) order[size_t(next[size_t(trees[t].group)]++)] = int32_t(t);
+  }
+  // Packed indices count from the batch (a large tree: from itself).
+  std::vector<int32_t> tree_ptr(n_trees + 1, 0), tree_base(n_trees), batch_tree{0}, quad_ptr{0};
+  size_t quads = 0;
+  int32_t batch = 0;
+  for (size_t k = 0; k < n_trees; ++k) {
+    const int32_t n = tree_ptr[k], size = trees[size_t(order[k])].size;
+    if (n > batch && n + size - batch > kPredBatchNodes) {
+      batch = n;
+      batch_tree.push_back(int32_t(k));
     }
-    group_ptr.push_back(int32_t(tree_ptr.size()) - 1);
+    tree_base[k] = batch;
+    tree_ptr[k + 1] = n + size;
   }
-  out.trees = int32_t(tree_ptr.size()) - 1;
-  out.groups = groups;
-  out.packed = packed;
-  if (batch_tree.back() != out.trees) batch_tree.push_back(out.trees);
-  out.batches = packed && batched ? int32_t(batch_tree.size()) - 1 : 0;
-  std::vector<int32_t> batch_node{0}, quad_ptr{0}, quads;
-  for (int32_t b = 0; b < out.batches; ++b) {
-    const int32_t t0 = batch_tree[size_t(b)], t1 = batch_tree[size_t(b) + 1];
-    for (int32_t t = t0; t < t1 || (t - t0) % 4 != 0; ++t)
-      quads.push_back(tree_ptr[size_t(std::min(t, t1 - 1))] - tree_ptr[size_t(t0)]);
-    quad_ptr.push_back(int32_t(quads.size()) / 4);
-    batch_node.push_back(tree_ptr[size_t(t1)]);
+  if (n_trees) batch_tree.push_back(int32_t(n_trees));
+  for (size_t b = 0; b + 1 < batch_tree.size(); ++b) {
+    quads += size_t(batch_tree[b + 1] - batch_tree[b] + 3) / 4;
+    quad_ptr.push_back(int32_t(quads));
   }
-  quads.insert(quads.end(), 4, 0);
-  auto put = [](auto& dst, const auto& src) {
-    const size_t bytes = src.size() * sizeof(src[0]);
-    dst.resize(std::max<size_t>(bytes, 16) / sizeof(*dst.p));
-    if (bytes) DP_HIP(hipMemcpy(dst.p, src.data(), bytes, hipMemcpyHostToDevice));
+  bool packed = n_features <= (1 << 14) && largest <= (1 << 16) && total < (size_t(1) << 29);
+  const bool batched = largest <= kPredBatchNodes;
+  // Tables at multiples of 16 bytes.
+  size_t bytes = 0;
+  auto take = [&](size_t n) {
+    const size_t at = bytes;
+    bytes += (std::max<size_t>(n, 1) + 15) / 16 * 16;
+    return at;
   };
-  if (packed) put(out.nodes, small);
-  else put(out.nodes, general);
-  put(out.leaf_values, leaves);
-  put(out.tree_ptr, tree_ptr);
-  put(out.tree_base, tree_base);
-  put(out.group_ptr, group_ptr);
-  put(out.batch_node, batch_node);
-  put(out.batch_tree, batch_tree);
-  put(out.quad_ptr, quad_ptr);
-  put(out.quads, quads);
-  put(out.base, base);
+  const size_t small = sizeof(int32_t);
+  const size_t at_tree_ptr = take(tree_ptr.size() * small), at_tree_base = take(n_trees * small),
+               at_group_ptr = take(group_ptr.size() * small), at_base = take(groups * small),
+               at_batch_node = take(batch_tree.size() * small),
+               at_batch_tree = take(batch_tree.size() * small),
+               at_quad_ptr = take(quad_ptr.size() * small), at_quads = take((quads + 1) * 4 * small),
+               at_leaves = take(packed ? total * sizeof(float) : 0),
+               at_nodes = take(total * (packed ? sizeof(PackedNode) : sizeof(PredNode)));
+  std::unique_ptr<uint8_t[]> host(new uint8_t[bytes]);  // not cleared
+  std::vector<uint32_t> state(static_cast<size_t>(largest));
+  int32_t depth = 0;
+  if (packed) {
+    auto* nodes = reinterpret_cast<PackedNode*>(host.get() + at_nodes);
+    auto* leaves = reinterpret_cast<float*>(host.get() + at_leaves);
+    for (size_t k = 0; packed && k < n_trees; ++k)
+      packed = pack_tree(trees[size_t(order[k])], uint32_t(tree_ptr[k] - tree_base[k]), state,
+                         nodes + tree_ptr[k], leaves + tree_ptr[k], depth);
+    if (!packed) {  // rare: the nodes take twice the room
+      bytes = at_nodes;
+      take(total * sizeof(PredNode));
+      host.reset(new uint8_t[bytes]);
+      depth = 0;
+    }
+  }
+  if (!packed) {
+    auto* nodes = reinterpret_cast<PredNode*>(host.get() + at_nodes);
+    for (size_t k = 0; k < n_trees; ++k)
+      copy_tree(trees[size_t(order[k])], state, nodes + tree_ptr[k], depth);
+  }
+  auto put = [&](size_t at, const auto& src) {
+    std::copy(src.begin(), src.end(), reinterpret_cast<std::decay_t<decltype(src[0])>*>(host.get() + at));
+  };
+  put(at_tree_ptr, tree_ptr);
+  put(at_tree_base, tree_base);
+  put(at_group_ptr, group_ptr);
+  put(at_base, base);
+  put(at_batch_tree, batch_tree);
+  put(at_quad_ptr, quad_ptr);
+  auto* batch_node = reinterpret_cast<int32_t*>(host.get() + at_batch_node);
+  auto* quad = reinterpret_cast<int32_t*>(host.get() + at_quads);
+  for (size_t b = 0; b < batch_tree.size(); ++b) batch_node[b] = tree_ptr[size_t(batch_tree[b])];
+  for (size_t b = 0; b + 1 < batch_tree.size(); ++b) {
+    const int32_t t0 = batch_tree[b], t1 = batch_tree[b + 1];
+    for (int32_t t = t0; t < t1 || (t - t0) % 4 != 0; ++t)
+      *quad++ = tree_ptr[size_t(std::min(t, t1 - 1))] - tree_ptr[size_t(t0)];
+  }
+  std::fill_n(quad, 4, 0);
+  out.block.resize(bytes);
+  DP_HIP(hipMemcpy(out.block.p, host.get(), bytes, hipMemcpyHostToDevice));
+  auto words = [&](size_t at) { return reinterpret_cast<const int32_t*>(out.block.p + at); };
+  out.nodes = out.block.p + at_nodes;
+  out.leaf_values = reinterpret_cast<const float*>(out.block.p + at_leaves);
+  out.tree_ptr = words(at_tree_ptr);
+  out.tree_base = words(at_tree_base);
+  out.group_ptr = words(at_group_ptr);
+  out.base = reinterpret_cast<const float*>(out.block.p + at_base);
+  out.batch_node = words(at_batch_node);
+  out.batch_tree = words(at_batch_tree);
+  out.quad_ptr = words(at_quad_ptr);
+  out.quads = words(at_quads);
+  out.packed = packed;
+  out.trees = int32_t(n_trees);
+  out.groups = int32_t(groups);
+  out.batches = packed && batched ? int32_t(batch_tree.size()) - 1 : 0;
+  out.depth = depth;
 }
 
 void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int64_t row_stride,
@@ -577,8 +656,8 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   int dev = 0, cus = 0;
   DP_HIP(hipGetDevice(&dev));
   DP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const auto* packed = reinterpret_cast<const PackedNode*>(forest.nodes.p);
-  const auto* general = reinterpret_cast<const PredNode*>(forest.nodes.p);
+  const auto* packed = static_cast<const PackedNode*>(forest.nodes);
+  const auto* general = static_cast<const PredNode*>(forest.nodes);
   // A row per thread in LDS when the rows fill the chip with workgroups of at least
   // 256 and their values fit LDS beside a batch of nodes.
   int R = kPredThreads;
@@ -610,9 +689,9 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
     auto run = [&](auto kernel, const auto* nodes) {
       hipLaunchKernelGGL(kernel, dim3(grid_for(n_rows, kDirectThreads, 16384)),
                          dim3(kDirectThreads), 0, s, values, n_rows, row_stride, missing, nodes,
-                         forest.leaf_values.p, forest.tree_ptr.p, forest.tree_base.p,
-                         forest.group_ptr.p, forest.groups, forest.trees, forest.depth,
-                         forest.base.p, transform, pairs, out);
+                         forest.leaf_values, forest.tree_ptr, forest.tree_base,
+                         forest.group_ptr, forest.groups, forest.trees, forest.depth,
+                         forest.base, transform, pairs, out);
       DP_HIP(hipGetLastError());
     };
     if (forest.packed) run(predict_direct_kernel<PackedNode>, packed);
@@ -626,10 +705,10 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
     allow_lds(reinterpret_cast<const void*>(kernel));
     hipLaunchKernelGGL(kernel, dim3(unsigned((n_rows + R - 1) / R)), dim3(R), rows_lds(R), s,
                        values, n_rows, n_features, row_stride, missing, packed,
-                       forest.leaf_values.p, forest.batch_node.p, forest.batch_tree.p,
-                       forest.quad_ptr.p, reinterpret_cast<const int4*>(forest.quads.p),
-                       forest.batches, forest.group_ptr.p, forest.groups, forest.depth,
-                       forest.base.p, transform, out);
+                       forest.leaf_values, forest.batch_node, forest.batch_tree,
+                       forest.quad_ptr, reinterpret_cast<const int4*>(forest.quads),
+                       forest.batches, forest.group_ptr, forest.groups, forest.depth,
+                       forest.base, transform, out);
     DP_HIP(hipGetLastError());
     return;
   }
@@ -675,9 +754,9 @@ void launch_predict(const float* values, int64_t n_rows, int32_t n_features, int
   auto run = [&](auto kernel, const auto* nodes) {
     allow_lds(reinterpret_cast<const void*>(kernel));
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, values, n_rows, n_features,
-                       row_stride, missing, nodes, forest.leaf_values.p, forest.tree_ptr.p,
-                       forest.tree_base.p, forest.group_ptr.p, forest.groups, forest.trees,
-                       forest.depth, forest.base.p, transform, rows, out);
+                       row_stride, missing, nodes, forest.leaf_values, forest.tree_ptr,
+                       forest.tree_base, forest.group_ptr, forest.groups, forest.trees,
+                       forest.depth, forest.base, transform, rows, out);
     DP_HIP(hipGetLastError());
   };
   if (forest.packed && stage) run(predict_trees_kernel<PackedNode, true>, packed);

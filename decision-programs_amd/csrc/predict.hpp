@@ -33,7 +33,8 @@ struct PredNode {
 //   missing right   children (right, left), sign, cond the float above -t:
 //                   -x >= cond exactly when x < t
 //   leaf            its own index, cond NaN: every row stays; its value is in
-//                   Forest::leaf_values
+//                   Forest::leaf_values, its feature its parent's (a lane at its leaf
+//                   before the others reads a value that it has read before)
 // Forests of at most 16,384 features, 65,536 nodes a tree, one parent for each
 // node that rows reach and no threshold that would make a NaN take it.
 struct alignas(8) PackedNode {
@@ -42,21 +43,23 @@ struct alignas(8) PackedNode {
 };
 
 // A forest laid out for prediction: trees grouped by output, in boosting order
-// within each.
+// within each.  One block and one copy: a program that loads a model to predict
+// once waits for both.
 struct Forest {
-  PooledBuffer<uint8_t> nodes;       // PackedNode or PredNode
-  PooledBuffer<float> leaf_values;   // packed: [nodes] a leaf's value
-  PooledBuffer<int32_t> tree_ptr;    // [trees + 1] first node of each tree
-  PooledBuffer<int32_t> tree_base;   // [trees] the node that the tree's indices count from
-  PooledBuffer<int32_t> group_ptr;   // [groups + 1] first tree of each output
+  PooledBuffer<uint8_t> block;  // the tables below
+  const void* nodes = nullptr;            // PackedNode or PredNode
+  const float* leaf_values = nullptr;     // packed: [nodes] a leaf's value
+  const int32_t* tree_ptr = nullptr;      // [trees + 1] first node of each tree
+  const int32_t* tree_base = nullptr;     // [trees] the node that the tree's indices count from
+  const int32_t* group_ptr = nullptr;     // [groups + 1] first tree of each output
+  const float* base = nullptr;            // [groups] margin before the first tree
   // Batches of trees whose nodes fit kPredBatchNodes: their first nodes, and per
   // batch the trees' first nodes, counted from the batch, in groups of four (the
   // last group repeats the last tree), quad_ptr[b] .. quad_ptr[b + 1] of them.
-  PooledBuffer<int32_t> batch_node;  // [batches + 1]
-  PooledBuffer<int32_t> quad_ptr;    // [batches + 1]
-  PooledBuffer<int32_t> quads;       // [groups of four][4]
-  PooledBuffer<int32_t> batch_tree;  // [batches + 1] first tree
-  PooledBuffer<float> base;          // [groups] margin before the first tree
+  const int32_t* batch_node = nullptr;    // [batches + 1]
+  const int32_t* batch_tree = nullptr;    // [batches + 1] first tree
+  const int32_t* quad_ptr = nullptr;      // [batches + 1]
+  const int32_t* quads = nullptr;         // [groups of four + 1][4]
   bool packed = false;
   int32_t trees = 0, groups = 1;
   int32_t batches = 0;  // 0: some tree alone exceeds kPredBatchNodes (or is not packed)
@@ -65,10 +68,13 @@ struct Forest {
 
 constexpr int32_t kPredBatchNodes = 4096;
 
-// Host-side description of one tree for build_forest.
+// One tree for build_forest: node arrays, children after their parents, left -1 for a
+// leaf (cond its value), right = left + 1.
 struct ForestTree {
-  int32_t group;
-  std::vector<PredNode> nodes;
+  const int32_t *left, *feature;
+  const float* cond;
+  const uint8_t* default_left;
+  int32_t size, group;
 };
 // trees: in boosting order.
 void build_forest(const std::vector<ForestTree>& trees, const std::vector<float>& base,

@@ -191,3 +191,48 @@ def test_logistic_outputs_of_the_margins(dp, device, rows, trees):
     m = bst.predict(x, margin=True).cpu().numpy().astype(np.float64).reshape(rows)
     np.testing.assert_allclose(bst.predict(x).cpu().numpy().reshape(rows), 1 / (1 + np.exp(-m)),
                                rtol=8 * 2.0 ** -24)
+
+
+SPECIALS = np.float32([np.inf, -np.inf, 3.4028235e38, -3.4028235e38, 1e-45, -1e-45, 0.0, -0.0,
+                       1.1754944e-38, -1.1754944e-38, 1.0])
+
+
+@pytest.mark.parametrize("rows,trees", [(300, 2), (300, 40), (70001, 40)])
+@pytest.mark.parametrize("general", ["none", "infinity", "nan"])
+def test_thresholds_at_the_ends_of_the_floats(dp, device, rows, trees, general):
+    """Packed, missing-right nodes compare -x with the float above -t.  A threshold of -inf with
+    missing values right, or of NaN, takes the general nodes."""
+    import torch
+
+    rng = np.random.default_rng(rows + trees)
+    forest = _forest(rng, trees, 5, 7, 1.0)
+    for left, _, cond, default in forest:
+        inner = left >= 0
+        cond[inner] = rng.choice(SPECIALS, inner.sum())
+        if general == "nan":
+            cond[inner & (rng.random(len(left)) < 0.2)] = np.nan
+        elif general == "none":
+            default[inner & (cond == -np.inf)] = 1
+    bst = dp.Booster.from_buffer(_model(forest, 7, 1))
+    x = rng.choice(np.append(SPECIALS, np.float32([np.nan, 2.0, -2.0])), (rows, 7))
+    x = x.astype(np.float32)
+    got = bst.predict(torch.as_tensor(x, device=device), margin=True).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), _margins(forest, x, 1).view(np.uint32))
+
+
+@pytest.mark.parametrize("splits,rows", [(2047, 40), (32767, 40)])
+def test_a_tree_as_deep_as_packed_nodes_count(dp, device, splits, rows):
+    import torch
+
+    n = 2 * splits + 1
+    inner = np.arange(n) % 2 == 0
+    inner[-1] = False
+    left = np.where(inner, np.arange(n) + 1, -1)
+    cond = np.where(inner, np.arange(n) / n, np.arange(n) % 100).astype(np.float32)
+    forest = [(left, np.where(inner, np.arange(n) % 3, 0), cond, (np.arange(n) // 2) % 2)]
+    rng = np.random.default_rng(splits)
+    x = np.repeat(rng.random((rows, 1)), 3, axis=1).astype(np.float32)
+    x[0], x[1, 1] = 2.0, np.nan
+    got = dp.Booster.from_buffer(_model(forest, 3, 1)).predict(
+        torch.as_tensor(x, device=device), margin=True).cpu().numpy()
+    np.testing.assert_array_equal(got.view(np.uint32), _margins(forest, x, 1).view(np.uint32))
