@@ -228,6 +228,9 @@ __global__ void copy_matrix_kernel(const float* __restrict__ src, int64_t row_st
 // thread in flight and no division of an element's place into row and feature.
 // Memory bounds it (8 B per value): 2M x 1,000 3.67 -> 3.05 ms (5.2 TB/s), 1M x 28
 // 57 -> 40 us.
+// Below a million values the other kernel's more and smaller workgroups are the faster
+// (100k x 7 4.0 us here and 3.5 there, 250k x 4 3.1 and 4.0).
+constexpr int64_t kCopyFlat = 1'000'000;
 constexpr int kCopyLoads = 4;
 constexpr int kCopyThreads = 256;
 __global__ __launch_bounds__(kCopyThreads) void copy_flat_kernel(
@@ -611,8 +614,8 @@ void launch_copy_matrix(const float* src, int64_t row_stride, int64_t n_rows, in
   launch_fill_u8(reinterpret_cast<uint8_t*>(bad), 4, 0, s);
   const int64_t total = n_rows * n_features;
   if (total <= 0) return;
-  if (row_stride == n_features && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(dst) % 16 == 0) {
+  if (total >= kCopyFlat && row_stride == n_features &&
+      reinterpret_cast<uintptr_t>(src) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0) {
     const int64_t per = int64_t(kCopyLoads) * kCopyThreads * 4;
     const int64_t blocks = std::min<int64_t>((total + per - 1) / per, 16384);
     hipLaunchKernelGGL(copy_flat_kernel, dim3(unsigned(blocks)), dim3(kCopyThreads), 0, s, reinterpret_cast<const float4*>(src), total,

@@ -57,7 +57,8 @@ def test_cuts_match_the_oracle(dp, oracle, ws, device, n, max_bin):
         assert missing == bool(np.isnan(part).any())
 
 
-@pytest.mark.parametrize("rows,features", [(1, 1), (3, 5), (256, 16), (256, 17), (241, 1003)])
+@pytest.mark.parametrize("rows,features", [(1, 1), (3, 5), (256, 16), (256, 17), (241, 1003),
+                                           (250, 4000), (255, 4113)])
 @pytest.mark.parametrize("missing", [-999.0, np.inf, -np.inf])
 def test_matrices_are_copied_whole(dp, device, rows, features, missing):
     """With at most 256 rows the cuts are the distinct values above the smallest: the copy is
