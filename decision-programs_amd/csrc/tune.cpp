@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 
@@ -91,6 +92,26 @@ double time_ms(Run&& run, hipStream_t s) {
   return double(ms) / 3.0;
 }
 
+// What the reduce-and-evaluate launches read besides the histograms: node sums of
+// zero, so that every candidate is refused at once, the same small evaluation whatever
+// the shape.
+struct EvalInputs {
+  DeviceBuffer<int32_t> nbins, exps;
+  DeviceBuffer<int64_t> sums;
+  DeviceBuffer<FeatCand> feat;
+  std::vector<int32_t> nb;  // alive until the stream has read it
+  EvalInputs(int32_t n_features, int32_t bin_stride, int32_t nodes, hipStream_t s)
+      : nbins(static_cast<size_t>(n_features)),
+        exps(2),
+        sums(2 * static_cast<size_t>(nodes)),
+        feat(static_cast<size_t>(n_features) * static_cast<size_t>(nodes)),
+        nb(static_cast<size_t>(n_features), bin_stride) {
+    DP_HIP(hipMemcpyAsync(nbins.p, nb.data(), nbins.bytes(), hipMemcpyHostToDevice, s));
+    DP_HIP(hipMemsetAsync(sums.p, 0, sums.bytes(), s));
+    DP_HIP(hipMemsetAsync(exps.p, 0, exps.bytes(), s));
+  }
+};
+
 // One timed pass: work lists of `nodes` nodes of `rows` positions each
 // (node i: [i * rows, (i + 1) * rows) of ridx) for cfg, hist + reduce.
 struct Pass {
@@ -104,7 +125,9 @@ struct Pass {
   int32_t bin_stride;
   const int32_t* gpair;
   int64_t* out;  // `nodes` node histograms
-  bool fmaj;     // the levels' feature-major partial slots (launch_hist's fmaj)
+  // The booster's launches: feature-major partial slots, reduced and evaluated in one
+  // launch; null for the operators' (LDS-image slots and the reduce alone).
+  const EvalInputs* eval;
 };
 
 double time_dense(const Pass& p, const HistConfig& cfg, hipStream_t s) {
@@ -124,12 +147,18 @@ double time_dense(const Pass& p, const HistConfig& cfg, hipStream_t s) {
   DP_HIP(hipMemcpyAsync(dj.p, j.data(), dj.bytes(), hipMemcpyHostToDevice, s));
   const double ms = time_ms(
       [&] {
-        // With fmaj the reduce below reads the slots in the other layout: its
-        // sums are discarded, its time stands for the levels' reduce.
         launch_hist(p.bins, *p.L, p.gpair, p.ridx, dw.p, int32_t(w.size()), nullptr,
-                    p.bin_stride, p.out, partial.p, s, p.rows_major, cfg, p.skip, p.fmaj);
-        launch_hist_reduce(partial.p, dj.p, p.nodes, p.L->n_tiles, p.L->n_features,
-                           p.bin_stride, p.out, false, s);
+                    p.bin_stride, p.out, partial.p, s, p.rows_major, cfg, p.skip,
+                    p.eval != nullptr);
+        if (p.eval)
+          launch_reduce_evaluate_dense(partial.p, dj.p, p.nodes, nullptr, p.L->n_tiles, 16,
+                                       p.L->n_features, p.bin_stride, nullptr, p.out,
+                                       p.eval->nbins.p, p.eval->sums.p, p.eval->exps.p,
+                                       dp_train_param{}, nullptr, nullptr, p.eval->feat.p, true,
+                                       s);
+        else
+          launch_hist_reduce(partial.p, dj.p, p.nodes, p.L->n_tiles, p.L->n_features,
+                             p.bin_stride, p.out, false, s);
       },
       s);
   DP_HIP(hipStreamSynchronize(s));  // before the buffers are freed
@@ -194,7 +223,9 @@ const HistTuning& tune_dense_hist(const dp_bin_layout& L, const uint8_t* bins, b
   const auto cands = dense_candidates(L.n_tiles, true);
   constexpr int32_t kStride = 32, kNodes = 12;  // the gathered pass's nodes (see above)
   DeviceBuffer<int64_t> out(size_t(kNodes) * size_t(L.n_features) * size_t(bin_stride) * 2);
-  Pass root{&L, bins, nullptr, skip, nullptr, L.n_rows, 1, bin_stride, gpair, out.p, false};
+  std::unique_ptr<EvalInputs> eval;
+  if (gathered) eval = std::make_unique<EvalInputs>(L.n_features, bin_stride, kNodes, s);
+  Pass root{&L, bins, nullptr, skip, nullptr, L.n_rows, 1, bin_stride, gpair, out.p, eval.get()};
   std::string report = "{";
   t.root = pick(cands, [&](const HistConfig& c) { return time_dense(root, c, s); }, report,
                 "root");
@@ -223,14 +254,12 @@ const HistTuning& tune_dense_hist(const dp_bin_layout& L, const uint8_t* bins, b
       }
       return it->second.p;
     };
-    // The levels' flush layout: feature-major, as the booster's reduce and
-    // evaluation read it (it costs more per item than the LDS image).
     report += ",";
     t.level = pick(
         dense_candidates(L.n_tiles, false),
         [&](const HistConfig& c) {
           Pass level{&L,  bins,   rows_for(c), skip, ridx.p, per, kNodes, bin_stride,
-                     gpair, out.p, true};
+                     gpair, out.p, eval.get()};
           return time_dense(level, c, s);
         },
         report, "gathered", kTieShareGathered);
@@ -265,19 +294,9 @@ const HistTuning& tune_sparse_hist(const SparseBins& sp, int64_t n_rows, int32_t
   // The booster sums the root's partial slots in the launch that also evaluates
   // them; with at most 64 bins its reduce runs one workgroup per 16 features
   // (reduce_evaluate_flat_kernel), so its time grows with the slots far more than
-  // a reduce-only launch's.  The timed pass runs that
-  // launch, with node sums of zero (every candidate is refused at once, the
-  // same small evaluation for each candidate count).
+  // a reduce-only launch's.  The timed pass runs that launch.
   const bool fused = bin_stride <= 64 && sp.tile_features % 16 == 0;  // as the booster decides
-  DeviceBuffer<int32_t> nbins(static_cast<size_t>(n_features));
-  DeviceBuffer<int64_t> sums(2);
-  DeviceBuffer<int32_t> exps(2);
-  DeviceBuffer<FeatCand> feat(static_cast<size_t>(n_features));
-  // alive until the stream has read it (synchronised below)
-  const std::vector<int32_t> nb(static_cast<size_t>(n_features), bin_stride);
-  DP_HIP(hipMemcpyAsync(nbins.p, nb.data(), nbins.bytes(), hipMemcpyHostToDevice, s));
-  DP_HIP(hipMemsetAsync(sums.p, 0, sums.bytes(), s));
-  DP_HIP(hipMemsetAsync(exps.p, 0, exps.bytes(), s));
+  const EvalInputs eval(n_features, bin_stride, 1, s);
   const dp_train_param zero{};
   dp_bin_layout L{};
   L.n_rows = n_rows;
@@ -305,13 +324,13 @@ const HistTuning& tune_sparse_hist(const SparseBins& sp, int64_t n_rows, int32_t
               if (fused)
                 launch_reduce_evaluate_flat(partial.p, dj.p, 1, nullptr, sp.n_tiles,
                                             sp.tile_features, n_features, bin_stride, nullptr,
-                                            out.p, nbins.p, sums.p, exps.p, zero, nullptr,
-                                            nullptr, feat.p, true, s);
+                                            out.p, eval.nbins.p, eval.sums.p, eval.exps.p, zero,
+                                            nullptr, nullptr, eval.feat.p, true, s);
               else
                 launch_reduce_evaluate_dense(partial.p, dj.p, 1, nullptr, sp.n_tiles,
                                              sp.tile_features, n_features, bin_stride, nullptr,
-                                             out.p, nbins.p, sums.p, exps.p, zero, nullptr,
-                                             nullptr, feat.p, true, s);
+                                             out.p, eval.nbins.p, eval.sums.p, eval.exps.p, zero,
+                                             nullptr, nullptr, eval.feat.p, true, s);
             },
             s);
         DP_HIP(hipStreamSynchronize(s));

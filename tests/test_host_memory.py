@@ -190,3 +190,26 @@ def test_kept_memory_can_be_handed_back(host):
     assert freed == before[0]
     assert after[0] == 4 * 1000 * 50  # the program's own array
     assert 4 * 10 * 5 * 2 <= after[1] <= before[1]  # a live matrix keeps its copy
+
+
+@pytest.mark.parametrize("rows,features", [(5000, 8), (5000, 40)])
+@pytest.mark.parametrize("booster", [True, False])
+def test_the_tuner_times_what_runs(host, rows, features, booster):
+    """The booster's passes end in the reduce that also evaluates, the operators' in the reduce
+    alone; the operators time the contiguous pass only."""
+    names = host(f"""
+        class Layout(ctypes.Structure):
+            _fields_ = [("rows", ctypes.c_int64), ("features", ctypes.c_int32),
+                        ("width", ctypes.c_int32), ("tiles", ctypes.c_int32),
+                        ("missing", ctypes.c_int32), ("pairs", ctypes.c_uint64)]
+        lay = Layout()
+        ok(lib.dp_layout_init(ctypes.c_int64({rows}), {features}, 0, -1, ctypes.byref(lay)))
+        p = ctypes.c_void_p()
+        ok(fake.hipMalloc(ctypes.byref(p), ctypes.c_size_t(1 << 20)))
+        tune = lib._ZN2dp15tune_dense_histERK13dp_bin_layoutPKhbiPKiP12ihipStream_tS4_
+        tune.restype = ctypes.c_void_p
+        tune(ctypes.byref(lay), p, ctypes.c_bool({booster}), 256, p, None, None)
+        print(json.dumps([x.split(" ")[0] for x in fake.fake_launches().decode().split(";") if x]))
+    """)
+    assert any("reduce_evaluate_dense" in n for n in names) == booster
+    assert any("hist_reduce" in n for n in names) != booster
