@@ -286,9 +286,6 @@ namespace dp {
 // Kernels that take (n_host, n_dev) process n_dev ? *n_dev : n_host items; the
 // host value is then an upper bound used to size a persistent grid.
 void launch_fill_i64(int64_t* p, int64_t n, int64_t value, hipStream_t s);
-// p[0 .. (*n_dev) * per) = 0, at most bound * per elements.
-void launch_zero_i64_dev(int64_t* p, const int32_t* n_dev, int64_t per, int64_t bound,
-                         hipStream_t s);
 void launch_fill_u8(uint8_t* p, int64_t n, uint8_t value, hipStream_t s);
 void launch_iota_u32(uint32_t* p, int64_t n, hipStream_t s);
 
@@ -340,7 +337,7 @@ void check_pairs(const dp_bin_layout& layout);
 // skip (matrices without missing values): per tile, the 16 features' skip
 // bins ([n_tiles][16] bytes); rows in a feature's skip bin add nothing, so that
 // bin's sums stay zero (the split evaluation restores them from the node's
-// totals: launch_evaluate's skip argument).  fmaj: partial slots are stored
+// totals: launch_reduce_evaluate_dense's skip_bins).  fmaj: partial slots are stored
 // feature-major, [16 features][bin_stride][g, h] (the node histogram's layout
 // restricted to the tile), for launch_reduce_evaluate_dense; otherwise as the
 // LDS image [bin][g of 16 features, h of 16 features] (launch_hist_reduce).

@@ -747,14 +747,6 @@ __device__ __forceinline__ long long sum_slots(const long long* __restrict__ src
   return ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
 }
 
-__global__ void zero_i64_dev_kernel(int64_t* __restrict__ p, const int32_t* __restrict__ n_dev,
-                                    int64_t per) {
-  const int64_t n = int64_t(*n_dev) * per;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += int64_t(blockDim.x) * gridDim.x)
-    p[i] = 0;
-}
-
 __global__ void subtract_kernel(const int64_t* __restrict__ parent,
                                 const int64_t* __restrict__ built, int64_t* __restrict__ sibling,
                                 int64_t n) {
@@ -1046,14 +1038,6 @@ void launch_hist(const uint8_t* bins, const dp_bin_layout& layout, const int32_t
                      layout.n_features, layout.n_tiles, gp, ridx, work, n_work, n_work_dev,
                      bin_stride, out, part, tile_step, row_step, fmaj ? 1 : 0, pairs,
                      layout.paired_tiles, joint_first);
-  DP_HIP(hipGetLastError());
-}
-
-void launch_zero_i64_dev(int64_t* p, const int32_t* n_dev, int64_t per, int64_t bound,
-                         hipStream_t s) {
-  if (bound <= 0 || per <= 0) return;
-  hipLaunchKernelGGL(zero_i64_dev_kernel, dim3(grid_for(bound * per, 256, 8192)), dim3(256), 0, s,
-                     p, n_dev, per);
   DP_HIP(hipGetLastError());
 }
 

@@ -139,22 +139,15 @@ __device__ __forceinline__ Cand feature_best(const FeatBins<BPL>& d, int32_t f, 
 }
 
 // One wavefront per (node, feature): the feature's best candidate.
-// Workgroups loop over (node, feature group) items; the node count may come
-// from device memory.
+// Workgroups loop over (node, feature group) items.
 template <int BPL>
 __global__ __launch_bounds__(64 * kFeatWaves) void evaluate_features_kernel(
-    const long long* __restrict__ hist, int32_t n_nodes_host,
-    const int32_t* __restrict__ n_nodes_dev, int32_t n_features, int32_t bin_stride,
-    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums,
-    const int32_t* __restrict__ exps, int32_t exp_g_host, int32_t exp_h_host, Param p,
-    const uint32_t* __restrict__ fmask, const uint8_t* __restrict__ skip_bins,
-    FeatCand* __restrict__ cand) {
+    const long long* __restrict__ hist, int32_t n_nodes, int32_t n_features, int32_t bin_stride,
+    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums, int32_t exp_g,
+    int32_t exp_h, Param p, FeatCand* __restrict__ cand) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int32_t n_nodes = n_nodes_dev ? *n_nodes_dev : n_nodes_host;
   const int32_t groups = (n_features + kFeatWaves - 1) / kFeatWaves;
   const int64_t n_items = int64_t(n_nodes) * groups;
-  const int exp_g = exps ? exps[0] : exp_g_host;
-  const int exp_h = exps ? exps[1] : exp_h_host;
   const double ug = ldexp(1.0, -exp_g), uh = ldexp(1.0, -exp_h);
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int32_t node = int32_t(item / groups);
@@ -164,10 +157,7 @@ __global__ __launch_bounds__(64 * kFeatWaves) void evaluate_features_kernel(
     load_feature<BPL>(hist, node, f, n_features, bin_stride, bins);
     const long long gp = node_sums[2 * node], hp = node_sums[2 * node + 1];
     const double parent_gain = calc_gain(p, double(gp) * ug, double(hp) * uh);
-    // A feature outside the node's sample has no bins to split at: loss -inf.
-    const int nb = feature_allowed(fmask, node, f, n_features) ? n_bins[f] : 0;
-    const int skip = skip_bins ? int(skip_bins[f]) : -1;
-    const Cand c = feature_best<BPL>(bins, f, nb, skip, gp, hp, parent_gain, ug, uh, p);
+    const Cand c = feature_best<BPL>(bins, f, n_bins[f], -1, gp, hp, parent_gain, ug, uh, p);
     if (lane == 0) cand[int64_t(node) * n_features + f] = FeatCand{c.loss, c.gl, c.hl, c.bin, c.dl};
   }
 }
@@ -175,20 +165,14 @@ __global__ __launch_bounds__(64 * kFeatWaves) void evaluate_features_kernel(
 // Up to 64 bins: four features per wavefront (seg_evaluate).  Workgroups loop
 // over (node, group of 16 features) items.
 __global__ __launch_bounds__(256) void evaluate_features_seg_kernel(
-    const long long* __restrict__ hist, int32_t n_nodes_host,
-    const int32_t* __restrict__ n_nodes_dev, int32_t n_features, int32_t bin_stride,
-    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums,
-    const int32_t* __restrict__ exps, int32_t exp_g_host, int32_t exp_h_host, Param p,
-    const uint32_t* __restrict__ fmask, const uint8_t* __restrict__ skip_bins,
-    FeatCand* __restrict__ cand) {
+    const long long* __restrict__ hist, int32_t n_nodes, int32_t n_features, int32_t bin_stride,
+    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums, int32_t exp_g,
+    int32_t exp_h, Param p, FeatCand* __restrict__ cand) {
   constexpr int BPL = 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int seg = lane >> 4, sub = lane & 15;
-  const int32_t n_nodes = n_nodes_dev ? *n_nodes_dev : n_nodes_host;
   const int32_t groups = (n_features + kSegFeatures - 1) / kSegFeatures;
   const int64_t n_items = int64_t(n_nodes) * groups;
-  const int exp_g = exps ? exps[0] : exp_g_host;
-  const int exp_h = exps ? exps[1] : exp_h_host;
   const double ug = ldexp(1.0, -exp_g), uh = ldexp(1.0, -exp_h);
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int32_t node = int32_t(item / groups);
@@ -202,8 +186,8 @@ __global__ __launch_bounds__(256) void evaluate_features_seg_kernel(
       dg[j] = live && b < bin_stride ? hf[2 * b] : 0;
       dh[j] = live && b < bin_stride ? hf[2 * b + 1] : 0;
     }
-    seg_evaluate(dg, dh, node, f, live, n_features, n_bins, node_sums, ug, uh, p, fmask,
-                 skip_bins, cand);
+    seg_evaluate(dg, dh, node, f, live, n_features, n_bins, node_sums, ug, uh, p, nullptr, nullptr,
+                 cand);
   }
 }
 
@@ -571,17 +555,11 @@ constexpr int kNodeFeatures = kEvalNodeFeatures;  // feature counts up to this u
 // the node's split record -- the whole evaluation in one launch.
 template <int BPL>
 __global__ __launch_bounds__(64 * kNodeWaves) void evaluate_nodes_kernel(
-    const long long* __restrict__ hist, int32_t n_nodes_host,
-    const int32_t* __restrict__ n_nodes_dev, int32_t n_features, int32_t bin_stride,
-    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums,
-    const int32_t* __restrict__ exps, int32_t exp_g_host, int32_t exp_h_host, Param p,
-    const uint32_t* __restrict__ fmask, const uint8_t* __restrict__ skip_bins,
-    dp_split_record* __restrict__ out) {
+    const long long* __restrict__ hist, int32_t n_nodes, int32_t n_features, int32_t bin_stride,
+    const int32_t* __restrict__ n_bins, const long long* __restrict__ node_sums, int32_t exp_g,
+    int32_t exp_h, Param p, dp_split_record* __restrict__ out) {
   __shared__ Cand wave_best[kNodeWaves];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int32_t n_nodes = n_nodes_dev ? *n_nodes_dev : n_nodes_host;
-  const int exp_g = exps ? exps[0] : exp_g_host;
-  const int exp_h = exps ? exps[1] : exp_h_host;
   const double ug = ldexp(1.0, -exp_g), uh = ldexp(1.0, -exp_h);
   for (int32_t node = blockIdx.x; node < n_nodes; node += gridDim.x) {
     // The wave's next feature is loaded while the current one is evaluated.
@@ -598,9 +576,7 @@ __global__ __launch_bounds__(64 * kNodeWaves) void evaluate_nodes_kernel(
     for (int32_t f = wave; f < n_features; f += kNodeWaves) {  // wave-uniform
       if (f + kNodeWaves < n_features)
         load_feature<BPL>(hist, node, f + kNodeWaves, n_features, bin_stride, nxt);
-      const int nb = feature_allowed(fmask, node, f, n_features) ? n_bins[f] : 0;
-      const int skip = skip_bins ? int(skip_bins[f]) : -1;
-      const Cand c = feature_best<BPL>(cur, f, nb, skip, gp, hp, parent_gain, ug, uh, p);
+      const Cand c = feature_best<BPL>(cur, f, n_bins[f], -1, gp, hp, parent_gain, ug, uh, p);
       if (c.loss > -INFINITY && better(c, best)) best = c;
       cur = nxt;
     }
@@ -732,12 +708,10 @@ constexpr int kSelectThreads = 256;
 // One workgroup per node (looping over nodes): argmax over the node's feature
 // candidates with ties to the lowest feature, then the split record.
 __global__ __launch_bounds__(kSelectThreads) void select_splits_kernel(
-    const FeatCand* __restrict__ cand, int32_t n_nodes_host,
-    const int32_t* __restrict__ n_nodes_dev, int32_t n_features, double gamma,
+    const FeatCand* __restrict__ cand, int32_t n_nodes, int32_t n_features, double gamma,
     dp_split_record* __restrict__ out) {
   __shared__ Cand wave_best[kSelectThreads / 64];
   __shared__ dp_split_record rec;
-  const int32_t n_nodes = n_nodes_dev ? *n_nodes_dev : n_nodes_host;
   for (int32_t node = blockIdx.x; node < n_nodes; node += gridDim.x) {
     const dp_split_record r =
         select_node<kSelectThreads>(cand, node, n_features, gamma, wave_best, &rec);
@@ -764,15 +738,11 @@ void launch_evaluate(const int64_t* hist, int32_t n_nodes, int32_t n_features, i
   const auto* sums = reinterpret_cast<const long long*>(node_sums);
   if (n_features <= kNodeFeatures) {
     const dim3 grid(n_nodes < 2048 ? n_nodes : 2048), block(64 * kNodeWaves);
-    if (bin_stride <= 64)
-      hipLaunchKernelGGL(evaluate_nodes_kernel<1>, grid, block, 0, s, h, n_nodes, nullptr,
-                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
-    else if (bin_stride <= 128)
-      hipLaunchKernelGGL(evaluate_nodes_kernel<2>, grid, block, 0, s, h, n_nodes, nullptr,
-                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
-    else
-      hipLaunchKernelGGL(evaluate_nodes_kernel<4>, grid, block, 0, s, h, n_nodes, nullptr,
-                         n_features, bin_stride, n_bins, sums, nullptr, exp_g, exp_h, p, nullptr, nullptr, out);
+    hipLaunchKernelGGL(bin_stride <= 64    ? evaluate_nodes_kernel<1>
+                       : bin_stride <= 128 ? evaluate_nodes_kernel<2>
+                                           : evaluate_nodes_kernel<4>,
+                       grid, block, 0, s, h, n_nodes, n_features, bin_stride, n_bins, sums, exp_g,
+                       exp_h, p, out);
     DP_HIP(hipGetLastError());
     return;
   }
@@ -780,19 +750,18 @@ void launch_evaluate(const int64_t* hist, int32_t n_nodes, int32_t n_features, i
   if (bin_stride <= 64) {
     const int64_t items = int64_t(n_nodes) * ((n_features + kSegFeatures - 1) / kSegFeatures);
     hipLaunchKernelGGL(evaluate_features_seg_kernel, dim3(items < 2048 ? items : 2048), dim3(256),
-                       0, s, h, n_nodes, nullptr, n_features, bin_stride, n_bins, sums, nullptr,
-                       exp_g, exp_h, p, nullptr, nullptr, cand);
+                       0, s, h, n_nodes, n_features, bin_stride, n_bins, sums, exp_g, exp_h, p,
+                       cand);
   } else {
     const int64_t groups = (n_features + kFeatWaves - 1) / kFeatWaves;
     const int64_t items = int64_t(n_nodes) * groups;
     hipLaunchKernelGGL(bin_stride <= 128 ? evaluate_features_kernel<2> : evaluate_features_kernel<4>,
                        dim3(int(items < 2048 ? items : 2048)), dim3(64 * kFeatWaves), 0, s, h,
-                       n_nodes, nullptr, n_features, bin_stride, n_bins, sums, nullptr, exp_g,
-                       exp_h, p, nullptr, nullptr, cand);
+                       n_nodes, n_features, bin_stride, n_bins, sums, exp_g, exp_h, p, cand);
   }
   DP_HIP(hipGetLastError());
   hipLaunchKernelGGL(select_splits_kernel, dim3(n_nodes < 1024 ? n_nodes : 1024),
-                     dim3(kSelectThreads), 0, s, cand, n_nodes, nullptr, n_features,
+                     dim3(kSelectThreads), 0, s, cand, n_nodes, n_features,
                      double(param.gamma), out);
   DP_HIP(hipGetLastError());
 }
