@@ -228,6 +228,7 @@ __global__ __launch_bounds__(kThreads) void sort_cuts_kernel(const float* __rest
 // ---------------------------------------------------------------------------
 // Many rows
 // ---------------------------------------------------------------------------
+// The "lowbias32" integer hash of C. Wellons' published search for 32-bit mixers.
 __device__ __forceinline__ uint32_t hash32(uint32_t x) {
   x ^= x >> 16;
   x *= 0x7feb352du;
@@ -776,6 +777,12 @@ int32_t sketch_chunks(int64_t n_rows, int32_t tiles, int32_t cus) {
   return best;
 }
 
+// Features of a block: whole groups of 128 (sample_kernel's order).
+int32_t sketch_block(int64_t n_rows) {
+  const int64_t fit = (int64_t(1) << 34) / n_rows / 128 * 128;
+  return int32_t(std::clamp<int64_t>(fit, 128, 1 << 16));
+}
+
 }  // namespace
 
 void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_t max_bin,
@@ -815,10 +822,12 @@ void sketch_cuts(const float* values, int64_t n_rows, int32_t n_features, int32_
       DP_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(kBucketLds)));
     DP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(plan_kernel),
                                hipFuncAttributeMaxDynamicSharedMemorySize, int(kPlanLds)));
-    // Blocks of features bound the tables (about 12 KiB a feature and chunk).
-    constexpr int32_t kBlock = 1 << 16;
-    for (int32_t f0 = 0; f0 < n_features; f0 += kBlock) {
-      const int32_t fc = std::min(kBlock, n_features - f0);
+    // Blocks of features bound the tables (12 KiB a feature, and 4 more per row chunk)
+    // and the gathered keys (about max_bin / kBuckets of a block's values: 17 GB for
+    // 256 bins and 2^34 values, what sorting blocks of 2^31 keys took).
+    const int32_t block = sketch_block(n_rows);
+    for (int32_t f0 = 0; f0 < n_features; f0 += block) {
+      const int32_t fc = std::min(block, n_features - f0);
       const int32_t tiles = (fc + kTile - 1) / kTile;
       const int32_t chunks = sketch_chunks(n_rows, tiles, cus);
       const int64_t chunk_rows = (n_rows + chunks - 1) / chunks;

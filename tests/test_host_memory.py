@@ -213,3 +213,23 @@ def test_the_tuner_times_what_runs(host, rows, features, booster):
     """)
     assert any("reduce_evaluate_dense" in n for n in names) == booster
     assert any("hist_reduce" in n for n in names) != booster
+
+
+@pytest.mark.parametrize("rows,features,blocks", [(20000, 65536, 1), (20000, 65537, 2),
+                                                  (1 << 26, 256, 1), (1 << 26, 1025, 5),
+                                                  (1 << 31, 300, 3)])
+def test_the_sketch_takes_features_by_blocks(host, rows, features, blocks):
+    """Its scratch is bounded: at most 2^16 features at once, and 2^34 values or 128 features."""
+    sampled = host(f"""
+        ws, p = ctypes.c_void_p(), ctypes.c_void_p()
+        ok(lib.dp_workspace_create(ctypes.byref(ws)))
+        ok(fake.hipMalloc(ctypes.byref(p), ctypes.c_size_t(4)))  # the kernels do not run
+        n = {features}
+        ptr, cuts = (ctypes.c_int32 * (n + 1))(), (ctypes.c_float * (n * 16))()
+        mins, missing = (ctypes.c_float * n)(), ctypes.c_int32()
+        lib.dp_sketch_cuts(ws, p, ctypes.c_int64({rows}), n, 16, ptr, cuts, mins,
+                           ctypes.byref(missing), None)
+        names = fake.fake_launches().decode().split(";")
+        print(json.dumps(sum("sample_kernel" in x for x in names)))
+    """)
+    assert sampled == blocks
