@@ -236,3 +236,33 @@ def test_a_tree_as_deep_as_packed_nodes_count(dp, device, splits, rows):
     got = dp.Booster.from_buffer(_model(forest, 3, 1)).predict(
         torch.as_tensor(x, device=device), margin=True).cpu().numpy()
     np.testing.assert_array_equal(got.view(np.uint32), _margins(forest, x, 1).view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,features,trees,depth", [
+    (300, 9, 2, 3),        # a small forest
+    (5000, 28, 40, 6),     # rows in LDS, several trees at a time
+    (2000, 5000, 12, 7),   # not worth that
+    (70001, 20, 40, 6)])   # a row per thread in LDS
+def test_rows_with_gaps_between_them(dp, device, rows, features, trees, depth):
+    import ctypes
+    import torch
+
+    rng = np.random.default_rng(rows)
+    forest = _forest(rng, trees, depth, features, 0.9)
+    bst = dp.Booster.from_buffer(_model(forest, features, 1))
+    wide = rng.normal(size=(rows, features + 3)).astype(np.float32)
+    dev = torch.as_tensor(wide, device=device)
+    shape, dim = ctypes.POINTER(ctypes.c_uint64)(), ctypes.c_uint64()
+    out = ctypes.POINTER(ctypes.c_float)()
+    a = json.dumps({"data": [dev.data_ptr(), True], "shape": [rows, features], "version": 3,
+                    "strides": [4 * (features + 3), 4], "typestr": "<f4", "stream": 1})
+    cfg = json.dumps({"type": 1, "training": False, "iteration_begin": 0, "iteration_end": 0,
+                      "strict_shape": True, "cache_id": 0, "missing": float("nan")})
+    dp.check(dp.load().XGBoosterPredictFromCudaArray(
+        bst.handle, a.encode(), cfg.encode(), None, ctypes.byref(shape), ctypes.byref(dim),
+        ctypes.byref(out)))
+    got = torch.empty((rows, 1), device=device)
+    dp._hip_memcpy()(ctypes.c_void_p(got.data_ptr()),
+                     ctypes.c_void_p(ctypes.addressof(out.contents)), rows * 4)
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32),
+                                  _margins(forest, wide[:, :features], 1).view(np.uint32))

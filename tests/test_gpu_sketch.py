@@ -153,3 +153,54 @@ def test_training_on_narrow_matrices_with_missing_values(dp, oracle, device, fea
         max_bin=max_bin, values_labels=(torch.as_tensor(x, device=device),
                                         torch.as_tensor(y, device=device)))
     _compare(bst, o_trees, o_margin, pos, n, 1)
+
+
+def test_cuts_of_more_features_than_a_block(dp, ws, device):
+    """65,536 features make a block: each feature's cuts are those it has among 48 (one block)."""
+    import torch
+    from dpgbdt import ops
+
+    n, base, features, max_bin = 16500, 48, (1 << 16) + 40, 16
+    rng = np.random.default_rng(1)
+    x = rng.normal(size=(n, base)).astype(np.float32)
+    x[:, 1] = rng.integers(0, 9, n)
+    x[:, 2] = np.nan
+    x[rng.random(x.shape) < 0.05] = np.nan
+    part = torch.as_tensor(x, device=device)
+    ptr, cuts, mins, missing = ops.sketch_cuts(ws, part, max_bin)
+    wide = part.repeat(1, features // base + 1)[:, :features].contiguous()
+    w_ptr, w_cuts, w_mins, w_missing = ops.sketch_cuts(ws, wide, max_bin)
+    of = np.arange(features) % base
+    np.testing.assert_array_equal(np.diff(w_ptr), np.diff(ptr)[of])
+    np.testing.assert_array_equal(w_mins.view(np.uint32), mins.view(np.uint32)[of])
+    want = np.concatenate([cuts[ptr[f]:ptr[f + 1]] for f in of])
+    np.testing.assert_array_equal(w_cuts.view(np.uint32), want.view(np.uint32))
+    assert missing and w_missing
+
+
+@pytest.mark.parametrize("rows,features", [(200, 7), (4000, 300), (70000, 20)])
+def test_matrices_with_gaps_between_rows(dp, device, rows, features):
+    """A matrix read from every row of a wider array trains what its copy trains."""
+    import ctypes
+    import json
+    import torch
+
+    rng = np.random.default_rng(rows)
+    wide = torch.as_tensor(rng.normal(size=(rows, features + 5)).astype(np.float32), device=device)
+    y = (wide[:, 0] > 0).float()
+    view = wide[:, :features]
+    d = dp.DMatrix.__new__(dp.DMatrix)
+    d.handle = ctypes.c_void_p()
+    a = json.dumps({"data": [view.data_ptr(), True], "shape": [rows, features], "version": 3,
+                    "strides": [4 * (features + 5), 4], "typestr": "<f4", "stream": 1})
+    dp.check(dp.load().XGDMatrixCreateFromCudaArrayInterface(a.encode(), b'{"missing": NaN}',
+                                                             ctypes.byref(d.handle)))
+    dp.check(dp.load().XGDMatrixSetInfoFromInterface(d.handle, b"label",
+                                                     dp.array_interface(y).encode()))
+    models = []
+    for m in (d, dp.DMatrix(view.contiguous(), y)):
+        bst = dp.Booster({"objective": "binary:logistic", "max_depth": 4, "dp_autotune": 0}, [m])
+        bst.update(m, 0)
+        bst.update(m, 1)
+        models.append(bst.save_raw())
+    assert models[0] == models[1]
