@@ -771,7 +771,9 @@ void DMatrix::release_pending() {
     }
   }
   pending.clear();
-  std::set<int> devices{values.dev, labels.dev};
+  std::set<int> devices;  // those only: another's first use would set it up
+  if (values.p) devices.insert(values.dev);
+  if (labels.p) devices.insert(labels.dev);
   for (const auto& q : quantized) devices.insert(q.second->d_nbins.dev);
   for (int device : devices) {
     try {

@@ -24,7 +24,7 @@
 //
 // One thread per row over global memory, the form these replaced, took 7,140 us
 // for 1M x 28 rows through 100 trees of depth 8, 2,700 us for 60k x 784 through
-// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 360, 240 and 12 us.
+// 500 of depth 6 (ten outputs) and 217 us for 64 rows; now 359, 230 and 7 us.
 // The first is bound by its vector instructions (11 per visit) and LDS reads (8
 // bytes of node from random banks, 4 of value), the second by the node loads of
 // its lanes, which rarely share a line.  Staging the second's nodes in LDS too

@@ -118,11 +118,14 @@ def test_a_matrix_waits_for_its_own_device(host):
         counts.append(fake.fake_synchronised(1))
         now = ctypes.c_int()
         ok(fake.hipGetDevice(ctypes.byref(now)))
-        print(json.dumps([counts, now.value]))
+        h = matrix(10, 5, device=1)  # without labels: nothing of it is on device 0
+        other = fake.fake_synchronised(0)
+        ok(lib.XGDMatrixFree(h))
+        print(json.dumps([counts, now.value, fake.fake_synchronised(0) - other]))
     """)
-    (start, labels, freed), device = out
+    (start, labels, freed), device, other = out
     assert start < labels < freed
-    assert device == 0
+    assert device == 0 and other == 0
 
 
 POOL = """
